@@ -169,7 +169,10 @@ typedef struct {
                            strips); a pack with a snapshot due at an intermediate step
                            falls back to fewer steps per launch; the last steps of a
                            run (up to two 7-step launches on one-wavefront strips)
-                           go in as few, evenly split launches                         */
+                           go in as few, evenly split launches
+                           (with every tile option at its default, grids whose states
+                           stay in the last-level cache run the window-tile kernel, 6 to
+                           16 steps per launch, instead: same results bit for bit)     */
   int graph_steps;      /* 0 = default (64, rounded up to an even number of launches);
                            < 0: no graphs. Fused kernel without snapshots: whole chunks
                            of this many steps replay one captured HIP graph (kernels

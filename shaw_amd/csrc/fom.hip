@@ -33,6 +33,9 @@
 //    wavefront (one thread per point, all columns of a 1- or 2-column block);
 //    neighbours move between lanes, and the waves of a workgroup share only
 //    a coefficient ring. The default: six steps per launch.
+//  * k_tile: six to sixteen steps per launch on grids whose states stay in
+//    the last-level cache; a workgroup holds a window of the grid, states and
+//    coefficients, in registers.
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
@@ -904,7 +907,7 @@ __global__ void __launch_bounds__(512) k_fusedN(StepArgsN<T, NS> aa) {
 constexpr int kDppWaveRol1 = 0x134, kDppWaveRor1 = 0x13C;
 template <int CTRL>
 __device__ __forceinline__ int dppMove(int x) {
-  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, false);
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true);
 }
 template <int CTRL>
 __device__ __forceinline__ double dppMove(double x) {
@@ -1227,6 +1230,267 @@ __global__ void __launch_bounds__(256) k_fusedW(StepArgsN<T, NS> aa) {
   }
 }
 
+// ------------------------------------------------------------ window tiles
+// k_tile: a.steps leapfrog steps of one window of the grid per workgroup, for
+// grids whose states stay in the last-level cache. There a launch of the
+// marching kernels is a chain of latencies rather than a stream (a k_fusedW
+// strip loads its rows one after another: 14-16 us per four steps at 21 x 51
+// as at 200 x 1000). A window is 64
+// points (one wavefront) by WV * RT rows; wave w holds rows w RT .. w RT + RT-1
+// of it in registers, states and coefficients, so the whole window is loaded
+// at once, stepped without touching memory and stored at the end. West and
+// east neighbours move between lanes (DPP), south and north ones are the
+// wave's own registers except at its first and last row, which pass through
+// two LDS rows and two barriers a step. Windows overlap by 2 a.halo rows and
+// points (halo >= steps; 0 in a direction that one window covers): a level's
+// values are valid one row and one point further inside than the level
+// before, and the stored part of a window is where the last level is valid.
+// The workgroup keeps the coefficients for its a.cbPer column blocks.
+// Bound by FP64 issue (92 VALU cycles a row, point column and step) and the
+// window's loads at the start of a launch. Two barriers a step: carrying the
+// velocity row north of a wave's last as well saves one and was slower (0.57
+// against 0.50 us a step at 21 x 51, its arithmetic costs more than the
+// barrier). Measured, us per step, k_fusedW before and k_tile now: 21 x 51
+// M = 1 3.72 -> 0.50; 200 x 1000 M = 1 4.17 -> 1.42; 256 x 1024 M = 4 9.17 ->
+// 4.04, M = 16 15.9 -> 13.0; 509 x 2051 M = 8 36.4 -> 28.7.
+// Every value is the one-step kernel's expression in its order. Where it
+// clamps a neighbour at the mesh's edge (a merged coefficient beside a zero
+// one), the merged coefficient moves to the neighbour that exists.
+template <class T>
+struct TileArgs {
+  const T* vIn;
+  T* vOut;
+  const T* sIn;
+  T* sOut;
+  const T* cv;          // [nVp][4]
+  const T* cs;          // [nSp][2]
+  const int64_t* src;   // as StepArgs
+  const T* srcRhoInv;
+  const double* ftab;   // [steps of the run][M]
+  const int32_t* recv;  // [nVp] receiver index or -1; nullptr: none
+  int64_t recvRow;      // the one grid row holding every receiver, or -1
+  double* seis;         // LayoutLeft [R x Tcap x M]
+  uint64_t R, Tcap;
+  uint32_t step0, steps, every;  // steps already taken, steps of this launch
+  uint32_t nr, nth, M, nb, cbPer;
+  uint32_t nTx, nTy, haloX, haloY;
+  T dt;
+  int rank1;
+};
+
+template <class T, int N>
+__device__ __forceinline__ void loadPair(T (&x)[N], T (&y)[N], const T* p) {
+  // 2 N values at T's alignment (a stress row's srp and stp of one point)
+  typedef T V __attribute__((ext_vector_type(2 * N), aligned(sizeof(T) * N)));
+  const V a = *reinterpret_cast<const V*>(p);
+#pragma unroll
+  for (int k = 0; k < N; ++k) { x[k] = a[k]; y[k] = a[N + k]; }
+}
+
+__device__ __forceinline__ double laneValue(double x, int l) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ float laneValue(float x, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
+}
+
+template <class T, int CPT, int RT, int WV>
+__global__ void __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV / 4, WV / 4))) k_tile(TileArgs<T> a) {
+  __shared__ T edgeV[WV][CPT][64];  // the first velocity row of each wave
+  __shared__ T edgeS[WV][CPT][64];  // the last srp row of each wave
+  const unsigned lb = xcdLogicalBlock(blockIdx.x, gridDim.x);
+  const uint32_t tx = lb % a.nTx, ty = (lb / a.nTx) % a.nTy, grp = lb / (a.nTx * a.nTy);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64)), lane = (int)(threadIdx.x % 64);
+  constexpr uint32_t ROWS = WV * RT;
+  const uint32_t nr = a.nr, nth = a.nth, rs = 2 * nth - 1;
+  const uint32_t i = tx * (64 - 2 * a.haloX) + lane, jw = ty * (ROWS - 2 * a.haloY);
+  const uint32_t j0 = jw + wave * RT;  // the wave's first row
+  // the part of the window this workgroup stores
+  const uint32_t iEnd = tx + 1 == a.nTx ? nth : tx * (64 - 2 * a.haloX) + 64 - a.haloX;
+  const uint32_t jLo = jw + (ty ? a.haloY : 0), jEnd = ty + 1 == a.nTy ? nr : jw + ROWS - a.haloY;
+  const bool live = i < nth, ownLane = live && (uint32_t)lane >= (tx ? a.haloX : 0) && i < iEnd;
+
+  // a row is a scalar offset, a point a lane offset (values)
+  const uint32_t oV = i * CPT, oV4 = 4 * i;
+  T c[RT][8];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) c[r][q] = T(0);
+    const uint32_t j = j0 + r;
+    if (j < nr && live) {
+      T cv[4];
+      load(cv, a.cv + (size_t)j * nth * 4 + oV4);
+      const bool top = j + 1 == nr;
+      c[r][0] = top ? T(0) : cv[0];
+      c[r][1] = top ? cv[0] : cv[1];
+      c[r][2] = i == 0 ? T(0) : cv[2];
+      c[r][3] = i == 0 ? cv[2] : cv[3];
+      if (!top) {
+        T s[2];
+        load(s, a.cs + (size_t)j * rs * 2 + oV4);
+        c[r][4] = s[0];
+        c[r][5] = s[1];
+      }
+      if (i + 1 < nth) {
+        T s[2];
+        load(s, a.cs + (size_t)j * rs * 2 + (top ? 2 * i : oV4 + 2));
+        c[r][6] = s[0];
+        c[r][7] = s[1];
+      }
+    }
+  }
+  // receivers: their one grid row when it is one of this wave's rows
+  const int recvAt = a.recv && a.recvRow >= 0 ? (int)((int64_t)a.recvRow - (int64_t)j0) : -1;
+  const bool recvHere = recvAt >= 0 && recvAt < RT && a.recvRow >= (int64_t)jLo && a.recvRow < (int64_t)jEnd;
+  const int32_t recvQ = recvHere && ownLane ? a.recv[(size_t)a.recvRow * nth + i] : -1;
+
+  const uint64_t nVp = (uint64_t)nr * nth, nSp = (uint64_t)(nr - 1) * nth + (uint64_t)nr * (nth - 1);
+  const uint32_t cbEnd = (grp + 1) * a.cbPer < a.nb ? (grp + 1) * a.cbPer : a.nb;
+  for (uint32_t cb = grp * a.cbPer; cb < cbEnd; ++cb) {
+    const T* vIn = a.vIn + (uint64_t)cb * nVp * CPT;
+    const T* sIn = a.sIn + (uint64_t)cb * nSp * CPT;
+    T v[RT][CPT], sr[RT][CPT], st[RT][CPT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) v[r][k] = sr[r][k] = st[r][k] = T(0);
+      const uint32_t j = j0 + r;
+      if (j < nr && live) {
+        load(v[r], vIn + (size_t)j * nth * CPT + oV);
+        if (j + 1 < nr) {
+          if (i + 1 < nth) loadPair(sr[r], st[r], sIn + (size_t)j * rs * CPT + 2 * oV);
+          else load(sr[r], sIn + (size_t)j * rs * CPT + 2 * oV);
+        } else if (i + 1 < nth) {
+          load(st[r], sIn + (size_t)j * rs * CPT + oV);
+        }
+      }
+    }
+    // the sources of this block's columns: the wave's row (or -1), the lane,
+    // and the increments of up to 64 steps, step l in lane l % 64
+    int srcAt[CPT], srcLane[CPT];
+    T inc[CPT];
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      const int64_t g = a.src[cb * CPT + k];
+      srcAt[k] = -1;
+      srcLane[k] = 0;
+      inc[k] = T(0);
+      if (g >= 0) {
+        const uint32_t row = (uint32_t)g / nth, at = (uint32_t)g % nth, iw = i - lane;
+        if (row >= j0 && row < j0 + RT && at >= iw && at < iw + 64) {
+          srcAt[k] = (int)(row - j0);
+          srcLane[k] = (int)(at - iw);
+        }
+      }
+    }
+    uint32_t sample = 0, phase = 0;  // samples taken, steps since the last
+    if (a.recv) {
+      sample = a.step0 / a.every;
+      phase = a.step0 % a.every;
+    }
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) edgeS[wave][k][lane] = sr[RT - 1][k];
+    __syncthreads();
+    for (uint32_t l = 0; l < a.steps; ++l) {
+      if (l % 64 == 0) {
+#pragma unroll
+        for (int k = 0; k < CPT; ++k)
+          if (srcAt[k] >= 0) {
+            const uint32_t col = cb * CPT + k, step = l + lane;
+            const T f = step < a.steps ? (T)a.ftab[(uint64_t)(a.step0 + step) * a.M + col] : T(0);
+            inc[k] = a.rank1 ? a.dt * a.srcRhoInv[col] * f : a.srcRhoInv[col] * f * a.dt;
+          }
+      }
+      T below[CPT];  // srp of the row south of the wave's first
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        below[k] = edgeS[wave > 0 ? wave - 1 : 0][k][lane];
+        if (wave == 0) below[k] = T(0);
+      }
+#pragma unroll
+      for (int r = RT - 1; r >= 0; --r)
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) {
+          const T W = fromWest(st[r][k]);
+          T sum = c[r][0] * sr[r][k] + c[r][1] * (r ? sr[r ? r - 1 : 0][k] : below[k]);
+          sum = sum + c[r][2] * W;
+          sum = sum + c[r][3] * st[r][k];
+          v[r][k] = v[r][k] + a.dt * sum;
+        }
+#pragma unroll
+      for (int k = 0; k < CPT; ++k)
+        if (srcAt[k] >= 0) {
+          const T add = laneValue(inc[k], (int)(l % 64));
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            if (r == srcAt[k]) v[r][k] = lane == srcLane[k] ? v[r][k] + add : v[r][k];
+        }
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) edgeV[wave][k][lane] = v[0][k];
+      if (a.recv && ++phase == a.every) {
+        phase = 0;
+        if (a.recvRow >= 0) {
+          if (recvHere && recvQ >= 0)
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+              if (r == recvAt)
+#pragma unroll
+                for (int k = 0; k < CPT; ++k)
+                  if (cb * CPT + k < a.M)
+                    a.seis[(uint64_t)recvQ + a.R * (sample + a.Tcap * (cb * CPT + k))] = (double)v[r][k];
+        } else if (ownLane) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            const uint32_t j = j0 + r;
+            if (j < jLo || j >= jEnd) continue;
+            const int32_t q = a.recv[(size_t)j * nth + i];
+            if (q < 0) continue;
+#pragma unroll
+            for (int k = 0; k < CPT; ++k)
+              if (cb * CPT + k < a.M) a.seis[(uint64_t)q + a.R * (sample + a.Tcap * (cb * CPT + k))] = (double)v[r][k];
+          }
+        }
+        ++sample;
+      }
+      __syncthreads();
+      T above[CPT];  // v of the row north of the wave's last
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) {
+        above[k] = edgeV[wave + 1 < WV ? wave + 1 : 0][k][lane];
+        if (wave + 1 == WV) above[k] = T(0);
+      }
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int k = 0; k < CPT; ++k) {
+          const T vUp = r + 1 < RT ? v[r + 1 < RT ? r + 1 : 0][k] : above[k];
+          sr[r][k] = sr[r][k] + a.dt * (c[r][4] * vUp + c[r][5] * v[r][k]);
+          const T vE = fromEast(v[r][k]);
+          st[r][k] = st[r][k] + a.dt * (c[r][6] * v[r][k] + c[r][7] * vE);
+        }
+#pragma unroll
+      for (int k = 0; k < CPT; ++k) edgeS[wave][k][lane] = sr[RT - 1][k];
+      __syncthreads();
+    }
+    T* vOut = a.vOut + (uint64_t)cb * nVp * CPT;
+    T* sOut = a.sOut + (uint64_t)cb * nSp * CPT;
+    if (ownLane)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+        const uint32_t j = j0 + r;
+        if (j < jLo || j >= jEnd) continue;
+        store(vOut + (size_t)j * nth * CPT + oV, v[r]);
+        T* sRow = sOut + (size_t)j * rs * CPT;
+        if (j + 1 < nr) store(sRow + 2 * oV, sr[r]);
+        if (i + 1 < nth) store(sRow + (j + 1 < nr ? 2 * oV + CPT : oV), st[r]);
+      }
+  }
+}
+
 // ------------------------------------------------------------ gathers
 template <class T>
 __global__ void k_snapshot(const T* __restrict__ x, uint64_t n, uint32_t MC, const uint32_t* __restrict__ cols,
@@ -1409,6 +1673,9 @@ class FomEngine final : public shaw_fom {
       SHAW_REQUIRE(spl_ <= 2 || fits32(), SHAW_ERR_ARG,
                    "3 or 4 steps per launch need a column block of fewer than 2^32 stress values");
       setStrips();
+      const bool asked = o.cols_per_thread > 0 || o.strip > 0 || o.segment > 0 || o.prefetch_rows > 0 ||
+                         o.steps_per_launch > 0 || o.col_block > 0;
+      if (!asked) planTile();
     }
     SHAW_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     SHAW_HIP(hipEventCreate(&ev0_));
@@ -1552,6 +1819,11 @@ class FomEngine final : public shaw_fom {
     for (int d = 0; d < 2; ++d)
       if (snap_[d].ncols) SHAW_REQUIRE(last / snap_[d].every <= snap_[d].Tcap, SHAW_ERR_STATE, "snapshot buffer too small");
     uint64_t k = 0;
+    if (tile_.steps && last < (1ull << 32)) {
+      while (k < nsteps) k += launchTile(nsteps - k);
+      SHAW_HIP(hipGetLastError());
+      return;
+    }
     // whole chunks of graphStep_ steps replay one captured graph (fused
     // kernels, no snapshots: a snapshot kernel would depend on the step)
     const bool graphs = graphSteps_ > 0 && kernel_ == SHAW_KERNEL_FUSED && !snap_[0].ncols && !snap_[1].ncols &&
@@ -1877,7 +2149,7 @@ class FomEngine final : public shaw_fom {
     snapshot(1, a.sOut);
   }
   // Tile autotuner of the fused kernel: every valid (columns per thread,
-  // strip, segment, rows prefetched) is timed for `trialSteps` steps on the
+  // strip, segment, rows prefetched), and k_tile where the defaults run it, is timed for `trialSteps` steps on the
   // current state (after one untimed step), the fastest is kept, and the
   // state is restored: the trials do not advance the run, record receivers
   // or take snapshots.
@@ -1895,7 +2167,17 @@ class FomEngine final : public shaw_fom {
     SHAW_HIP(hipMemcpy(ss.p, s_[cur0].p, ss.n * sizeof(T), hipMemcpyDeviceToDevice));
     struct Cfg { int cpt; uint32_t P, SEG; int pf, spl; };
     Cfg best{cpt_, P_, SEG_, pf_, spl_};
-    double bestT = 1e300;
+    double bestT = 1e300, tileT = 1e300;
+    if (tile_.steps && step_ + tile_.steps <= ftabSteps_ && step_ + tile_.steps < (1ull << 32)) {
+      launchTile(tile_.steps, true);
+      SHAW_HIP(hipEventRecord(ev0_, stream_));
+      for (uint64_t k = 0; k < trialSteps; ++k) launchTile(tile_.steps, true);
+      SHAW_HIP(hipEventRecord(ev1_, stream_));
+      SHAW_HIP(hipEventSynchronize(ev1_));
+      float ms = 0;
+      SHAW_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
+      tileT = ms / (double)(trialSteps * tile_.steps);
+    }
     auto apply = [&](const Cfg& c) {
       cpt_ = c.cpt; P_ = c.P; SEG_ = c.SEG; pf_ = c.pf; spl_ = c.spl;
       graphSteps_ = graphStepsFor(spl_);
@@ -1934,6 +2216,8 @@ class FomEngine final : public shaw_fom {
       }
     }
     apply(best);
+    if (tileT < bestT) bestT = tileT;
+    else tile_.steps = 0;
     SHAW_HIP(hipMemcpy(v_[cur0].p, sv.p, sv.n * sizeof(T), hipMemcpyDeviceToDevice));
     SHAW_HIP(hipMemcpy(s_[cur0].p, ss.p, ss.n * sizeof(T), hipMemcpyDeviceToDevice));
     cur_ = cur0;
@@ -2164,6 +2448,110 @@ class FomEngine final : public shaw_fom {
       default: fused ? launchFused<8>(a) : launchSplit<8>(a); break;
     }
     step_ = stepNo;
+  }
+  // k_tile (default tile options only): rows per wave (12 waves), steps per
+  // launch (0: the marching kernels run) and column blocks per workgroup
+  struct Tile {
+    uint32_t rows = 4, steps = 0, cbPer = 1;
+  } tile_;
+  static constexpr uint32_t kTileWaves = 12;
+  // windows of `size` cells over n, overlapping by `halo` on each inner side
+  static uint32_t windows(uint64_t n, uint32_t size, uint32_t halo) {
+    return n <= size ? 1 : (uint32_t)((n - 2 * halo + (size - 2 * halo) - 1) / (size - 2 * halo));
+  }
+  // microseconds per step of a launch: a workgroup loads its coefficients,
+  // then per column block loads and stores the states and takes its steps;
+  // ceil(workgroups / CUs) of them run one after another on a CU. The
+  // constants are a fit to 900 timed launches (21 x 51 to 1024 x 4096, 1 to 48
+  // columns, both precisions; standard deviation 10 %), whose pick was within
+  // 4 % of the fastest measured one on 33 of 38 grids and 8 % on all.
+  double tileCost(const Tile& t) const {
+    const uint32_t rows = kTileWaves * t.rows;
+    const bool whole = nth_ <= 64 && nr_ <= rows;
+    const uint32_t wg = windows(nth_, 64, t.steps) * windows(nr_, rows, t.steps) * ((nb_ + t.cbPer - 1) / t.cbPer);
+    const double kb100 = rows * 64.0 * sizeof(T) / 1e5, steps = whole ? 200 : t.steps;
+    const double step = 0.095 * t.rows * MC_ + 0.27;
+    const double block = 4.26 * 3 * MC_ * kb100 + steps * step;
+    return (0.8 + ((wg + 255) / 256) * (3.2 * 8 * kb100 + std::min(t.cbPer, nb_) * block)) / steps;
+  }
+  // The tile kernel where one copy of the states is at most 240 MB (FP64) or
+  // 42 MB (FP32): 509 x 2051 M = 8 (200 MB) 36.4 us/step marching, 28.7 tiled;
+  // M = 16 (400 MB) 48.6 and 63.3, the marching kernel then being the one that
+  // moves fewer bytes; FP32 256 x 1024 M = 12 (38 MB) 9.2 and 7.0, M = 16
+  // (50 MB) 9.4 and 9.7. Fewer than 6 steps a launch never won.
+  void planTile() {
+    const double state = 3.0 * (double)nVp_ * nb_ * MC_ * sizeof(T);
+    if (MC_ > 2 || !fits32() || state > (sizeof(T) == 8 ? 240e6 : 42e6)) return;
+    double best = 1e300;
+    for (uint32_t rows = 2; rows <= 4; ++rows)
+      for (uint32_t steps = 6; steps <= 16 && 2 * steps < kTileWaves * rows; steps += 2)
+        for (uint32_t cb = 1; cb <= 4; cb *= 2) {
+          if (cb > 1 && cb > nb_) continue;
+          const Tile t{rows, steps, cb};
+          const double c = tileCost(t);
+          if (c < best) { best = c; tile_ = t; }
+        }
+  }
+  // one launch of at most `left` steps, evenly split up to the next snapshot
+  // or the end of the run; returns its steps. A trial records nothing and
+  // does not advance the run.
+  uint64_t launchTile(uint64_t left, bool trial = false) {
+    const uint32_t rows = kTileWaves * tile_.rows;
+    uint64_t ns = left;
+    for (int d = 0; d < 2; ++d)
+      if (snap_[d].ncols && !trial) ns = std::min(ns, snap_[d].every - step_ % snap_[d].every);
+    if (nth_ > 64 || nr_ > rows) {  // one window holds the whole grid: any number of steps
+      const uint64_t n = (ns + tile_.steps - 1) / tile_.steps;
+      ns = (ns + n - 1) / n;
+    }
+    TileArgs<T> a{};
+    a.vIn = v_[cur_].p;
+    a.sIn = s_[cur_].p;
+    a.vOut = v_[cur_ ^ 1].p;
+    a.sOut = s_[cur_ ^ 1].p;
+    a.cv = cv_.p;
+    a.cs = cs_.p;
+    a.src = src_.p;
+    a.srcRhoInv = srcRho_.p;
+    a.ftab = ftab_.p;
+    a.recv = R_ && !trial && every_ <= ~0u ? recv_.p : nullptr;  // (a longer period is never due)
+    a.recvRow = recvRow_;
+    a.seis = seis_.p;
+    a.R = R_;
+    a.Tcap = Tcap_;
+    a.step0 = (uint32_t)step_;
+    a.steps = (uint32_t)ns;
+    a.every = (uint32_t)every_;
+    a.nr = (uint32_t)nr_;
+    a.nth = (uint32_t)nth_;
+    a.M = (uint32_t)M_;
+    a.nb = nb_;
+    a.cbPer = tile_.cbPer;
+    a.haloX = nth_ <= 64 ? 0 : (uint32_t)ns;
+    a.haloY = nr_ <= rows ? 0 : (uint32_t)ns;
+    a.nTx = windows(nth_, 64, a.haloX);
+    a.nTy = windows(nr_, rows, a.haloY);
+    a.dt = (T)dt_;
+    a.rank1 = rank1_;
+    if (MC_ == 1) tileKernel<1>(a);
+    else tileKernel<2>(a);
+    cur_ ^= 1;
+    if (!trial) {
+      step_ += ns;
+      stepForSnap_ = step_;
+      snapshot(0, v_[cur_].p);
+      snapshot(1, s_[cur_].p);
+    }
+    return ns;
+  }
+  template <int CPT>
+  void tileKernel(const TileArgs<T>& a) {
+    const dim3 grid(a.nTx * a.nTy * ((a.nb + a.cbPer - 1) / a.cbPer)), block(kTileWaves * 64);
+    switch (tile_.rows) {
+      case 2: hipLaunchKernelGGL((k_tile<T, CPT, 2, kTileWaves>), grid, block, 0, stream_, a); break;
+      case 3: hipLaunchKernelGGL((k_tile<T, CPT, 3, kTileWaves>), grid, block, 0, stream_, a); break;
+      default: hipLaunchKernelGGL((k_tile<T, CPT, 4, kTileWaves>), grid, block, 0, stream_, a); break;
+    }
   }
   void snapshot(int dof, const T* x) {
     Snap& s = snap_[dof];
