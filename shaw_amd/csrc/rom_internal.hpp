@@ -56,6 +56,12 @@ void macroOperator(const double* arV, const double* arS, uint64_t kv, uint64_t k
                    std::vector<double>& gss);
 void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t kout, double* out,
             const double* base, double alpha, hipStream_t stream);
+// rom_resident.hip: the padded modes per dof (a multiple of 64) when a BF16
+// engine's operators (parts = 2 or 3 bf16 parts) stay on the CU, else 0; the
+// launch of such an engine (a.Kvp = a.Ksp = that size), only enqueued
+struct RomArgs;
+uint32_t residentModes(int parts, uint64_t kv, uint64_t ks);
+void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream);
 uint64_t projPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);
 uint32_t gramChunks(uint64_t n, uint64_t Ka, uint64_t Kb);
 uint64_t gramPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);

@@ -1,0 +1,386 @@
+// The BF16 reduced leapfrog for operators of up to 256 modes per dof: the
+// operators stay on the CU.
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "rom_device.hpp"
+#include "rom_internal.hpp"
+#include "shaw_common.hpp"
+
+namespace shaw {
+namespace {
+
+typedef float flt2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// writeSplitRows with the hardware's conversion (round to nearest even, as
+// f32ToBf16; a NaN becomes a quiet NaN)
+__device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, int lane, const double (&q)[4]) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  u2 h, l;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const flt2 x = {(float)q[2 * p], (float)q[2 * p + 1]};
+    const unsigned hb = __builtin_bit_cast(unsigned, __builtin_convertvector(x, bf16x2));
+    h[p] = hb;
+    const flt2 hf = {__uint_as_float(hb << 16), __uint_as_float(hb & 0xffff0000u)};
+    l[p] = __builtin_bit_cast(unsigned, __builtin_convertvector(x - hf, bf16x2));
+  }
+  const int item = (4 * (rt / 2) + lane / 16) * kTileCols + lane % 16;
+  reinterpret_cast<u2*>(S + item)[rt % 2] = h;
+  reinterpret_cast<u2*>(S + loOff + item)[rt % 2] = l;
+}
+
+// Where a step reads the operators' k-groups from: RR groups of every row tile
+// sit in registers, LL in LDS, the other KG - RR - LL stream from L2 through a
+// ring of DR groups. The streamed groups are spread evenly, so the products of
+// the resident ones hide each refill.
+template <int KG, int RR, int LL, int DR>
+struct Place {
+  static constexpr int S = KG - RR - LL;
+  static constexpr int group(int s) { return s * KG / (S > 0 ? S : 1); }  // the s-th streamed group
+  static constexpr bool streamed(int g) {
+    for (int q = 0; q < S; ++q)
+      if (group(q) == g) return true;
+    return false;
+  }
+  // index of group g among those of its kind (streamed, or not: LDS first)
+  static constexpr int index(int g) {
+    int n = 0;
+    for (int q = 0; q < g; ++q) n += streamed(q) == streamed(g);
+    return n;
+  }
+};
+
+// One workgroup advances 16 column slots as k_rom_steps_bf / k_rom_steps_bfm
+// do (same splits, products and FP64 updates in the same order, so every value
+// is theirs); here both operators, 2 KG row tiles by KG groups, are loaded into
+// registers and LDS once per launch. Those kernels re-read both operators from
+// L2 every step, and a CU's share of the L2 (about 90 GB/s measured, 64 B a
+// clock at most) set their time. Bound now by the chain of a half-step (split
+// -> LDS -> barrier -> products -> FP64 update), by MFMA from K = 192, and at
+// K = 256 by the groups that still stream. Per step at 1024 columns, before ->
+// now: BF16x3 K = 64 2.19 -> 0.54 us, 128 2.21 -> 0.90, 192 5.52 -> 1.57, 256
+// 5.56 -> 2.62; BF16x4 2.56 -> 0.60, 2.57 -> 1.00, 7.20 -> 2.25, 7.25 -> 4.46.
+// Waves: 2 KG row tiles in one or two per wave, at most 256 VGPRs, so that no
+// operand passes through an AGPR; four waves of twice the tiles copy every
+// operand out of AGPRs before its product (K = 192 BF16x3 1.98 against 2.40).
+template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, bool MACRO>
+__global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
+  constexpr int K = 32 * KG, TILES = 2 * KG, TPW = TILES / WAVES;
+  static_assert(TILES % WAVES == 0, "whole row tiles per wave");
+  using P = Place<KG, RR, LL, DR>;
+  constexpr int S = P::S, NR = S < DR ? S : DR;  // ring slots in use
+  using Item = typename Prec<PARTS>::Item;
+  using Acc = typename Prec<PARTS>::Acc;
+  extern __shared__ double sm[];
+  int4v* Sv = reinterpret_cast<int4v*>(sm);
+  int4v* Ss = Sv + 4 * K;
+  constexpr int lo = 2 * K;
+  int4v* Al = Ss + 4 * K;  // [operator][tile][LL][part][lane]
+  const int slot0 = blockIdx.x * kTileCols;
+  const int tid = threadIdx.x, lane = tid % 64, col = lane % 16;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  int rt[TPW];  // this wave's row tiles, the same of both operators
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) rt[t] = wave + t * WAVES;
+  const uint64_t colQ = (uint64_t)(slot0 + col) * K;
+  double qv[TPW][4], qs[TPW][4], bv[TPW][4];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      bv[t][r] = a.b[colQ + rt[t] * 16 + rowBf16(lane, r)];
+      qv[t][r] = a.qv[colQ + rt[t] * 16 + rowBf16(lane, r)];
+      qs[t][r] = a.qs[colQ + rt[t] * 16 + rowBf16(lane, r)];
+    }
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) {
+    writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
+    writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+  }
+  const uint32_t s0 = (uint32_t)a.stepCol[slot0 + col];
+  const uint32_t hz = (uint32_t)a.horizon[slot0 + col];
+  const uint32_t ev = (uint32_t)a.every[slot0 + col];
+  const double* fcol = a.ftab + (uint64_t)(slot0 + col) * a.maxSteps;
+  uint32_t span = hz > s0 ? hz - s0 : 0;  // steps to the tile's last horizon
+#pragma unroll
+  for (int off = 32; off >= 1; off /= 2) {
+    const uint32_t o = (uint32_t)__shfl_xor((int)span, off);
+    span = o > span ? o : span;
+  }
+  uint32_t steps = (uint64_t)span > a.nsteps ? (uint32_t)a.nsteps : span;
+  uint32_t mk = 0, mk2 = 0;  // mk one-steps, mk2 macro steps, then one-steps to the end
+  if constexpr (MACRO) launchPlan(a, s0, hz, ev, a.quiet[slot0 + col], span, steps, mk, mk2);
+  steps = (uint32_t)__builtin_amdgcn_readfirstlane((int)steps);
+
+  // Item of group g of row tile t (of this wave) of an operator: a scalar base
+  // and a lane offset. The bases are opaque where their loads belong (inside
+  // the step loop for the streamed groups): the loads are loop invariants
+  // that the compiler would otherwise keep in registers it does not have.
+  const uint32_t laneOff = (uint32_t)lane * sizeof(Item);
+  auto at = [&](const char* op, int t, int g) -> const Item& {
+    return *reinterpret_cast<const Item*>(op + ((size_t)rt[t] * KG + g) * 64 * sizeof(Item) + laneOff);
+  };
+  auto opaque = [](const void* x) {
+    const char* y = static_cast<const char*>(x);
+    asm volatile("" : "+s"(y));
+    return y;
+  };
+  const char* A[2];
+  Item res[2][TPW][RR > 0 ? RR : 1], ring[NR > 0 ? NR : 1][TPW];
+  Acc acc[TPW];
+  // acc = (operator op) X; the ring holds the first NR streamed groups of op on
+  // entry and of the other operator at the end
+  auto products = [&](auto opc, const int4v* X) {
+    constexpr int op = decltype(opc)::value;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) acc[t] = Acc{0, 0, 0, 0};
+    // the state's operands are read two groups ahead
+    const int4v* Xl = X + (lane / 16) * kTileCols + col;
+    int4v xb[3][2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      xb[g][0] = Xl[4 * g * kTileCols];
+      xb[g][1] = Xl[lo + 4 * g * kTileCols];
+    }
+#pragma unroll
+    for (int g = 0; g < KG; ++g) {
+      if (g + 2 < KG) {
+        xb[(g + 2) % 3][0] = Xl[4 * (g + 2) * kTileCols];
+        xb[(g + 2) % 3][1] = Xl[lo + 4 * (g + 2) * kTileCols];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const int4v xh = xb[g % 3][0], xl = xb[g % 3][1];
+      const bool str = P::streamed(g);
+      const int n = P::index(g);
+      Item it[TPW];
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        if (str) {
+          it[t] = ring[n % (NR > 0 ? NR : 1)][t];
+        } else if (n < LL) {
+#pragma unroll
+          for (int p = 0; p < PARTS; ++p) it[t].p[p] = Al[(((op * TILES + rt[t]) * LL + n) * PARTS + p) * 64 + lane];
+        } else {
+          it[t] = res[op][t][n >= LL ? n - LL : 0];
+        }
+      }
+      // the row tiles take turns, so that consecutive MFMAs are independent
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) acc[t] = mfmaBf16x32(it[t].p[0], xh, acc[t]);
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) acc[t] = mfmaBf16x32(it[t].p[0], xl, acc[t]);
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) acc[t] = mfmaBf16x32(it[t].p[1], xh, acc[t]);
+      if constexpr (PARTS == 3)
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) acc[t] = mfmaBf16x32(it[t].p[2], xh, acc[t]);
+      if (str) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+          ring[n % (NR > 0 ? NR : 1)][t] =
+              n + NR < S ? at(A[op], t, P::group(n + NR < S ? n + NR : 0))
+                         : at(A[1 - op], t, P::group(n % (NR > 0 ? NR : 1)));
+        __builtin_amdgcn_sched_barrier(0);  // the refill leaves here, not at the end of the products
+      }
+    }
+  };
+  // fills the registers, LDS and ring (every wave reads back only what it wrote)
+  auto loadOperators = [&] {
+    A[0] = opaque(a.av);
+    A[1] = opaque(a.as);
+#pragma unroll
+    for (int op = 0; op < 2; ++op)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int g = 0; g < KG; ++g) {
+          const int n = P::index(g);
+          if (P::streamed(g)) {
+            if (op == 0 && n < NR) ring[n < NR ? n : 0][t] = at(A[0], t, g);
+          } else if (n < LL) {
+            const Item it = at(A[op], t, g);
+#pragma unroll
+            for (int p = 0; p < PARTS; ++p) Al[(((op * TILES + rt[t]) * LL + n) * PARTS + p) * 64 + lane] = it.p[p];
+          } else {
+            res[op][t][n >= LL ? n - LL : 0] = at(A[op], t, g);
+          }
+        }
+  };
+#pragma nounroll
+  for (int seg = 0; seg < (MACRO ? 2 : 1); ++seg) {
+    const uint32_t from = seg == 0 ? 0u : mk + a.macro * mk2;
+    const uint32_t to = seg == 0 ? (mk2 ? mk : steps) : (mk2 ? steps : 0u);
+    if (from < to) {
+      loadOperators();
+      __syncthreads();  // both splits are in LDS
+      const uint32_t sf = s0 + from;
+      // forcing of four steps at a time, step j of them in lanes 16 j .. 16 j + 15
+      // (one column each), the next four loaded during these: a step does not
+      // wait for memory
+      auto forcing = [&](uint32_t s) { return s + lane / 16 < hz ? fcol[s + lane / 16] : 0.0; };
+      double f4 = forcing(sf), f4next = f4;
+      uint32_t phase = ev ? (sf + 1) % ev : 0;
+      uint32_t nextIdx = ev ? (sf + 1) / ev : 0;
+      for (uint32_t it = from; it < to; ++it) {
+        A[0] = opaque(a.av);
+        A[1] = opaque(a.as);
+        const uint32_t s = s0 + it;
+        const bool act = s < hz;
+        const uint32_t j = (it - from) % 4;
+        if (j == 0) {
+          f4 = f4next;
+          f4next = forcing(s + 4);
+        }
+        const double fdt = __shfl(f4, (int)(16 * j) + col) * a.dt;  // (0 past the horizon)
+        const bool smp = act && ev > 0 && phase == 0;
+        const bool anySample = (__ballot(smp) & 0xffffull) != 0;
+        // velocity: q_v += dt Ar_v q_s ; q_v += (f dt) b
+        products(std::integral_constant<int, 0>{}, Ss);
+        // (selects, kept from becoming branches: the tiles' updates are one
+        // block of independent chains)
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double y = qv[t][r] + a.dt * (double)acc[t][r];
+            double z = y + fdt * bv[t][r];
+            asm("" : "+v"(z));
+            qv[t][r] = act ? z : qv[t][r];
+          }
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
+        __syncthreads();
+        // stress: q_s += dt Ar_s q_v
+        products(std::integral_constant<int, 1>{}, Sv);
+        if (anySample) receivers<PARTS, 1, WAVES, 2>(a, Sv, lo, wave, lane, smp, nextIdx - 1, slot0);
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            double z = qs[t][r] + a.dt * (double)acc[t][r];
+            asm("" : "+v"(z));
+            qs[t][r] = act ? z : qs[t][r];
+          }
+#pragma unroll
+        for (int t = 0; t < TPW; ++t) writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+        __syncthreads();
+        if (ev && act) {
+          phase = phase + 1 == ev ? 0 : phase + 1;
+          if (phase == 0) ++nextIdx;
+        }
+      }
+    }
+    if constexpr (MACRO) {
+      if (seg == 0 && mk2) {
+        // macro steps: the blocks of G stream from L2 through a two-deep
+        // ring, which starts on the next block while one ends
+        const bool act = s0 + mk < hz;
+        Item mring[2][TPW];
+        auto stream = [&](auto zero, const char* G, const char* next, const int4v* X) {
+          if constexpr (decltype(zero)::value)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) acc[t] = Acc{0, 0, 0, 0};
+#pragma unroll
+          for (int g = 0; g < KG; ++g) {
+            groupProducts<PARTS, TPW>(mring[g % 2], g, X, lo, lane, acc);
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) mring[g % 2][t] = g + 2 < KG ? at(G, t, g + 2) : at(next, t, g + 2 - KG);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        };
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int t = 0; t < TPW; ++t) mring[g][t] = at(opaque(a.gvv), t, g);
+        __syncthreads();  // both splits are in LDS
+        for (uint32_t it = 0; it < mk2; ++it) {
+          const char *gvv = opaque(a.gvv), *gvs = opaque(a.gvs), *gsv = opaque(a.gsv), *gss = opaque(a.gss);
+          stream(std::true_type{}, gvv, gvs, Sv);
+          stream(std::false_type{}, gvs, gsv, Ss);
+          if (act)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) qv[t][r] = qv[t][r] + a.dt * (double)acc[t][r];
+          stream(std::true_type{}, gsv, gss, Sv);
+          stream(std::false_type{}, gss, gvv, Ss);
+          if (act)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) qs[t][r] = qs[t][r] + a.dt * (double)acc[t][r];
+          __syncthreads();  // every read of the old splits done
+#pragma unroll
+          for (int t = 0; t < TPW; ++t) {
+            writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
+            writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+          }
+          __syncthreads();  // the new splits complete
+          // the macro step's last step is sampled when it ends at a multiple of the period
+          const uint64_t sn = (uint64_t)s0 + mk + (uint64_t)(it + 1) * a.macro;
+          const bool smp = act && ev > 0 && sn % ev == 0;
+          if ((__ballot(smp) & 0xffffull) != 0)
+            receivers<PARTS, 1, WAVES, 2>(a, Sv, lo, wave, lane, smp, smp ? (uint32_t)(sn / ev - 1) : 0u, slot0);
+        }
+        __syncthreads();  // the next one-steps write the split the receivers read
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < TPW; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      a.qv[colQ + rt[t] * 16 + rowBf16(lane, r)] = qv[t][r];
+      a.qs[colQ + rt[t] * 16 + rowBf16(lane, r)] = qs[t][r];
+    }
+  if (tid < kTileCols) {
+    // a.nsteps steps, or fewer when every column reached its horizon (the
+    // same counts), or more under a time budget
+    const uint64_t h = a.horizon[slot0 + tid];
+    const uint64_t st = a.stepCol[slot0 + tid], s = st + (MACRO ? (uint64_t)steps : a.nsteps);
+    a.stepCol[slot0 + tid] = s < h ? s : (st < h ? h : st);
+  }
+}
+
+template <int PARTS, int KG, int WAVES, int RR, int LL, int DR>
+void launchKG(const RomArgs& a, dim3 grid, hipStream_t stream) {
+  constexpr size_t lds = (8 * 32 * KG + (size_t)2 * 2 * KG * LL * PARTS * 64) * 16;
+  static_assert(lds <= 160 * 1024, "LDS of one CU");
+  auto go = [&](auto kernel) {
+    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(kernel, grid, dim3(WAVES * 64), lds, stream, a);
+  };
+  if (a.macro) go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, true>);
+  else go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, false>);
+}
+
+}  // namespace
+
+uint32_t residentModes(int parts, uint64_t kv, uint64_t ks) {
+  const uint64_t k = kv > ks ? kv : ks;
+  return parts == 0 || k > 256 ? 0 : (uint32_t)((k + 63) / 64 * 64);
+}
+
+void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream) {
+  const int kg = (int)a.Kvp / 32;
+  if (parts == 2) {
+    switch (kg) {
+      case 2: launchKG<2, 2, 4, 2, 0, 1>(a, grid, stream); break;
+      case 4: launchKG<2, 4, 8, 4, 0, 1>(a, grid, stream); break;
+      case 6: launchKG<2, 6, 12, 5, 1, 1>(a, grid, stream); break;
+      default: launchKG<2, 8, 8, 3, 2, 1>(a, grid, stream); break;
+    }
+  } else {
+    switch (kg) {
+      case 2: launchKG<3, 2, 4, 2, 0, 1>(a, grid, stream); break;
+      case 4: launchKG<3, 4, 8, 4, 0, 1>(a, grid, stream); break;
+      case 6: launchKG<3, 6, 12, 2, 1, 1>(a, grid, stream); break;
+      default: launchKG<3, 8, 8, 2, 1, 1>(a, grid, stream); break;
+    }
+  }
+}
+
+}  // namespace shaw
