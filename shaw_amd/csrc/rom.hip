@@ -641,11 +641,27 @@ __global__ void __launch_bounds__(256) k_quiet(const double* __restrict__ f, uin
   if (t == 0) quiet[j] = last[0] < 0xffffffffull ? (uint32_t)last[0] : 0xffffffffu;
 }
 
-// admission: column j of the staged inputs (forcing column, series, quiet
-// step) goes to slot slots[j]; its states start at zero
+// out[c * ld + r] = in[r * n + c], r < rows, c < n: a host forcing table's rows
+// (one step each) to per-column series, through a 32 x 33 LDS tile
+__global__ void __launch_bounds__(256) k_transpose(const double* __restrict__ in, uint64_t rows, uint64_t n,
+                                                   double* __restrict__ out, uint64_t ld) {
+  __shared__ double tile[32][33];
+  const uint64_t c0 = (uint64_t)blockIdx.x * 32, x = threadIdx.x % 32, y = threadIdx.x / 32;
+  for (uint64_t r0 = (uint64_t)blockIdx.y * 32; r0 < rows; r0 += (uint64_t)gridDim.y * 32) {
+    for (uint64_t r = y; r < 32; r += 8)
+      if (r0 + r < rows && c0 + x < n) tile[r][x] = in[(r0 + r) * n + c0 + x];
+    __syncthreads();
+    for (uint64_t c = y; c < 32; c += 8)
+      if (c0 + c < n && r0 + x < rows) out[(c0 + c) * ld + r0 + x] = tile[x][c];
+    __syncthreads();
+  }
+}
+
+// admission: column j of the staged inputs (forcing column j of bStage [kv][n],
+// series, quiet step) goes to slot slots[j]; its states start at zero
 __global__ void k_admit_scatter(const uint64_t* __restrict__ slots, uint64_t n, const double* __restrict__ bStage,
                                 const double* __restrict__ fStage, const uint32_t* __restrict__ quietStage,
-                                uint32_t kvp, uint32_t ksp, uint64_t nsteps, uint64_t maxSteps,
+                                uint32_t kv, uint32_t kvp, uint32_t ksp, uint64_t nsteps, uint64_t maxSteps,
                                 double* __restrict__ b, double* __restrict__ ftab, double* __restrict__ qv,
                                 double* __restrict__ qs, uint32_t* __restrict__ quiet) {
   const uint64_t j = blockIdx.y;
@@ -655,7 +671,7 @@ __global__ void k_admit_scatter(const uint64_t* __restrict__ slots, uint64_t n, 
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nsteps; e += (uint64_t)gridDim.x * blockDim.x)
     ftab[s * maxSteps + e] = fStage[j * nsteps + e];
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < kvp; e += (uint64_t)gridDim.x * blockDim.x) {
-    b[s * kvp + e] = bStage[j * kvp + e];
+    b[s * kvp + e] = e < kv ? bStage[e * n + j] : 0.0;
     qv[s * kvp + e] = 0.0;
   }
   for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < ksp; e += (uint64_t)gridDim.x * blockDim.x)
@@ -927,7 +943,8 @@ struct shaw_rom {
   shaw::DevBuf<uint64_t> stepCol, horizon, every;
   std::vector<uint64_t> hStep, hHorizon, hEvery;
   std::vector<uint8_t> used;
-  shaw::DevBuf<double> stage;          // admission inputs, [n][Kvp] then [n][nsteps]
+  shaw::DevBuf<double> stage;          // admission inputs, [kv][n] then [n][nsteps]
+  shaw::DevBuf<double> stageTable;     // rows of a host forcing table (at most 64 MB, or one row)
   shaw::DevBuf<uint64_t> stageSlots;
   void* pinned = nullptr;              // host staging of retired seismograms
   size_t pinnedBytes = 0;
@@ -1336,37 +1353,43 @@ void admit(shaw_rom_t h, uint64_t n, const double* b, uint64_t nsteps, const dou
       std::swap(nb.n, h->ftab.n);
       h->maxSteps = need;
     }
-    // stage [n][Kvp] forcing columns and [n][nsteps] forcing series, one scatter.
-    // With signals only b, the parameters [n][3] (after the series region)
-    // and the slots cross PCIe, from the pinned admission buffer on the
-    // engine's stream, and the series is evaluated on the device.
-    const uint64_t stageNeed = n * (h->kvp + nsteps) + (ftab ? 0 : 3 * n);
+    // stage the forcing columns [kv][n] as they are given and the series
+    // [n][nsteps], one scatter; the transposes run on the device (on one host
+    // thread they took 40 ms of a 4096-column admission of 250 modes). With
+    // signals only b, the parameters [n][3] (after the series region) and the
+    // slots cross PCIe, from the pinned admission buffer on the engine's
+    // stream, and the series is evaluated on the device.
+    const uint64_t stageNeed = n * (h->kv + nsteps) + (ftab ? 0 : 3 * n);
     if (h->stage.n < stageNeed) h->stage.alloc(stageNeed);
+    double* const series = h->stage.p + n * h->kv;
     uint64_t* hSlots = nullptr;  // pinned slots of the signal path
     if (ftab) {
-      std::vector<double> st(n * (h->kvp + nsteps), 0.0);
-      for (uint64_t j = 0; j < n; ++j) {
-        for (uint64_t k = 0; k < h->kv; ++k) st[j * h->kvp + k] = b[k * n + j];
-        double* f = st.data() + n * h->kvp + j * nsteps;
-        for (uint64_t t = 0; t < nsteps; ++t) f[t] = ftab[t * n + j];
+      SHAW_HIP(hipMemcpyAsync(h->stage.p, b, n * h->kv * sizeof(double), hipMemcpyHostToDevice, h->stream));
+      // the table in chunks of at most 64 MB
+      const uint64_t chunk = std::max<uint64_t>(1, std::min<uint64_t>(nsteps, (64ull << 20) / (n * sizeof(double))));
+      if (h->stageTable.n < chunk * n) h->stageTable.alloc(chunk * n);
+      for (uint64_t r0 = 0; r0 < nsteps; r0 += chunk) {
+        const uint64_t rows = std::min(chunk, nsteps - r0);
+        SHAW_HIP(hipMemcpyAsync(h->stageTable.p, ftab + r0 * n, rows * n * sizeof(double), hipMemcpyHostToDevice, h->stream));
+        hipLaunchKernelGGL(k_transpose, dim3((unsigned)((n + 31) / 32), (unsigned)std::min<uint64_t>((rows + 31) / 32, 4096)),
+                           dim3(256), 0, h->stream, h->stageTable.p, rows, n, series + r0, nsteps);
+        SHAW_HIP(hipGetLastError());
       }
-      h->stage.upload(st.data(), st.size());
+      SHAW_HIP(hipStreamSynchronize(h->stream));  // the caller's arrays are done with
     } else {
       const std::vector<double> par = signalParams(n, kinds, delays, periods);
-      double* hb = static_cast<double*>(h->admitStage((n * h->kvp + 3 * n) * sizeof(double) + n * sizeof(uint64_t)));
-      std::fill(hb, hb + n * h->kvp, 0.0);
-      for (uint64_t j = 0; j < n; ++j)
-        for (uint64_t k = 0; k < h->kv; ++k) hb[j * h->kvp + k] = b[k * n + j];
-      std::copy(par.begin(), par.end(), hb + n * h->kvp);
-      hSlots = reinterpret_cast<uint64_t*>(hb + n * h->kvp + 3 * n);
-      double* dPar = h->stage.p + n * (h->kvp + nsteps);
-      SHAW_HIP(hipMemcpyAsync(h->stage.p, hb, n * h->kvp * sizeof(double), hipMemcpyHostToDevice, h->stream));
-      SHAW_HIP(hipMemcpyAsync(dPar, hb + n * h->kvp, 3 * n * sizeof(double), hipMemcpyHostToDevice, h->stream));
-      forcingTableFromParams(n, dPar, h->dt, nsteps, h->stage.p + n * h->kvp, nsteps, h->stream);
+      double* hb = static_cast<double*>(h->admitStage((n * h->kv + 3 * n) * sizeof(double) + n * sizeof(uint64_t)));
+      parallelCopy(hb, b, n * h->kv * sizeof(double));
+      std::copy(par.begin(), par.end(), hb + n * h->kv);
+      hSlots = reinterpret_cast<uint64_t*>(hb + n * h->kv + 3 * n);
+      double* dPar = series + n * nsteps;
+      SHAW_HIP(hipMemcpyAsync(h->stage.p, hb, n * h->kv * sizeof(double), hipMemcpyHostToDevice, h->stream));
+      SHAW_HIP(hipMemcpyAsync(dPar, hb + n * h->kv, 3 * n * sizeof(double), hipMemcpyHostToDevice, h->stream));
+      forcingTableFromParams(n, dPar, h->dt, nsteps, series, nsteps, h->stream);
     }
     // each column's first quiet step, staged; the scatter puts it at the slot
     if (h->quietStage.n < n) h->quietStage.alloc(n);
-    hipLaunchKernelGGL(k_quiet, dim3((unsigned)n), dim3(256), 0, h->stream, h->stage.p + n * h->kvp, nsteps,
+    hipLaunchKernelGGL(k_quiet, dim3((unsigned)n), dim3(256), 0, h->stream, series, nsteps,
                        h->quietStage.p);
     SHAW_HIP(hipGetLastError());
     std::vector<uint64_t> slotOf(free);  // column j -> slot
@@ -1397,7 +1420,7 @@ void admit(shaw_rom_t h, uint64_t n, const double* b, uint64_t nsteps, const dou
       h->stageSlots.upload(slotOf.data(), n);
     }
     hipLaunchKernelGGL(k_admit_scatter, dim3(64, (unsigned)n), dim3(256), 0, h->stream, h->stageSlots.p, n, h->stage.p,
-                       h->stage.p + n * h->kvp, h->quietStage.p, h->kvp, h->ksp, nsteps, h->maxSteps, h->b.p,
+                       series, h->quietStage.p, (uint32_t)h->kv, h->kvp, h->ksp, nsteps, h->maxSteps, h->b.p,
                        h->ftab.p, h->qv.p, h->qs.p, h->quiet.p);
     SHAW_HIP(hipGetLastError());
     for (uint64_t j = 0; j < n; ++j) {
