@@ -144,16 +144,17 @@ __device__ __forceinline__ void halfStep(const RomArgs& a, const void* A, int ro
   }
 }
 
-// The FP64 reduced leapfrog. One workgroup (WAVES waves: 16 when the
-// operators have 9 to 16 row tiles, one tile per wave, which doubles the
-// loads in flight per CU for the same operator stream; else 8) owns
-// kTileCols column slots and advances them a.nsteps steps, states resident
-// in LDS; each wave owns up to TPW row tiles of each operator. Lane l works on column l % 16 in every product, so each
-// lane keeps its column's step counter, horizon, sampling period and next
-// forcing value in registers (the forcing of step s + 1 is loaded during
-// step s); the block-uniform decisions (stop, sample) come from values every
-// wave computes identically, so a step needs only the two barriers between
-// the half-steps.
+// The FP64 reduced leapfrog for the engines and loads that k_rom_f64
+// (rom_f64.hip) does not take: more than 128 active tiles above 128 modes. One
+// workgroup (WAVES waves: 16 when the operators have 9 to 16 row tiles, one
+// tile per wave, which doubles the loads in flight per CU for the same operator
+// stream; else 8) owns kTileCols column slots and advances them a.nsteps steps,
+// states resident in LDS; each wave owns up to TPW row tiles of each operator.
+// Lane l works on column l % 16 in every product, so each lane keeps its
+// column's step counter, horizon, sampling period and next forcing value in
+// registers (the forcing of step s + 1 is loaded during step s); the
+// block-uniform decisions (stop, sample) come from values every wave computes
+// identically, so a step needs only the two barriers between the half-steps.
 template <int PARTS, int TPW, int WAVES>
 __global__ void __launch_bounds__(WAVES * 64) k_rom_steps(RomArgs a) {
   static_assert(PARTS == 0, "the bf16 variants run k_rom_steps_bf");
@@ -1013,6 +1014,16 @@ struct shaw_rom {
   size_t ldsBytes() const {
     return (size_t)(kvp + ksp) * shaw::kTileCols * (precision == SHAW_ROM_FP64 ? sizeof(double) : 4);
   }
+  // tiles of 16 slots with a column short of its horizon
+  uint64_t activeTiles() const {
+    uint64_t n = 0;
+    for (uint64_t t = 0; t < maxCols; t += shaw::kTileCols) {
+      bool any = false;
+      for (uint64_t c = t; c < t + shaw::kTileCols; ++c) any = any || hStep[c] < hHorizon[c];
+      n += any;
+    }
+    return n;
+  }
   void launch(uint64_t nsteps) {
     using namespace shaw;
     RomArgs a{};
@@ -1029,7 +1040,8 @@ struct shaw_rom {
     a.budget = a.macro ? timeBudget : 0;
     const dim3 grid((unsigned)(maxCols / kTileCols));
     const size_t lds = ldsBytes();
-    if (resident) launchRomResident(parts(), a, grid, stream);
+    if (resident && precision != SHAW_ROM_FP64) launchRomResident(parts(), a, grid, stream);
+    else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, maxCols, stream);
     else if (precision == SHAW_ROM_FP64) launchRomSteps<0>(tpw, grid, lds, stream, a);
     else if (precision == SHAW_ROM_BF16X3) launchRomSteps<2>(tpw, grid, lds, stream, a);
     else launchRomSteps<3>(tpw, grid, lds, stream, a);
@@ -1249,7 +1261,7 @@ int shaw_rom_create(const shaw_rom_desc* d, shaw_rom_t* out) {
     const uint32_t kq = (d->precision == SHAW_ROM_FP64 ? 16 : 32) * kRing;
     h->kvp = roundUp(d->kv, kq);
     h->ksp = roundUp(d->ks, kq);
-    h->resident = residentModes(h->parts(), d->kv, d->ks);
+    h->resident = residentModes(h->parts(), d->kv, d->ks, d->max_cols);
     if (h->resident) h->kvp = h->ksp = h->resident;
     h->rp = roundUp(std::max<uint64_t>(d->r, 1), 16);
     h->maxCols = roundUp(d->max_cols, kTileCols);

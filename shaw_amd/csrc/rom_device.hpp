@@ -176,6 +176,27 @@ __device__ __forceinline__ void launchPlan(const RomArgs& a, uint32_t s0, uint32
   mk2Out = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)mk2);
 }
 
+// Where a step reads the operators' k-groups from: RR groups of every row tile
+// sit in registers, LL in LDS, the other KG - RR - LL stream from L2 through a
+// ring of DR groups. The streamed groups are spread evenly, so the products of
+// the resident ones hide each refill.
+template <int KG, int RR, int LL, int DR>
+struct Place {
+  static constexpr int S = KG - RR - LL;
+  static constexpr int group(int s) { return s * KG / (S > 0 ? S : 1); }  // the s-th streamed group
+  static constexpr bool streamed(int g) {
+    for (int q = 0; q < S; ++q)
+      if (group(q) == g) return true;
+    return false;
+  }
+  // index of group g among those of its kind (streamed, or not: LDS first)
+  static constexpr int index(int g) {
+    int n = 0;
+    for (int q = 0; q < g; ++q) n += streamed(q) == streamed(g);
+    return n;
+  }
+};
+
 constexpr int kRing = 4;  // operator groups kept in flight per row tile
 
 // PARTS = 0: FP64 operators; 2: bf16 hi + lo (BF16x3); 3: bf16 hi + lo +

@@ -56,12 +56,17 @@ void macroOperator(const double* arV, const double* arS, uint64_t kv, uint64_t k
                    std::vector<double>& gss);
 void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t kout, double* out,
             const double* base, double alpha, hipStream_t stream);
-// rom_resident.hip: the padded modes per dof (a multiple of 64) when a BF16
-// engine's operators (parts = 2 or 3 bf16 parts) stay on the CU, else 0; the
-// launch of such an engine (a.Kvp = a.Ksp = that size), only enqueued
+// The padded modes per dof of an engine whose operators stay on the CU as far
+// as they fit (parts: 0 FP64, else the bf16 parts; cols: column slots), 0 where
+// k_rom_steps* run it. Such an engine has a.Kvp = a.Ksp = that size and runs
+// launchRomResident (BF16, rom_resident.hip) or launchRomF64 (FP64, rom_f64.hip;
+// romF64Fits says whether that is the faster kernel for the active tiles of 16
+// columns, k_rom_steps taking the same operators with the same results).
 struct RomArgs;
-uint32_t residentModes(int parts, uint64_t kv, uint64_t ks);
+uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols);
 void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream);
+bool romF64Fits(uint32_t modes, uint64_t activeTiles);
+void launchRomF64(const RomArgs& a, uint64_t cols, hipStream_t stream);
 uint64_t projPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);
 uint32_t gramChunks(uint64_t n, uint64_t Ka, uint64_t Kb);
 uint64_t gramPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);

@@ -32,27 +32,6 @@ __device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, in
   reinterpret_cast<u2*>(S + loOff + item)[rt % 2] = l;
 }
 
-// Where a step reads the operators' k-groups from: RR groups of every row tile
-// sit in registers, LL in LDS, the other KG - RR - LL stream from L2 through a
-// ring of DR groups. The streamed groups are spread evenly, so the products of
-// the resident ones hide each refill.
-template <int KG, int RR, int LL, int DR>
-struct Place {
-  static constexpr int S = KG - RR - LL;
-  static constexpr int group(int s) { return s * KG / (S > 0 ? S : 1); }  // the s-th streamed group
-  static constexpr bool streamed(int g) {
-    for (int q = 0; q < S; ++q)
-      if (group(q) == g) return true;
-    return false;
-  }
-  // index of group g among those of its kind (streamed, or not: LDS first)
-  static constexpr int index(int g) {
-    int n = 0;
-    for (int q = 0; q < g; ++q) n += streamed(q) == streamed(g);
-    return n;
-  }
-};
-
 // One workgroup advances 16 column slots as k_rom_steps_bf / k_rom_steps_bfm
 // do (same splits, products and FP64 updates in the same order, so every value
 // is theirs); here both operators, 2 KG row tiles by KG groups, are loaded into
@@ -359,9 +338,15 @@ void launchKG(const RomArgs& a, dim3 grid, hipStream_t stream) {
 
 }  // namespace
 
-uint32_t residentModes(int parts, uint64_t kv, uint64_t ks) {
+uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols) {
   const uint64_t k = kv > ks ? kv : ks;
-  return parts == 0 || k > 256 ? 0 : (uint32_t)((k + 63) / 64 * 64);
+  // FP64 pads both dofs alike where k_rom_f64 runs them whatever the load, or
+  // where that costs k_rom_steps nothing
+  if (parts == 0 && cols > 2048 && k > 128 && (kv + 63) / 64 != (ks + 63) / 64) return 0;
+  if (k <= 256) return (uint32_t)((k + 63) / 64 * 64);
+  // K = 384, 2048 columns: 35.4 us a step against 38.2; K = 512 1024 columns
+  // 34.5 against 65.6, 2048 67.1 against 65.5
+  return parts == 0 && cols <= (k <= 384 ? 2048 : 1024) ? (k <= 384 ? 384 : 512) : 0;
 }
 
 void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream) {
