@@ -550,13 +550,15 @@ def main() -> int:
     value = w.m * args.steps / (total_ms / 1000.0)
     log(f"{total_ms:.2f} ms for {args.steps} steps -> {ms_per_step:.4f} ms/step, {value:.0f} forcing-steps/s")
     kernel_bytes, model_bytes = fom.bytes_per_step()
-    cfg = fom.config()
-    spl = cfg["steps_per_launch"]  # a launch of the k-step kernel advances k steps
+    bytes_per_launch = kernel_bytes * fom.config()["steps_per_launch"]  # whatever a launch's steps
+    # the launches as planned: k steps and rows per segment
+    shape = fom.launch_shape(ROOF_STEPS)
+    spl = shape["steps_per_launch"]
+    cfg = {**fom.config(), "steps_per_launch": spl, "segment": shape["segment"]}
     # the dominant kernel alone: whole launches, HIP events on the FOM stream
     roof_launches = ROOF_STEPS // spl
     roof_ms, _ = fom.time(roof_launches * spl)
     launch_ms = roof_ms / roof_launches
-    bytes_per_launch = kernel_bytes * spl
     achieved = bytes_per_launch / (launch_ms / 1000.0) / 1e9
     log(f"{roof_launches} launches of {spl} steps: {launch_ms:.4f} ms per launch, {achieved:.0f} GB/s algorithmic "
         f"({bytes_per_launch / 1e9:.3f} GB per launch), {roof_launches * spl / (roof_ms / 1e3) * w.m:.0f} "
@@ -569,7 +571,7 @@ def main() -> int:
     seis = fom.seismogram()
     assert np.isfinite(seis).all(), "seismogram is not finite"
 
-    traffic = measured_traffic(fom.config())
+    traffic = measured_traffic(cfg)
     out = {
         "metric": METRIC,
         "value": value,

@@ -170,9 +170,10 @@ typedef struct {
                            falls back to fewer steps per launch; the last steps of a
                            run (up to two 7-step launches on one-wavefront strips)
                            go in as few, evenly split launches
-                           (with every tile option at its default, grids whose states
-                           stay in the last-level cache run the window-tile kernel, 6 to
-                           16 steps per launch, instead: same results bit for bit)     */
+                           (with every tile option at its default the launches are
+                           planned from the grid instead, window tiles of 6 to 16
+                           steps or strips of 4 to 7: shaw_fom_launch_shape; same
+                           results bit for bit)                                        */
   int graph_steps;      /* 0 = default (64, rounded up to an even number of launches);
                            < 0: no graphs. Fused kernel without snapshots: whole chunks
                            of this many steps replay one captured HIP graph (kernels
@@ -249,6 +250,12 @@ int shaw_fom_bytes_per_step(shaw_fom_t h, double* kernel_bytes, double* model_by
  * prefetch_rows, steps_per_launch, col_block (any pointer may be null). */
 int shaw_fom_config(shaw_fom_t h, int* kernel, int* cols_per_thread, int* strip, int* segment,
                     int* prefetch_rows, int* steps_per_launch, int* col_block);
+/* How an advance by nsteps (without snapshots) is launched: launches, leapfrog
+ * steps of the longest one and its rows per segment (0: window tiles). With the
+ * tile options at their defaults these are planned from the grid and the column
+ * count and differ from shaw_fom_config's shape, which is the one that
+ * explicit options, the autotuner and graphs start from (any may be null). */
+int shaw_fom_launch_shape(shaw_fom_t h, uint64_t nsteps, uint64_t* launches, int* steps, int* segment);
 /* Tile autotuner of the fused kernel (no counterpart in the reference, whose
  * launch shapes are fixed Kokkos policies): times every valid (columns per
  * thread, strip, segment, rows prefetched, steps per launch) for

@@ -109,6 +109,7 @@ def lib():
         "shaw_fom_complexity": (i32, [u64, u64, u64, u64, u64, i32, P(dbl), P(dbl)]),
         "shaw_fom_bytes_per_step": (i32, [vp, P(dbl), P(dbl)]),
         "shaw_fom_config": (i32, [vp, P(i32), P(i32), P(i32), P(i32), P(i32), P(i32), P(i32)]),
+        "shaw_fom_launch_shape": (i32, [vp, u64, P(u64), P(i32), P(i32)]),
         "shaw_fom_autotune": (i32, [vp, u64, P(C.c_double)]),
         "shaw_fom_destroy": (None, [vp]),
         "shaw_fom_pod": (i32, [vp, i32, u64, vp, vp]),
@@ -513,6 +514,13 @@ class Fom:
         ms = C.c_double()
         _check(lib().shaw_fom_autotune(self._h, trial_steps, C.byref(ms)))
         return ms.value
+
+    def launch_shape(self, nsteps: int):
+        """How an advance by nsteps is launched: launches, steps of the longest
+        and its rows per segment (0: window tiles)."""
+        n, steps, seg = C.c_uint64(), C.c_int(), C.c_int()
+        _check(lib().shaw_fom_launch_shape(self._h, nsteps, C.byref(n), C.byref(steps), C.byref(seg)))
+        return {"launches": int(n.value), "steps_per_launch": steps.value, "segment": seg.value}
 
     def config(self):
         v = [C.c_int() for _ in range(7)]

@@ -29,7 +29,7 @@
 //  * k_fused2 / k_fusedN: two, three or four steps per launch, the
 //    intermediate levels kept in registers and LDS, so the states are read
 //    and written once per launch (recomputed halo rows and points).
-//  * k_fusedW: three to six steps per launch when a 64-point strip is one
+//  * k_fusedW: three to seven steps per launch when a 64-point strip is one
 //    wavefront (one thread per point, all columns of a 1- or 2-column block);
 //    neighbours move between lanes, and the waves of a workgroup share only
 //    a coefficient ring. The default: six steps per launch.
@@ -1232,7 +1232,7 @@ __global__ void __launch_bounds__(256) k_fusedW(StepArgsN<T, NS> aa) {
 
 // ------------------------------------------------------------ window tiles
 // k_tile: a.steps leapfrog steps of one window of the grid per workgroup, for
-// grids whose states stay in the last-level cache. There a launch of the
+// grids that stay in the last-level cache. There a launch of the
 // marching kernels is a chain of latencies rather than a stream (a k_fusedW
 // strip loads its rows one after another: 14-16 us per four steps at 21 x 51
 // as at 200 x 1000). A window is 64
@@ -1251,8 +1251,8 @@ __global__ void __launch_bounds__(256) k_fusedW(StepArgsN<T, NS> aa) {
 // velocity row north of a wave's last as well saves one and was slower (0.57
 // against 0.50 us a step at 21 x 51, its arithmetic costs more than the
 // barrier). Measured, us per step, k_fusedW before and k_tile now: 21 x 51
-// M = 1 3.72 -> 0.50; 200 x 1000 M = 1 4.17 -> 1.42; 256 x 1024 M = 4 9.17 ->
-// 4.04, M = 16 15.9 -> 13.0; 509 x 2051 M = 8 36.4 -> 28.7.
+// M = 1 3.72 -> 0.50; 200 x 1000 M = 1 4.17 -> 1.37; 256 x 1024 M = 4 9.17 ->
+// 4.0, M = 8 11.2 -> 6.9; 509 x 2051 M = 1 14.9 -> 5.8.
 // Every value is the one-step kernel's expression in its order. Where it
 // clamps a neighbour at the mesh's edge (a merged coefficient beside a zero
 // one), the merged coefficient moves to the neighbour that exists.
@@ -1583,6 +1583,7 @@ struct shaw_fom {
   virtual void timeChunks(uint64_t nsteps, uint64_t chunk, double* ms) = 0;
   virtual void bytes(double* kernel, double* model) const = 0;
   virtual void config(int* kernel, int* cpt, int* strip, int* seg, int* pf, int* spl, int* colBlock) const = 0;
+  virtual void launchShape(uint64_t nsteps, uint64_t* launches, int* steps, int* segment) const = 0;
   virtual void pod(int dof, uint64_t k, const double* w, double* phi, double* sigma) = 0;
   // POD into a device buffer dPhi [n x k]; podSize: snapshots of the dof (n: rows)
   virtual void podTo(int dof, uint64_t k, const double* w, double* dPhi, double* sigma) = 0;
@@ -1675,7 +1676,7 @@ class FomEngine final : public shaw_fom {
       setStrips();
       const bool asked = o.cols_per_thread > 0 || o.strip > 0 || o.segment > 0 || o.prefetch_rows > 0 ||
                          o.steps_per_launch > 0 || o.col_block > 0;
-      if (!asked) planTile();
+      if (!asked) plan();
     }
     SHAW_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
     SHAW_HIP(hipEventCreate(&ev0_));
@@ -1825,8 +1826,10 @@ class FomEngine final : public shaw_fom {
       return;
     }
     // whole chunks of graphStep_ steps replay one captured graph (fused
-    // kernels, no snapshots: a snapshot kernel would depend on the step)
-    const bool graphs = graphSteps_ > 0 && kernel_ == SHAW_KERNEL_FUSED && !snap_[0].ncols && !snap_[1].ncols &&
+    // kernels, no snapshots: a snapshot kernel would depend on the step);
+    // planned packs run eagerly: their launches last far longer than the host
+    // takes to enqueue one
+    const bool graphs = graphSteps_ > 0 && !packSteps_ && kernel_ == SHAW_KERNEL_FUSED && !snap_[0].ncols && !snap_[1].ncols &&
                         nsteps >= (uint64_t)graphSteps_;
     if (graphs) {
       ensureGraph();
@@ -1849,7 +1852,12 @@ class FomEngine final : public shaw_fom {
     for (; k < nsteps;) {
       const uint64_t left = nsteps - k;
       int ns = spl_;
-      if (spl_ >= 3) {
+      if (packSteps_) {  // up to the next snapshot or the end in as few, evenly split launches
+        uint64_t to = left;
+        for (int d = 0; d < 2; ++d)
+          if (snap_[d].ncols) to = std::min(to, snap_[d].every - step_ % snap_[d].every);
+        ns = (int)packOf(to);
+      } else if (spl_ >= 3) {
         const uint64_t top = longestPack();
         if (left <= top) ns = (int)left;                           // one launch
         else if (left <= 2 * top) ns = (int)((left + 1) / 2);      // two, balanced
@@ -2101,6 +2109,16 @@ class FomEngine final : public shaw_fom {
     if (pf) *pf = pf_;
     if (spl) *spl = kernel_ == SHAW_KERNEL_FUSED ? spl_ : 1;
   }
+  // of an advance by nsteps without snapshots
+  void launchShape(uint64_t nsteps, uint64_t* launches, int* steps, int* segment) const override {
+    const uint32_t top = tile_.steps ? tile_.steps : packSteps_ ? packSteps_ : kernel_ == SHAW_KERNEL_FUSED ? spl_ : 1;
+    const bool whole = tile_.steps && nth_ <= 64 && nr_ <= kTileWaves * tile_.rows;
+    const uint64_t n = whole ? 1 : (nsteps + top - 1) / top;
+    const uint64_t len = n ? (nsteps + n - 1) / n : 0;
+    if (launches) *launches = n;
+    if (steps) *steps = (int)len;
+    if (segment) *segment = tile_.steps ? 0 : packSteps_ && len <= (uint64_t)kMaxSpl && packSeg_[len] ? (int)packSeg_[len] : (int)SEG_;
+  }
 
  private:
   struct Snap {
@@ -2168,6 +2186,7 @@ class FomEngine final : public shaw_fom {
     struct Cfg { int cpt; uint32_t P, SEG; int pf, spl; };
     Cfg best{cpt_, P_, SEG_, pf_, spl_};
     double bestT = 1e300, tileT = 1e300;
+    packSteps_ = 0;  // the trials' shapes rule from here on
     if (tile_.steps && step_ + tile_.steps <= ftabSteps_ && step_ + tile_.steps < (1ull << 32)) {
       launchTile(tile_.steps, true);
       SHAW_HIP(hipEventRecord(ev0_, stream_));
@@ -2365,6 +2384,11 @@ class FomEngine final : public shaw_fom {
     }
     if constexpr (CPT <= 2) {
       if (waveStrip(CPT, P_)) {
+        if (packSteps_ && packSeg_[NS])
+          for (int l = 0; l < NS; ++l) {
+            aa.s[l].SEG = packSeg_[NS];
+            aa.s[l].nSegs = (uint32_t)((nr_ + packSeg_[NS] - 1) / packSeg_[NS]);
+          }
         switch (waveGroup()) {
           case 1: launchWave<CPT, NS, 1>(aa); break;
           case 2: launchWave<CPT, NS, 2>(aa); break;
@@ -2393,7 +2417,7 @@ class FomEngine final : public shaw_fom {
   }
   template <int CPT, int NS, int G>
   void launchWave(StepArgsN<T, NS>& aa) {
-    const unsigned blocks = nStripsK_[NS] * nSegs_ * ((nb_ + G - 1) / G);
+    const unsigned blocks = nStripsK_[NS] * aa.s[0].nSegs * ((nb_ + G - 1) / G);
     if constexpr (NS <= 4) {
       if (pf_ == 2) {
         hipLaunchKernelGGL((k_fusedW<T, CPT, NS, 2, G>), dim3(blocks), dim3(G * 64), ldsBytesW(NS), stream_, aa);
@@ -2449,6 +2473,10 @@ class FomEngine final : public shaw_fom {
     }
     step_ = stepNo;
   }
+  // planned k_fusedW packs (default tile options only): steps per launch (0:
+  // spl_ and SEG_ rule) and the segment of a launch of each length
+  int packSteps_ = 0;
+  uint32_t packSeg_[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   // k_tile (default tile options only): rows per wave (12 waves), steps per
   // launch (0: the marching kernels run) and column blocks per workgroup
   struct Tile {
@@ -2463,8 +2491,9 @@ class FomEngine final : public shaw_fom {
   // then per column block loads and stores the states and takes its steps;
   // ceil(workgroups / CUs) of them run one after another on a CU. The
   // constants are a fit to 900 timed launches (21 x 51 to 1024 x 4096, 1 to 48
-  // columns, both precisions; standard deviation 10 %), whose pick was within
-  // 4 % of the fastest measured one on 33 of 38 grids and 8 % on all.
+  // columns, both precisions; standard deviation 10 %; the larger grids were
+  // 5 to 14 % slower than it, hence 1.08), whose pick was within 4 % of the
+  // fastest measured one on 33 of 38 grids and 8 % on all.
   double tileCost(const Tile& t) const {
     const uint32_t rows = kTileWaves * t.rows;
     const bool whole = nth_ <= 64 && nr_ <= rows;
@@ -2472,25 +2501,79 @@ class FomEngine final : public shaw_fom {
     const double kb100 = rows * 64.0 * sizeof(T) / 1e5, steps = whole ? 200 : t.steps;
     const double step = 0.095 * t.rows * MC_ + 0.27;
     const double block = 4.26 * 3 * MC_ * kb100 + steps * step;
-    return (0.8 + ((wg + 255) / 256) * (3.2 * 8 * kb100 + std::min(t.cbPer, nb_) * block)) / steps;
+    return 1.08 * (0.8 + ((wg + 255) / 256) * (3.2 * 8 * kb100 + std::min(t.cbPer, nb_) * block)) / steps;
   }
-  // The tile kernel where one copy of the states is at most 240 MB (FP64) or
-  // 42 MB (FP32): 509 x 2051 M = 8 (200 MB) 36.4 us/step marching, 28.7 tiled;
-  // M = 16 (400 MB) 48.6 and 63.3, the marching kernel then being the one that
-  // moves fewer bytes; FP32 256 x 1024 M = 12 (38 MB) 9.2 and 7.0, M = 16
-  // (50 MB) 9.4 and 9.7. Fewer than 6 steps a launch never won.
-  void planTile() {
-    const double state = 3.0 * (double)nVp_ * nb_ * MC_ * sizeof(T);
-    if (MC_ > 2 || !fits32() || state > (sizeof(T) == 8 ? 240e6 : 42e6)) return;
-    double best = 1e300;
-    for (uint32_t rows = 2; rows <= 4; ++rows)
-      for (uint32_t steps = 6; steps <= 16 && 2 * steps < kTileWaves * rows; steps += 2)
-        for (uint32_t cb = 1; cb <= 4; cb *= 2) {
-          if (cb > 1 && cb > nb_) continue;
-          const Tile t{rows, steps, cb};
-          const double c = tileCost(t);
-          if (c < best) { best = c; tile_ = t; }
+  // both copies of the states and the coefficients in (about) the last-level
+  // cache of 256 MB
+  bool inCache() const { return (6.0 * MC_ * nb_ + 8.0) * sizeof(T) * (double)nVp_ < 300e6; }
+  // Which kernel and launch shape run a FOM whose tile options are all at their
+  // defaults: k_tile (tile_) or k_fusedW with the pack length and segments
+  // planned here (packSteps_, packSeg_), by their estimated times per step.
+  void plan() {
+    if (MC_ > 2 || !fits32()) return;
+    double march = 1e300;
+    if (waveStrip(cpt_, P_)) {
+      for (int ns = 4; ns <= kMaxSpl; ++ns) {
+        double best = 1e300;
+        for (uint64_t n = 1; n <= nr_; ++n) {
+          const uint32_t seg = (uint32_t)((nr_ + n - 1) / n);
+          if (seg > 192) continue;
+          if (seg < 4 && n > 1) break;
+          const double c = marchCost(ns, seg);
+          if (c < best) { best = c; packSeg_[ns] = seg; }
         }
+        if (best < march) { march = best; packSteps_ = ns; }
+      }
+    }
+    // k_tile where everything stays in the last-level cache (FP32: one copy of
+    // the states at most 42 MB), where its estimate holds, and that is the
+    // lower one: 256 x 1024 M = 8 6.9 us a step against 8.9 marching, 509 x 2051
+    // M = 1 5.8 against 8.4, but 509 x 2051 M = 4 14.0 and 12.5; past the cache
+    // 1024 x 4096 M = 2 37.4 and 30.1, 509 x 2051 M = 8 28.7 and 21.4. Fewer than
+    // 6 steps a launch never won.
+    const double state = 3.0 * (double)nVp_ * nb_ * MC_ * sizeof(T);
+    if (inCache() && (sizeof(T) == 8 || state <= 42e6)) {
+      double best = march;
+      for (uint32_t rows = 2; rows <= 4; ++rows)
+        for (uint32_t steps = 6; steps <= 16 && 2 * steps < kTileWaves * rows; steps += 2)
+          for (uint32_t cb = 1; cb <= 4; cb *= 2) {
+            if (cb > 1 && cb > nb_) continue;
+            const Tile t{rows, steps, cb};
+            const double c = tileCost(t);
+            if (c < best) { best = c; tile_ = t; }
+          }
+    }
+  }
+  // Microseconds per step of k_fusedW at ns steps a launch in segments of seg
+  // rows: every wave marches seg + 2 ns - 1 rows. The chip holds 2 (FP64) or 4
+  // (FP32) waves a SIMD, so a launch takes whole rounds of them. A row takes
+  // its loads and levels (0.7 + 0.2 ns us, less for one-column blocks) while the
+  // SIMDs are half empty. When they fill the chip it takes 2.5 (FP32 2.85)
+  // us from HBM, whatever ns, in proportion to what a wave row loads; from the
+  // last-level cache 1 + 0.22 ns (FP32 0.28 ns), the share of the coefficients
+  // counting less. Full rounds overlap by 12 %. Fitted to sweeps of packs and
+  // segments on 18 grids (200 x 1000 to 2048 x 8192, 1 to 48 columns). Per
+  // step, the plan against the former six steps in 64 or 128 rows: 1024 x 4096
+  // M = 32 233 us (seven steps, 171 rows) and 258; 509 x 2051 M = 15 36.1 (85
+  // rows, one round) and 47.9; 2048 x 8192 M = 8 FP32 142 and 157.
+  double marchCost(int ns, uint32_t seg) const {
+    const uint32_t g = waveGroup();
+    const uint64_t waves = (uint64_t)nStripsK_[ns] * ((nr_ + seg - 1) / seg) * ((nb_ + g - 1) / g) * g;
+    const uint64_t slots = sizeof(T) == 8 ? 2048 : 4096, rounds = (waves + slots - 1) / slots;
+    const double full = inCache() ? 1.0 + (sizeof(T) == 8 ? 0.22 : 0.28) * ns : sizeof(T) == 8 ? 2.5 : 2.85;
+    const double lone = (0.7 + 0.2 * ns) * (MC_ == 1 ? 0.8 : 1.0);
+    double bytes = (24.0 * MC_ + 64.0 / g) / 64.0;
+    if (inCache() && MC_ == 2) bytes = 1.0 + 0.6 * (bytes - 1.0);
+    const double fill = (double)waves / slots;
+    const double row = rounds > 1      ? 0.88 * rounds * full * bytes
+                       : fill > 0.5   ? std::max(lone, (0.7 + 0.3 * fill) * full * bytes)
+                                       : std::max(lone, fill * full * bytes);
+    return row * (seg + 2 * ns - 1) / ns;
+  }
+  // steps of the next planned pack when `left` steps are to go
+  uint64_t packOf(uint64_t left) const {
+    const uint64_t n = (left + packSteps_ - 1) / packSteps_;
+    return n ? (left + n - 1) / n : 0;
   }
   // one launch of at most `left` steps, evenly split up to the next snapshot
   // or the end of the run; returns its steps. A trial records nothing and
@@ -2686,6 +2769,12 @@ int shaw_fom_time_chunks(shaw_fom_t h, uint64_t nsteps, uint64_t chunk, double* 
   return guarded([&] {
     SHAW_REQUIRE(h && chunk_ms && chunk > 0, SHAW_ERR_ARG, "bad argument");
     h->timeChunks(nsteps, chunk, chunk_ms);
+  });
+}
+int shaw_fom_launch_shape(shaw_fom_t h, uint64_t nsteps, uint64_t* launches, int* steps, int* segment) {
+  return guarded([&] {
+    SHAW_REQUIRE(h, SHAW_ERR_ARG, "null handle");
+    h->launchShape(nsteps, launches, steps, segment);
   });
 }
 int shaw_fom_bytes_per_step(shaw_fom_t h, double* kernel, double* model) {

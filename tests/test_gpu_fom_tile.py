@@ -67,3 +67,37 @@ def test_tiles_equal_single_steps(nr, nth, m, precision):
     for x, y in zip(*out):
         np.testing.assert_array_equal(x, y)
     assert np.abs(out[0][1]).max() > 0
+
+
+@pytest.mark.parametrize("n,every", [(75, (5, 25, 15)), (33, (1, 0, 0)), (8, (2, 4, 8))])
+def test_planned_packs_equal_oracle(n, every):
+    """A grid on which the default options plan marching strips of their own
+    pack length and segments: runs split evenly, up to snapshots too."""
+    say(f"[gpu] planned packs n={n} every={every}")
+    nr, nth, m = 200, 1000, 24
+    rng = np.random.default_rng(n)
+    app = shaw_amd.App.structured(nr, nth, LAYERED)
+    fom = shaw_amd.Fom(app, m, 0.25)
+    shape = fom.launch_shape(n)
+    fom.close()
+    assert shape["segment"] > 0 and 4 <= shape["steps_per_launch"] <= 7
+    ora = oracle.App("", LAYERED, structured=(nr, nth, 0.0, 180.0, 3480.0, 6371.0))
+    src = random_sources(rng, m, 600.0)
+    rec = list(range(0, 180, 7))
+    a = shaw_amd.fom_run(app, 0.25, n, src, True, rec, *every)
+    b = ora.fom_run(0.25, n, src, True, rec, *every)
+    for key in b:
+        np.testing.assert_array_equal(a[key], b[key], err_msg=key)
+
+
+def test_planned_packs_fp32_equal_single_steps():
+    say("[gpu] planned packs FP32")
+    nr, nth, m, n = 200, 1000, 24, 60
+    rng = np.random.default_rng(3)
+    app = shaw_amd.App.structured(nr, nth, LAYERED)
+    src = random_sources(rng, m, 600.0)
+    rec = list(range(0, 180, 7))
+    a = shaw_amd.fom_run(app, 0.25, n, src, True, rec, 3, 20, 12, precision=shaw_amd.FP32)
+    b = shaw_amd.fom_run(app, 0.25, n, src, True, rec, 3, 20, 12, precision=shaw_amd.FP32, steps_per_launch=1)
+    for key in b:
+        np.testing.assert_array_equal(a[key], b[key], err_msg=key)
