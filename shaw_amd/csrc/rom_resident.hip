@@ -344,9 +344,13 @@ uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols) {
   // where that costs k_rom_steps nothing
   if (parts == 0 && cols > 2048 && k > 128 && (kv + 63) / 64 != (ks + 63) / 64) return 0;
   if (k <= 256) return (uint32_t)((k + 63) / 64 * 64);
-  // K = 384, 2048 columns: 35.4 us a step against 38.2; K = 512 1024 columns
-  // 34.5 against 65.6, 2048 67.1 against 65.5
-  return parts == 0 && cols <= (k <= 384 ? 2048 : 1024) ? (k <= 384 ? 384 : 512) : 0;
+  const uint32_t modes = k <= 384 ? 384 : 512;
+  // BF16: nearly all of the operators stream, and a square pad of unequal dofs
+  // would add to it
+  if (parts) return (kv + 127) / 128 == (ks + 127) / 128 ? modes : 0;
+  // FP64: K = 384, 2048 columns: 35.4 us a step against 38.2; K = 512 1024
+  // columns 34.5 against 65.6, 2048 67.1 against 65.5
+  return cols <= (k <= 384 ? 2048 : 1024) ? modes : 0;
 }
 
 void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream) {
@@ -356,14 +360,18 @@ void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t strea
       case 2: launchKG<2, 2, 4, 2, 0, 1>(a, grid, stream); break;
       case 4: launchKG<2, 4, 8, 4, 0, 1>(a, grid, stream); break;
       case 6: launchKG<2, 6, 12, 5, 1, 1>(a, grid, stream); break;
-      default: launchKG<2, 8, 8, 3, 2, 1>(a, grid, stream); break;
+      case 8: launchKG<2, 8, 8, 3, 2, 1>(a, grid, stream); break;
+      case 12: launchKG<2, 12, 8, 1, 1, 1>(a, grid, stream); break;
+      default: launchKG<2, 16, 8, 0, 0, 1>(a, grid, stream); break;
     }
   } else {
     switch (kg) {
       case 2: launchKG<3, 2, 4, 2, 0, 1>(a, grid, stream); break;
       case 4: launchKG<3, 4, 8, 4, 0, 1>(a, grid, stream); break;
       case 6: launchKG<3, 6, 12, 2, 1, 1>(a, grid, stream); break;
-      default: launchKG<3, 8, 8, 2, 1, 1>(a, grid, stream); break;
+      case 8: launchKG<3, 8, 8, 2, 1, 1>(a, grid, stream); break;
+      case 12: launchKG<3, 12, 8, 0, 0, 2>(a, grid, stream); break;
+      default: launchKG<3, 16, 8, 0, 0, 1>(a, grid, stream); break;
     }
   }
 }
