@@ -49,6 +49,7 @@ struct ProjArgs {
   double* part;        // [nch][Ka][Kb]
   uint64_t n, nX, chunk;
   uint32_t Ka, Kb, nr, nth;
+  int symmetric;       // L = X, unweighted: tiles below the diagonal are skipped
 };
 
 __device__ __forceinline__ dbl4 mfma64(double a, double b, dbl4 c) {
@@ -100,6 +101,7 @@ __global__ void __launch_bounds__(256) k_proj_tn(ProjArgs p) {
   __shared__ double Ls[kRows][kTile + 1];
   __shared__ double Js[kRows][kTile + 1];
   const uint32_t a0 = blockIdx.x * kTile, b0 = blockIdx.y * kTile, ch = blockIdx.z;
+  if (OP == 2 && p.symmetric && a0 > b0) return;  // k_sum_chunks mirrors tile (b0, a0)
   const uint64_t r0 = (uint64_t)ch * p.chunk;
   const uint64_t r1 = r0 + p.chunk < p.n ? r0 + p.chunk : p.n;
   const int t = threadIdx.x, rr = t % kRows, cg = t / kRows;  // staging: one row, 8 column groups
@@ -111,41 +113,53 @@ __global__ void __launch_bounds__(256) k_proj_tn(ProjArgs p) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
 
-  for (uint64_t rb = r0; rb < r1; rb += kRows) {
+  // A stage's loads are issued during the products of the stage before it:
+  // workgroups are few where the output is small (64 x 64 modes: 64 of them),
+  // so nothing else hides them. 64 x 64 modes at 256 x 1024 points, J_sp / J_vp:
+  // 2280 / 1394 -> 678 / 502 us; Gram products of 200 snapshots (also without
+  // the tiles below the diagonal) 1498 -> 639 us on average.
+  constexpr int U = kTile / 8, NX = OP == 0 ? 4 : OP == 1 ? 2 : 1;
+  double lv[U], xv[NX][U], cf[4], wr = 1.0;
+  bool live = false;
+  auto fetch = [&](uint64_t rb) {
     const uint64_t r = rb + rr;
-    const bool live = r < r1;
+    live = r < r1;
     uint64_t nb[4] = {0, 0, 0, 0};
-    double cf[4] = {0.0, 0.0, 0.0, 0.0};
-    double wr = 1.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) cf[q] = 0.0;
+    wr = 1.0;
     if (live) {
       stencilRow<OP>(p, r, nb, cf);
       if (p.w) wr = p.w[r];
     }
 #pragma unroll
-    for (int u = 0; u < kTile / 8; ++u) {
+    for (int u = 0; u < U; ++u) {
       const uint32_t c = cg + 8 * u;
-      double lv = 0.0, jv = 0.0;
-      if (live && a0 + c < p.Ka) {
-        const double x = p.L[r + p.n * (a0 + c)];
-        lv = p.w ? wr * x : x;
-      }
-      if (live && b0 + c < p.Kb) {
-        const double* x = p.X + p.nX * (b0 + c);
+      lv[u] = live && a0 + c < p.Ka ? p.L[r + p.n * (a0 + c)] : 0.0;
+      const double* x = p.X + p.nX * (b0 + c);
+      const bool on = live && b0 + c < p.Kb;
+#pragma unroll
+      for (int q = 0; q < NX; ++q) xv[q][u] = on ? x[OP == 2 ? r : nb[q]] : 0.0;
+    }
+  };
+  fetch(r0);
+  for (uint64_t rb = r0; rb < r1; rb += kRows) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t c = cg + 8 * u;
+      double jv = xv[0][u];
+      if constexpr (OP < 2) {
+        jv = cf[0] * xv[0][u] + cf[1] * xv[1][u];
         if constexpr (OP == 0) {
-          double s = cf[0] * x[nb[0]] + cf[1] * x[nb[1]];
-          s = s + cf[2] * x[nb[2]];
-          s = s + cf[3] * x[nb[3]];
-          jv = s;
-        } else if constexpr (OP == 1) {
-          jv = cf[0] * x[nb[0]] + cf[1] * x[nb[1]];
-        } else {
-          jv = x[r];
+          jv = jv + cf[2] * xv[2][u];
+          jv = jv + cf[3] * xv[3][u];
         }
       }
-      Ls[rr][c] = lv;
+      Ls[rr][c] = p.w ? wr * lv[u] : lv[u];
       Js[rr][c] = jv;
     }
     __syncthreads();
+    if (rb + kRows < r1) fetch(rb + kRows);
 #pragma unroll
     for (int kk = 0; kk < kRows / 4; ++kk) {
       // A operand: lane l holds A[l % 16][l / 16] = L[row 4kk + l/16][col l % 16]
@@ -176,10 +190,12 @@ __global__ void __launch_bounds__(256) k_proj_tn(ProjArgs p) {
 // out[r + n c] = base + alpha * sum_k X[r + n k] W[k kout + c] on MFMA: the
 // transposed product D = W^T X^T, so a result register holds 16 consecutive
 // rows of one output column (coalesced stores). A workgroup owns 64 rows x
-// 128 columns, each wave 32 rows x 64 columns; W is staged in LDS 16 k at a
-// time, the wave's X values for the next stage are loaded during the
-// current stage's products.
-constexpr int nRows = 64, nCols = 128, nK = 16;
+// nCols columns (128, or 64 for outputs that narrow, half of whose products
+// would be padding: 523,000 x 200 x 64 505 -> 238 us), each wave 32 rows x half of them; W is
+// staged in LDS 16 k at a time, the wave's X values for the next stage are
+// loaded during the current stage's products.
+constexpr int nRows = 64, nK = 16;
+template <int nCols>
 __global__ void __launch_bounds__(256) k_gemm_nn_mfma(const double* __restrict__ X, const double* __restrict__ W,
                                                       double* out, const double* base, double alpha, uint64_t n,
                                                       uint32_t kin, uint32_t kout) {
@@ -187,10 +203,11 @@ __global__ void __launch_bounds__(256) k_gemm_nn_mfma(const double* __restrict__
   const uint64_t r0 = (uint64_t)blockIdx.x * nRows;
   const uint32_t c0 = blockIdx.y * nCols;
   const int t = threadIdx.x, lane = t % 64, wv = t / 64;
-  const int wr = (wv & 1) * 32, wc = (wv >> 1) * 64;
-  dbl4 acc[4][2];
+  constexpr int NI = nCols / 32;  // 16-column tiles per wave
+  const int wr = (wv & 1) * 32, wc = (wv >> 1) * (nCols / 2);
+  dbl4 acc[NI][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
   // B operand (4 k x 16 rows): lane l holds X[row l % 16][k l / 16]
@@ -221,11 +238,11 @@ __global__ void __launch_bounds__(256) k_gemm_nn_mfma(const double* __restrict__
 #pragma unroll
     for (int kk = 0; kk < nK / 4; ++kk) {
       // A operand (16 columns x 4 k): lane l holds W[k l / 16][column l % 16]
-      double A[4];
+      double A[NI];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) A[i] = Ws[4 * kk + lane / 16][wc + 16 * i + lane % 16];
+      for (int i = 0; i < NI; ++i) A[i] = Ws[4 * kk + lane / 16][wc + 16 * i + lane % 16];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = mfma64(A[i], xc[kk][j], acc[i][j]);
     }
@@ -233,7 +250,7 @@ __global__ void __launch_bounds__(256) k_gemm_nn_mfma(const double* __restrict__
   }
   // D register v of lane l holds D[l / 16 + 4 v][l % 16]: column l / 16 + 4 v, row l % 16
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -247,13 +264,18 @@ __global__ void __launch_bounds__(256) k_gemm_nn_mfma(const double* __restrict__
       }
 }
 
-// out[e] = sum over chunks c = 0, 1, ... of part[c][e], in that order
-__global__ void k_sum_chunks(const double* __restrict__ part, double* __restrict__ out, uint64_t ne, uint32_t nch) {
-  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
+// out[a][b] = sum over chunks c = 0, 1, ... of part[c][a][b], in that order.
+// symmetric: from the mirrored entry below the tile diagonal (both have the
+// same terms in the same order, so the same bits)
+__global__ void k_sum_chunks(const double* __restrict__ part, double* __restrict__ out, uint64_t ne, uint32_t nch,
+                             uint32_t Kb, int symmetric) {
+  const uint64_t o = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (o >= ne) return;
+  const uint64_t a = o / Kb, b = o % Kb;
+  const uint64_t e = symmetric && a / kTile > b / kTile ? b * Kb + a : o;
   double s = 0.0;
   for (uint32_t c = 0; c < nch; ++c) s += part[(uint64_t)c * ne + e];
-  out[e] = s;
+  out[o] = s;
 }
 
 }  // namespace
@@ -290,20 +312,24 @@ void projectTN(int op, uint32_t nr, uint32_t nth, uint64_t n, uint64_t nX, const
   p.chunk = (n + nch - 1) / nch;
   p.chunk = (p.chunk + kRows - 1) / kRows * kRows;
   p.Ka = Ka; p.Kb = Kb; p.nr = nr; p.nth = nth;
+  p.symmetric = op == 2 && L == X && Ka == Kb && !w;
   const dim3 grid((Ka + kTile - 1) / kTile, (Kb + kTile - 1) / kTile, nch);
   if (op == 0) hipLaunchKernelGGL(k_proj_tn<0>, grid, dim3(256), 0, stream, p);
   else if (op == 1) hipLaunchKernelGGL(k_proj_tn<1>, grid, dim3(256), 0, stream, p);
   else hipLaunchKernelGGL(k_proj_tn<2>, grid, dim3(256), 0, stream, p);
   const uint64_t ne = (uint64_t)Ka * Kb;
-  hipLaunchKernelGGL(k_sum_chunks, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, stream, part, out, ne, nch);
+  hipLaunchKernelGGL(k_sum_chunks, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, stream, part, out, ne, nch, Kb,
+                     p.symmetric);
   SHAW_HIP(hipGetLastError());
 }
 
 void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t kout, double* out,
             const double* base, double alpha, hipStream_t stream) {
   SHAW_REQUIRE(n > 0 && kin > 0 && kout > 0, SHAW_ERR_ARG, "gemm: bad shape");
-  const dim3 grid((unsigned)((n + nRows - 1) / nRows), (kout + nCols - 1) / nCols);
-  hipLaunchKernelGGL(k_gemm_nn_mfma, grid, dim3(256), 0, stream, X, W, out, base, alpha, n, kin, kout);
+  const uint32_t cols = kout <= 64 ? 64 : 128;
+  const dim3 grid((unsigned)((n + nRows - 1) / nRows), (kout + cols - 1) / cols);
+  if (cols == 64) hipLaunchKernelGGL(k_gemm_nn_mfma<64>, grid, dim3(256), 0, stream, X, W, out, base, alpha, n, kin, kout);
+  else hipLaunchKernelGGL(k_gemm_nn_mfma<128>, grid, dim3(256), 0, stream, X, W, out, base, alpha, n, kin, kout);
   SHAW_HIP(hipGetLastError());
 }
 
