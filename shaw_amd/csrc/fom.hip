@@ -1802,13 +1802,12 @@ class FomEngine final : public shaw_fom {
     s.buf.alloc(n * maxSamples * ncols);
   }
   void reset() override {
-    for (int b = 0; b < 2; ++b) {
-      if (v_[b].p) SHAW_HIP(hipMemsetAsync(v_[b].p, 0, v_[b].n * sizeof(T), stream_));
-      if (s_[b].p) SHAW_HIP(hipMemsetAsync(s_[b].p, 0, s_[b].n * sizeof(T), stream_));
-    }
-    SHAW_HIP(hipStreamSynchronize(stream_));
+    // only the current states: a launch writes every point of the other copy
+    // before anything reads it
     step_ = 0;
     cur_ = 0;
+    SHAW_HIP(hipMemsetAsync(v_[0].p, 0, v_[0].n * sizeof(T), stream_));
+    SHAW_HIP(hipMemsetAsync(s_[0].p, 0, s_[0].n * sizeof(T), stream_));
   }
 
   void advance(uint64_t nsteps) override {
@@ -1980,8 +1979,7 @@ class FomEngine final : public shaw_fom {
     sync();
     const uint64_t T_ = R_ ? step_ / every_ : 0;
     // device [R x Tcap x M] -> host [R x T x M]
-    for (uint64_t m = 0; m < M_ && T_; ++m)
-      SHAW_HIP(hipMemcpy(out + R_ * T_ * m, seis_.p + R_ * Tcap_ * m, R_ * T_ * sizeof(double), hipMemcpyDeviceToHost));
+    copyRows(out, seis_.p, R_ * T_, R_ * Tcap_, M_);
     // receivers sharing a grid point with an earlier receiver
     for (const auto& d : dupRecv_)
       for (uint64_t m = 0; m < M_; ++m)
@@ -1992,8 +1990,7 @@ class FomEngine final : public shaw_fom {
     sync();
     const Snap& s = snap_[dof];
     const uint64_t T_ = s.ncols ? step_ / s.every : 0, n = dof == 0 ? nVp_ : nSp_;
-    for (uint64_t c = 0; c < s.ncols && T_; ++c)
-      SHAW_HIP(hipMemcpy(out + n * T_ * c, s.buf.p + n * s.Tcap * c, n * T_ * sizeof(double), hipMemcpyDeviceToHost));
+    copyRows(out, s.buf.p, n * T_, n * s.Tcap, s.ncols);
     return T_;
   }
   void getState(double* vp, double* sp) override {
@@ -2126,6 +2123,18 @@ class FomEngine final : public shaw_fom {
     DevBuf<double> buf;
     uint64_t ncols = 0, every = 0, Tcap = 0;
   };
+
+  // rows of `len` of `pitch` device values each, packed on the host: one copy
+  // for all of them where they are contiguous (a complete run)
+  void copyRows(double* out, const double* dev, uint64_t len, uint64_t pitch, uint64_t rows) {
+    if (len == 0 || rows == 0) return;
+    if (len == pitch) {
+      SHAW_HIP(hipMemcpy(out, dev, len * rows * sizeof(double), hipMemcpyDeviceToHost));
+      return;
+    }
+    for (uint64_t r = 0; r < rows; ++r)
+      SHAW_HIP(hipMemcpy(out + len * r, dev + pitch * r, len * sizeof(double), hipMemcpyDeviceToHost));
+  }
 
   StepArgs<T> args(uint64_t stepNo) {
     StepArgs<T> a{};
