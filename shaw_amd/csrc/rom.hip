@@ -924,6 +924,9 @@ struct shaw_rom {
   double dt = 0;
   int precision = 0;
   uint32_t resident = 0;  // padded modes per dof when the operators stay on the CU (k_rom_resident), else 0
+  uint32_t split = 1;     // workgroups of a tile of columns there, their exchange buffers and flags
+  shaw::DevBuf<uint64_t> xbuf, flags;
+  uint64_t launches = 0;
   int parts() const { return precision == SHAW_ROM_FP64 ? 0 : precision == SHAW_ROM_BF16X3 ? 2 : 3; }
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1038,9 +1041,12 @@ struct shaw_rom {
     a.quiet = quiet.p;
     a.macro = precision == SHAW_ROM_FP64 ? 0 : macro;
     a.budget = a.macro ? timeBudget : 0;
+    a.tiles = (uint32_t)(maxCols / kTileCols);
+    a.xbuf = xbuf.p; a.flags = flags.p;
+    a.epoch = launches++ << 33;  // horizons lie below 2^31: at most 2^32 exchanges a launch
     const dim3 grid((unsigned)(maxCols / kTileCols));
     const size_t lds = ldsBytes();
-    if (resident && precision != SHAW_ROM_FP64) launchRomResident(parts(), a, grid, stream);
+    if (resident && precision != SHAW_ROM_FP64) launchRomResident(parts(), a, split, stream);
     else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, maxCols, stream);
     else if (precision == SHAW_ROM_FP64) launchRomSteps<0>(tpw, grid, lds, stream, a);
     else if (precision == SHAW_ROM_BF16X3) launchRomSteps<2>(tpw, grid, lds, stream, a);
@@ -1293,6 +1299,18 @@ int shaw_rom_create(const shaw_rom_desc* d, shaw_rom_t* out) {
     }
     pack(cPad.data(), h->rp, d->kv, h->rp, h->kvp, h->c);
     const uint64_t C = h->maxCols;
+    if (h->resident) {
+      int dev = 0, cus = 0, coop = 0;
+      SHAW_HIP(hipGetDevice(&dev));
+      SHAW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+      SHAW_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+      if (coop) h->split = residentSplit(h->parts(), h->resident, C / kTileCols, cus);
+      if (h->split > 1) {
+        h->xbuf.alloc(residentExchange(h->resident, C / kTileCols));
+        h->flags.alloc(C / kTileCols * kMaxRowTiles);
+        SHAW_HIP(hipMemset(h->flags.p, 0, h->flags.n * sizeof(uint64_t)));
+      }
+    }
     h->qv.alloc(C * h->kvp); h->qs.alloc(C * h->ksp); h->b.alloc(C * h->kvp);
     SHAW_HIP(hipMemset(h->qv.p, 0, h->qv.n * 8)); SHAW_HIP(hipMemset(h->qs.p, 0, h->qs.n * 8));
     SHAW_HIP(hipMemset(h->b.p, 0, h->b.n * 8));

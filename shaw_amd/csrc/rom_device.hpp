@@ -46,6 +46,13 @@ struct RomArgs {
   // time of nsteps one-steps for every tile, a macro step costing w of them,
   // so tiles taking macro steps advance further (stepCol holds how far)
   uint32_t budget;
+  // tiles of 16 columns; and where several workgroups share one (k_rom_resident
+  // with SPLIT > 1): each tile's exchange buffers and kMaxRowTiles flags, and a
+  // count above all that earlier launches left there
+  uint32_t tiles;
+  uint64_t* xbuf;
+  uint64_t* flags;
+  uint64_t epoch;
 };
 
 namespace {
@@ -56,6 +63,8 @@ typedef short shrt4 __attribute__((ext_vector_type(4)));
 typedef short shrt16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTileCols = 16;  // column slots per workgroup
+constexpr uint32_t kMaxTries = 1u << 24;  // of a bounded wait, each a read of memory (about 10 s)
+constexpr int kMaxRowTiles = 32;
 constexpr int kWaves = 8;      // waves per ROM workgroup (16 at 9..16 row tiles)
 
 // ------------------------------------------------------------ bf16 helpers

@@ -64,7 +64,11 @@ void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t
 // columns, k_rom_steps taking the same operators with the same results).
 struct RomArgs;
 uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols);
-void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream);
+// The workgroups that share a tile of 16 columns (BF16), the 64-bit words of
+// a.xbuf that they then need, and the launch, cooperative if split > 1.
+uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus);
+uint64_t residentExchange(uint32_t modes, uint64_t tiles);
+void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream);
 bool romF64Fits(uint32_t modes, uint64_t activeTiles);
 void launchRomF64(const RomArgs& a, uint64_t cols, hipStream_t stream);
 uint64_t projPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);

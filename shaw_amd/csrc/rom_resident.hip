@@ -1,5 +1,5 @@
-// The BF16 reduced leapfrog for operators of up to 256 modes per dof: the
-// operators stay on the CU.
+// The BF16 reduced leapfrog with the operators on the CU as far as they fit; of
+// few columns and many modes, on several CUs.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -14,11 +14,11 @@ namespace {
 typedef float flt2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-// writeSplitRows with the hardware's conversion (round to nearest even, as
-// f32ToBf16; a NaN becomes a quiet NaN)
-__device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, int lane, const double (&q)[4]) {
-  typedef unsigned u2 __attribute__((ext_vector_type(2)));
-  u2 h, l;
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
+
+// the split of writeSplitRows with the hardware's conversion (round to nearest
+// even, as f32ToBf16; a NaN becomes a quiet NaN)
+__device__ __forceinline__ void splitRowsHw(const double (&q)[4], u2& h, u2& l) {
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
     const flt2 x = {(float)q[2 * p], (float)q[2 * p + 1]};
@@ -27,6 +27,11 @@ __device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, in
     const flt2 hf = {__uint_as_float(hb << 16), __uint_as_float(hb & 0xffff0000u)};
     l[p] = __builtin_bit_cast(unsigned, __builtin_convertvector(x - hf, bf16x2));
   }
+}
+
+__device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, int lane, const double (&q)[4]) {
+  u2 h, l;
+  splitRowsHw(q, h, l);
   const int item = (4 * (rt / 2) + lane / 16) * kTileCols + lane % 16;
   reinterpret_cast<u2*>(S + item)[rt % 2] = h;
   reinterpret_cast<u2*>(S + loOff + item)[rt % 2] = l;
@@ -45,10 +50,22 @@ __device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, in
 // Waves: 2 KG row tiles in one or two per wave, at most 256 VGPRs, so that no
 // operand passes through an AGPR; four waves of twice the tiles copy every
 // operand out of AGPRs before its product (K = 192 BF16x3 1.98 against 2.40).
-template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, bool MACRO>
+//
+// SPLIT > 1: that many workgroups share a tile of 16 columns, each with 1 /
+// SPLIT of the row tiles (one per wave), so that the operators fit the CUs that
+// few columns would leave idle. After a half-step each wave writes its rows'
+// split to a.xbuf and its count of half-steps to a.flags, waits for every wave
+// of the tile, and the workgroup reads the whole split back. Bound by that
+// exchange (2 to 4 us) and the chain of 2 KG or more products; one workgroup a
+// tile is bound by streaming the operators. Per step, one (of 4096 columns, all
+// CUs streaming) -> several: BF16x4
+// K = 384 16.2 us -> 6.0 at 16 columns, 8.5 at 384, 8.8 at 640, 12.4 at 1280,
+// K = 512 26.6 -> 12.1 at 512, 18.4 at 1024; BF16x3 K = 384 at 640 columns 9.6
+// -> 8.5, K = 512 17.8 -> 11.9 at 512, 14.8 at 1024.
+template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, bool MACRO, int SPLIT>
 __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
-  constexpr int K = 32 * KG, TILES = 2 * KG, TPW = TILES / WAVES;
-  static_assert(TILES % WAVES == 0, "whole row tiles per wave");
+  constexpr int K = 32 * KG, TILES = 2 * KG, OWN = TILES / SPLIT, TPW = OWN / WAVES;
+  static_assert(TILES % (SPLIT * WAVES) == 0, "whole row tiles per wave");
   using P = Place<KG, RR, LL, DR>;
   constexpr int S = P::S, NR = S < DR ? S : DR;  // ring slots in use
   using Item = typename Prec<PARTS>::Item;
@@ -57,13 +74,18 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   int4v* Sv = reinterpret_cast<int4v*>(sm);
   int4v* Ss = Sv + 4 * K;
   constexpr int lo = 2 * K;
-  int4v* Al = Ss + 4 * K;  // [operator][tile][LL][part][lane]
-  const int slot0 = blockIdx.x * kTileCols;
+  int4v* Al = Ss + 4 * K;  // [operator][own tile][LL][part][lane]
+  // the workgroups of a tile are eight apart: on one XCD, in whose L2 they share
+  // what still streams of the operators, where workgroups go round the eight
+  const int tile = SPLIT == 1 ? (int)blockIdx.x : (int)(blockIdx.x / (8 * SPLIT) * 8 + blockIdx.x % 8);
+  const int part = SPLIT == 1 ? 0 : (int)(blockIdx.x / 8 % SPLIT);
+  if (SPLIT > 1 && tile >= (int)a.tiles) return;
+  const int slot0 = tile * kTileCols;
   const int tid = threadIdx.x, lane = tid % 64, col = lane % 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   int rt[TPW];  // this wave's row tiles, the same of both operators
 #pragma unroll
-  for (int t = 0; t < TPW; ++t) rt[t] = wave + t * WAVES;
+  for (int t = 0; t < TPW; ++t) rt[t] = part * OWN + wave + t * WAVES;
   const uint64_t colQ = (uint64_t)(slot0 + col) * K;
   double qv[TPW][4], qs[TPW][4], bv[TPW][4];
 #pragma unroll
@@ -74,10 +96,24 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       qv[t][r] = a.qv[colQ + rt[t] * 16 + rowBf16(lane, r)];
       qs[t][r] = a.qs[colQ + rt[t] * 16 + rowBf16(lane, r)];
     }
+  if constexpr (SPLIT == 1) {
 #pragma unroll
-  for (int t = 0; t < TPW; ++t) {
-    writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
-    writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+    for (int t = 0; t < TPW; ++t) {
+      writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
+      writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+    }
+  } else {
+#pragma nounroll
+    for (int x = wave; x < TILES; x += WAVES) {
+      double v[4], s[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = a.qv[colQ + x * 16 + rowBf16(lane, r)];
+        s[r] = a.qs[colQ + x * 16 + rowBf16(lane, r)];
+      }
+      writeSplitRowsHw(Sv, lo, x, lane, v);
+      writeSplitRowsHw(Ss, lo, x, lane, s);
+    }
   }
   const uint32_t s0 = (uint32_t)a.stepCol[slot0 + col];
   const uint32_t hz = (uint32_t)a.horizon[slot0 + col];
@@ -141,7 +177,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
           it[t] = ring[n % (NR > 0 ? NR : 1)][t];
         } else if (n < LL) {
 #pragma unroll
-          for (int p = 0; p < PARTS; ++p) it[t].p[p] = Al[(((op * TILES + rt[t]) * LL + n) * PARTS + p) * 64 + lane];
+          for (int p = 0; p < PARTS; ++p) it[t].p[p] = Al[(((op * OWN + wave + t * WAVES) * LL + n) * PARTS + p) * 64 + lane];
         } else {
           it[t] = res[op][t][n >= LL ? n - LL : 0];
         }
@@ -182,12 +218,87 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
           } else if (n < LL) {
             const Item it = at(A[op], t, g);
 #pragma unroll
-            for (int p = 0; p < PARTS; ++p) Al[(((op * TILES + rt[t]) * LL + n) * PARTS + p) * 64 + lane] = it.p[p];
+            for (int p = 0; p < PARTS; ++p) Al[(((op * OWN + wave + t * WAVES) * LL + n) * PARTS + p) * 64 + lane] = it.p[p];
           } else {
             res[op][t][n >= LL ? n - LL : 0] = at(A[op], t, g);
           }
         }
   };
+  // SPLIT > 1: an exchange moves a split (or both) from the tile's waves to all
+  // its workgroups. It alternates between two buffers: a wave writes one again
+  // two exchanges later, when every wave has reached the one between and so has
+  // read it. The counts go on from launch to launch (a.epoch), so a flag of an
+  // earlier launch never passes for one of this.
+  uint64_t* const flags = a.flags + (uint64_t)tile * kMaxRowTiles;
+  uint64_t* const xbuf = a.xbuf + (uint64_t)tile * 4 * 8 * K;  // [exchange % 2][dof][8 K]
+  uint64_t epoch = a.epoch;
+  bool lost = false;
+  // Device scope throughout, past the L1 and the L2 of an XCD (2.3 us an
+  // exchange of one tile at K = 384). With all of a tile's workgroups on one XCD
+  // its L2 could serve, but only an acquire fence drops the L1, and fences of
+  // many waves hold each other up: 24 tiles 10.8 us a step against 8.5, 80 tiles
+  // 54 against 12.4.
+  auto put = [](uint64_t* x, uint64_t v) { __hip_atomic_store(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  auto get = [](const uint64_t* x) { return __hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  // waits until every wave of the tile has come as far (the launch is
+  // cooperative, so they run; should one never come, the wave goes on without it
+  // and its rows become NaN)
+  auto meet = [&] {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's rows are out
+    const uint64_t want = epoch + 1;
+    if (lane == 0) put(flags + part * WAVES + wave, want);
+    for (uint32_t tries = 0; !lost; ++tries) {
+      uint64_t f = want;
+      if (lane < SPLIT * WAVES) f = get(flags + lane);
+      if (__ballot(f < want) == 0) break;
+      lost = tries > kMaxTries;
+    }
+    asm volatile("" ::: "memory");
+  };
+  auto publish = [&](int dof, double (&q)[TPW][4]) {
+    uint64_t* x = xbuf + ((epoch % 2) * 2 + dof) * 8 * K;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      u2 h, l;
+      splitRowsHw(q[t], h, l);
+      const int item = 2 * ((4 * (rt[t] / 2) + lane / 16) * kTileCols + col) + rt[t] % 2;
+      put(x + item, __builtin_bit_cast(uint64_t, h));
+      put(x + 2 * lo + item, __builtin_bit_cast(uint64_t, l));
+    }
+  };
+  auto collect = [&](int dof, int4v* S) {
+    const uint64_t* x = xbuf + ((epoch % 2) * 2 + dof) * 8 * K;
+    uint64_t* d = reinterpret_cast<uint64_t*>(S);
+    constexpr int N = 8 * K / (64 * WAVES);
+    static_assert(8 * K % (64 * WAVES) == 0, "whole rounds");
+    uint64_t v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = get(x + i * 64 * WAVES + tid);
+#pragma unroll
+    for (int i = 0; i < N; ++i) d[i * 64 * WAVES + tid] = v[i];
+  };
+  auto poison = [&](double (&q)[TPW][4]) {
+    if (lost)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) q[t][r] = __builtin_nan("");
+  };
+  // the new split of a dof to every wave that reads it
+  auto share = [&](int dof, double (&q)[TPW][4], int4v* S) {
+    if constexpr (SPLIT == 1) {
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) writeSplitRowsHw(S, lo, rt[t], lane, q[t]);
+    } else {
+      publish(dof, q);
+      meet();
+      collect(dof, S);
+      poison(q);
+      ++epoch;
+    }
+    __syncthreads();
+  };
+  constexpr int RW = SPLIT * WAVES;  // waves that take the receivers' row tiles
 #pragma nounroll
   for (int seg = 0; seg < (MACRO ? 2 : 1); ++seg) {
     const uint32_t from = seg == 0 ? 0u : mk + a.macro * mk2;
@@ -229,12 +340,10 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
             asm("" : "+v"(z));
             qv[t][r] = act ? z : qv[t][r];
           }
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
-        __syncthreads();
+        share(0, qv, Sv);
         // stress: q_s += dt Ar_s q_v
         products(std::integral_constant<int, 1>{}, Sv);
-        if (anySample) receivers<PARTS, 1, WAVES, 2>(a, Sv, lo, wave, lane, smp, nextIdx - 1, slot0);
+        if (anySample) receivers<PARTS, 1, RW, 2>(a, Sv, lo, part * WAVES + wave, lane, smp, nextIdx - 1, slot0);
 #pragma unroll
         for (int t = 0; t < TPW; ++t)
 #pragma unroll
@@ -243,9 +352,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
             asm("" : "+v"(z));
             qs[t][r] = act ? z : qs[t][r];
           }
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
-        __syncthreads();
+        share(1, qs, Ss);
         if (ev && act) {
           phase = phase + 1 == ev ? 0 : phase + 1;
           if (phase == 0) ++nextIdx;
@@ -291,18 +398,29 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
             for (int t = 0; t < TPW; ++t)
 #pragma unroll
               for (int r = 0; r < 4; ++r) qs[t][r] = qs[t][r] + a.dt * (double)acc[t][r];
-          __syncthreads();  // every read of the old splits done
+          if constexpr (SPLIT == 1) {
+            __syncthreads();  // every read of the old splits done
 #pragma unroll
-          for (int t = 0; t < TPW; ++t) {
-            writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
-            writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+            for (int t = 0; t < TPW; ++t) {
+              writeSplitRowsHw(Sv, lo, rt[t], lane, qv[t]);
+              writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
+            }
+          } else {
+            publish(0, qv);
+            publish(1, qs);
+            meet();
+            collect(0, Sv);
+            collect(1, Ss);
+            poison(qv);
+            poison(qs);
+            ++epoch;
           }
           __syncthreads();  // the new splits complete
           // the macro step's last step is sampled when it ends at a multiple of the period
           const uint64_t sn = (uint64_t)s0 + mk + (uint64_t)(it + 1) * a.macro;
           const bool smp = act && ev > 0 && sn % ev == 0;
           if ((__ballot(smp) & 0xffffull) != 0)
-            receivers<PARTS, 1, WAVES, 2>(a, Sv, lo, wave, lane, smp, smp ? (uint32_t)(sn / ev - 1) : 0u, slot0);
+            receivers<PARTS, 1, RW, 2>(a, Sv, lo, part * WAVES + wave, lane, smp, smp ? (uint32_t)(sn / ev - 1) : 0u, slot0);
         }
         __syncthreads();  // the next one-steps write the split the receivers read
       }
@@ -315,7 +433,9 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       a.qv[colQ + rt[t] * 16 + rowBf16(lane, r)] = qv[t][r];
       a.qs[colQ + rt[t] * 16 + rowBf16(lane, r)] = qs[t][r];
     }
-  if (tid < kTileCols) {
+  // (no workgroup of the tile is still to read its counters or states: a tile
+  // with steps has had an exchange, one without writes what it read)
+  if (part == 0 && tid < kTileCols) {
     // a.nsteps steps, or fewer when every column reached its horizon (the
     // same counts), or more under a time budget
     const uint64_t h = a.horizon[slot0 + tid];
@@ -324,16 +444,22 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   }
 }
 
-template <int PARTS, int KG, int WAVES, int RR, int LL, int DR>
-void launchKG(const RomArgs& a, dim3 grid, hipStream_t stream) {
-  constexpr size_t lds = (8 * 32 * KG + (size_t)2 * 2 * KG * LL * PARTS * 64) * 16;
-  static_assert(lds <= 160 * 1024, "LDS of one CU");
+template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, int SPLIT = 1>
+void launchKG(RomArgs a, uint32_t tiles, hipStream_t stream) {
+  constexpr size_t lds = (8 * 32 * KG + (size_t)2 * (2 * KG / SPLIT) * LL * PARTS * 64) * 16;
+  static_assert(lds <= 160 * 1024 && 2 * KG <= kMaxRowTiles, "LDS of one CU, a flag per wave");
   auto go = [&](auto kernel) {
-    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(kernel, grid, dim3(WAVES * 64), lds, stream, a);
+    SHAW_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if constexpr (SPLIT == 1) {
+      hipLaunchKernelGGL(kernel, dim3(tiles), dim3(WAVES * 64), lds, stream, a);
+    } else {
+      void* args[] = {&a};
+      SHAW_HIP(hipLaunchCooperativeKernel((const void*)kernel, dim3((tiles + 7) / 8 * 8 * SPLIT), dim3(WAVES * 64), args,
+                                          (unsigned)lds, stream));
+    }
   };
-  if (a.macro) go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, true>);
-  else go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, false>);
+  if (a.macro) go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, true, SPLIT>);
+  else go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, false, SPLIT>);
 }
 
 }  // namespace
@@ -353,8 +479,35 @@ uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols) {
   return cols <= (k <= 384 ? 2048 : 1024) ? modes : 0;
 }
 
-void launchRomResident(int parts, const RomArgs& a, dim3 grid, hipStream_t stream) {
+// The workgroups of a tile of 16 columns of a BF16 engine (1: one): four row
+// tiles each, or eight, while the chip holds all workgroups at once, one to a
+// CU. Not up to 256 modes (one workgroup: BF16x4 4.3 us a step, two exchanges
+// alone 4.6), nor BF16x3 of 384 in threes (10.2 us at 1280 columns against 9.6).
+uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus) {
+  if (parts == 0 || modes < 384) return 1;
+  const uint32_t most = modes / 64;
+  auto fits = [&](uint32_t split) { return (tiles + 7) / 8 * 8 * split <= (uint64_t)cus; };
+  if (fits(most)) return most;
+  return fits(most / 2) && !(parts == 2 && modes == 384) ? most / 2 : 1;
+}
+uint64_t residentExchange(uint32_t modes, uint64_t tiles) { return tiles * 4 * 8 * modes; }
+
+void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream) {
   const int kg = (int)a.Kvp / 32;
+  const uint32_t grid = a.tiles;
+  if (split > 1) {
+    if (parts == 2) {
+      if (kg == 12) launchKG<2, 12, 4, 8, 4, 1, 6>(a, grid, stream);
+      else if (split == 8) launchKG<2, 16, 4, 10, 6, 1, 8>(a, grid, stream);
+      else launchKG<2, 16, 8, 9, 3, 1, 4>(a, grid, stream);
+    } else {
+      if (kg == 12 && split == 6) launchKG<3, 12, 4, 8, 4, 1, 6>(a, grid, stream);
+      else if (kg == 12) launchKG<3, 12, 8, 6, 2, 1, 3>(a, grid, stream);
+      else if (split == 8) launchKG<3, 16, 4, 12, 4, 1, 8>(a, grid, stream);
+      else launchKG<3, 16, 8, 6, 2, 1, 4>(a, grid, stream);
+    }
+    return;
+  }
   if (parts == 2) {
     switch (kg) {
       case 2: launchKG<2, 2, 4, 2, 0, 1>(a, grid, stream); break;
