@@ -1043,11 +1043,15 @@ struct shaw_rom {
     a.budget = a.macro ? timeBudget : 0;
     a.tiles = (uint32_t)(maxCols / kTileCols);
     a.xbuf = xbuf.p; a.flags = flags.p;
-    a.epoch = launches++ << 33;  // horizons lie below 2^31: at most 2^32 exchanges a launch
+    a.launch = ++launches;
     const dim3 grid((unsigned)(maxCols / kTileCols));
     const size_t lds = ldsBytes();
-    if (resident && precision != SHAW_ROM_FP64) launchRomResident(parts(), a, split, stream);
-    else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, maxCols, stream);
+    if (resident && precision != SHAW_ROM_FP64) {
+      // a cooperative launch and its first meeting cost about what three steps
+      // save (1280 columns of K = 384 BF16x3, launches in a row: 4 steps 56 us
+      // against 57, 2 steps 48 against 37)
+      launchRomResident(parts(), a, nsteps >= 4 ? split : 1, stream);
+    } else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, maxCols, stream);
     else if (precision == SHAW_ROM_FP64) launchRomSteps<0>(tpw, grid, lds, stream, a);
     else if (precision == SHAW_ROM_BF16X3) launchRomSteps<2>(tpw, grid, lds, stream, a);
     else launchRomSteps<3>(tpw, grid, lds, stream, a);
@@ -1267,7 +1271,12 @@ int shaw_rom_create(const shaw_rom_desc* d, shaw_rom_t* out) {
     const uint32_t kq = (d->precision == SHAW_ROM_FP64 ? 16 : 32) * kRing;
     h->kvp = roundUp(d->kv, kq);
     h->ksp = roundUp(d->ks, kq);
-    h->resident = residentModes(h->parts(), d->kv, d->ks, d->max_cols);
+    int dev = 0, cus = 0, coop = 0;
+    SHAW_HIP(hipGetDevice(&dev));
+    SHAW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    SHAW_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    if (!coop) cus = 0;
+    h->resident = residentModes(h->parts(), d->kv, d->ks, d->max_cols, cus);
     if (h->resident) h->kvp = h->ksp = h->resident;
     h->rp = roundUp(std::max<uint64_t>(d->r, 1), 16);
     h->maxCols = roundUp(d->max_cols, kTileCols);
@@ -1299,17 +1308,11 @@ int shaw_rom_create(const shaw_rom_desc* d, shaw_rom_t* out) {
     }
     pack(cPad.data(), h->rp, d->kv, h->rp, h->kvp, h->c);
     const uint64_t C = h->maxCols;
-    if (h->resident) {
-      int dev = 0, cus = 0, coop = 0;
-      SHAW_HIP(hipGetDevice(&dev));
-      SHAW_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-      SHAW_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-      if (coop) h->split = residentSplit(h->parts(), h->resident, C / kTileCols, cus);
-      if (h->split > 1) {
-        h->xbuf.alloc(residentExchange(h->resident, C / kTileCols));
-        h->flags.alloc(C / kTileCols * kMaxRowTiles);
-        SHAW_HIP(hipMemset(h->flags.p, 0, h->flags.n * sizeof(uint64_t)));
-      }
+    h->split = residentSplit(h->resident ? h->parts() : 0, h->resident, C / kTileCols, cus);
+    if (h->split > 1) {
+      h->xbuf.alloc(residentExchange(h->resident, C / kTileCols));
+      h->flags.alloc(C / kTileCols * kMaxRowTiles);
+      SHAW_HIP(hipMemset(h->flags.p, 0, h->flags.n * sizeof(uint64_t)));
     }
     h->qv.alloc(C * h->kvp); h->qs.alloc(C * h->ksp); h->b.alloc(C * h->kvp);
     SHAW_HIP(hipMemset(h->qv.p, 0, h->qv.n * 8)); SHAW_HIP(hipMemset(h->qs.p, 0, h->qs.n * 8));

@@ -47,12 +47,12 @@ struct RomArgs {
   // so tiles taking macro steps advance further (stepCol holds how far)
   uint32_t budget;
   // tiles of 16 columns; and where several workgroups share one (k_rom_resident
-  // with SPLIT > 1): each tile's exchange buffers and kMaxRowTiles flags, and a
-  // count above all that earlier launches left there
+  // with SPLIT > 1): each tile's exchange buffers and kMaxRowTiles flags, and the
+  // launch's number, from 1
   uint32_t tiles;
   uint64_t* xbuf;
   uint64_t* flags;
-  uint64_t epoch;
+  uint64_t launch;
 };
 
 namespace {

@@ -57,13 +57,14 @@ void macroOperator(const double* arV, const double* arS, uint64_t kv, uint64_t k
 void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t kout, double* out,
             const double* base, double alpha, hipStream_t stream);
 // The padded modes per dof of an engine whose operators stay on the CU as far
-// as they fit (parts: 0 FP64, else the bf16 parts; cols: column slots), 0 where
+// as they fit (parts: 0 FP64, else the bf16 parts; cols: column slots; cus: the
+// device's CUs, 0 if it takes no cooperative launch), 0 where
 // k_rom_steps* run it. Such an engine has a.Kvp = a.Ksp = that size and runs
 // launchRomResident (BF16, rom_resident.hip) or launchRomF64 (FP64, rom_f64.hip;
 // romF64Fits says whether that is the faster kernel for the active tiles of 16
 // columns, k_rom_steps taking the same operators with the same results).
 struct RomArgs;
-uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols);
+uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int cus);
 // The workgroups that share a tile of 16 columns (BF16), the 64-bit words of
 // a.xbuf that they then need, and the launch, cooperative if split > 1.
 uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus);

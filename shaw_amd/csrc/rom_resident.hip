@@ -11,6 +11,10 @@
 namespace shaw {
 namespace {
 
+// words of an exchange buffer without a value: four NaNs' bits; the buffers
+constexpr uint64_t kEmpty = ~0ull;
+constexpr int kXbufs = 3;
+
 typedef float flt2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -54,14 +58,15 @@ __device__ __forceinline__ void writeSplitRowsHw(int4v* S, int loOff, int rt, in
 // SPLIT > 1: that many workgroups share a tile of 16 columns, each with 1 /
 // SPLIT of the row tiles (one per wave), so that the operators fit the CUs that
 // few columns would leave idle. After a half-step each wave writes its rows'
-// split to a.xbuf and its count of half-steps to a.flags, waits for every wave
-// of the tile, and the workgroup reads the whole split back. Bound by that
-// exchange (2 to 4 us) and the chain of 2 KG or more products; one workgroup a
-// tile is bound by streaming the operators. Per step, one (of 4096 columns, all
-// CUs streaming) -> several: BF16x4
-// K = 384 16.2 us -> 6.0 at 16 columns, 8.5 at 384, 8.8 at 640, 12.4 at 1280,
-// K = 512 26.6 -> 12.1 at 512, 18.4 at 1024; BF16x3 K = 384 at 640 columns 9.6
-// -> 8.5, K = 512 17.8 -> 11.9 at 512, 14.8 at 1024.
+// split to a.xbuf and the workgroup reads the whole of it back from there. Bound
+// by that exchange (1.4 us; more as the workgroups fill the chip) and the chain
+// of 2 KG or more products; one workgroup a tile is bound by streaming the
+// operators. Per step, one (of 4096 columns, all CUs streaming) -> several:
+// BF16x4 K = 384 16.2 us -> 4.2 at 16 columns, 4.4 at 384, 4.6 at 640, 7.9 at
+// 1280; K = 512 26.6 -> 4.8 at 16, 7.4 at 512, 12.7 at 1024; BF16x3 K = 384 9.6
+// -> 4.3 at 640, 5.0 at 1280; K = 512 17.8 -> 9.0 at 512, 11.8 at 1024. (Flags that say the
+// rows are there, read before them, are two more trips to memory: K = 384 5.8 us
+// at 16 columns, 8.2 at 384.)
 template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, bool MACRO, int SPLIT>
 __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   constexpr int K = 32 * KG, TILES = 2 * KG, OWN = TILES / SPLIT, TPW = OWN / WAVES;
@@ -225,78 +230,101 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
         }
   };
   // SPLIT > 1: an exchange moves a split (or both) from the tile's waves to all
-  // its workgroups. It alternates between two buffers: a wave writes one again
-  // two exchanges later, when every wave has reached the one between and so has
-  // read it. The counts go on from launch to launch (a.epoch), so a flag of an
-  // earlier launch never passes for one of this.
+  // its workgroups, in device scope. A reader takes each word from memory until
+  // it is not kEmpty, so nothing is waited for but the data. Exchanges take
+  // turns on three buffers. After exchange e every wave has read e - 1, and its
+  // writer empties it; that is out before the writer's words of e + 1, and so
+  // before anyone who has them looks there for exchange e + 2.
   uint64_t* const flags = a.flags + (uint64_t)tile * kMaxRowTiles;
-  uint64_t* const xbuf = a.xbuf + (uint64_t)tile * 4 * 8 * K;  // [exchange % 2][dof][8 K]
-  uint64_t epoch = a.epoch;
-  bool lost = false;
-  // Device scope throughout, past the L1 and the L2 of an XCD (2.3 us an
-  // exchange of one tile at K = 384). With all of a tile's workgroups on one XCD
-  // its L2 could serve, but only an acquire fence drops the L1, and fences of
-  // many waves hold each other up: 24 tiles 10.8 us a step against 8.5, 80 tiles
-  // 54 against 12.4.
+  uint64_t* const xbuf = a.xbuf + (uint64_t)tile * kXbufs * 2 * 8 * K;  // [buffer][dof][8 K]
+  int cur = 0, old = kXbufs - 1;  // buffers of this exchange and the one before
+  bool both = false, lost = false;    // the exchange before moved both dofs; a word never came
   auto put = [](uint64_t* x, uint64_t v) { __hip_atomic_store(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
   auto get = [](const uint64_t* x) { return __hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  // waits until every wave of the tile has come as far (the launch is
-  // cooperative, so they run; should one never come, the wave goes on without it
-  // and its rows become NaN)
-  auto meet = [&] {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's rows are out
-    const uint64_t want = epoch + 1;
-    if (lane == 0) put(flags + part * WAVES + wave, want);
-    for (uint32_t tries = 0; !lost; ++tries) {
-      uint64_t f = want;
-      if (lane < SPLIT * WAVES) f = get(flags + lane);
-      if (__ballot(f < want) == 0) break;
-      lost = tries > kMaxTries;
-    }
-    asm volatile("" ::: "memory");
-  };
+  auto written = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+  // place of this lane's rows of tile t among the words of a buffer's dof
+  auto word = [&](int t) { return 2 * ((4 * (rt[t] / 2) + lane / 16) * kTileCols + col) + rt[t] % 2; };
   auto publish = [&](int dof, double (&q)[TPW][4]) {
-    uint64_t* x = xbuf + ((epoch % 2) * 2 + dof) * 8 * K;
+    uint64_t* x = xbuf + (cur * 2 + dof) * 8 * K;
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
-      u2 h, l;
-      splitRowsHw(q[t], h, l);
-      const int item = 2 * ((4 * (rt[t] / 2) + lane / 16) * kTileCols + col) + rt[t] % 2;
-      put(x + item, __builtin_bit_cast(uint64_t, h));
-      put(x + 2 * lo + item, __builtin_bit_cast(uint64_t, l));
+      u2 hl[2];
+      splitRowsHw(q[t], hl[0], hl[1]);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const uint64_t w = __builtin_bit_cast(uint64_t, hl[p]);
+        put(x + p * 2 * lo + word(t), w == kEmpty ? kEmpty >> 1 : w);
+      }
     }
   };
+  auto empty = [&](int buf, int dof) {
+    uint64_t* x = xbuf + (buf * 2 + dof) * 8 * K;
+#pragma unroll
+    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) put(x + p * 2 * lo + word(t), kEmpty);
+  };
+  // (The launch is cooperative, so the other workgroups run and every word
+  // comes. Should one not, the wave goes on with what it has: kEmpty is NaNs.)
   auto collect = [&](int dof, int4v* S) {
-    const uint64_t* x = xbuf + ((epoch % 2) * 2 + dof) * 8 * K;
-    uint64_t* d = reinterpret_cast<uint64_t*>(S);
+    const uint64_t* x = xbuf + (cur * 2 + dof) * 8 * K + tid;
+    uint64_t* d = reinterpret_cast<uint64_t*>(S) + tid;
     constexpr int N = 8 * K / (64 * WAVES);
     static_assert(8 * K % (64 * WAVES) == 0, "whole rounds");
     uint64_t v[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = get(x + i * 64 * WAVES + tid);
+    for (int i = 0; i < N; ++i) v[i] = kEmpty;
+    for (uint32_t tries = 0;; ++tries) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) d[i * 64 * WAVES + tid] = v[i];
+      for (int i = 0; i < N; ++i)
+        if (v[i] == kEmpty) v[i] = get(x + i * 64 * WAVES);
+      bool missing = false;
+#pragma unroll
+      for (int i = 0; i < N; ++i) missing |= v[i] == kEmpty;
+      if (lost || __ballot(missing) == 0) break;
+      lost = tries > kMaxTries;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) d[i * 64 * WAVES] = v[i];
   };
-  auto poison = [&](double (&q)[TPW][4]) {
-    if (lost)
-#pragma unroll
-      for (int t = 0; t < TPW; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) q[t][r] = __builtin_nan("");
+  auto turn = [&] {
+    old = cur;
+    cur = cur + 1 == kXbufs ? 0 : cur + 1;
   };
+  if (SPLIT > 1 && steps) {
+    // once a launch: all buffers empty, in every wave of the tile, before the
+    // first exchange (flags count launches)
+    for (int x = 0; x < kXbufs; ++x) {
+      empty(x, 0);
+      empty(x, 1);
+    }
+    written();
+    if (lane == 0) put(flags + part * WAVES + wave, a.launch);
+    for (uint32_t tries = 0; !lost; ++tries) {
+      uint64_t f = a.launch;
+      if (lane < SPLIT * WAVES) f = get(flags + lane);
+      if (__ballot(f != a.launch) == 0) break;
+      lost = tries > kMaxTries;
+    }
+    asm volatile("" ::: "memory");
+  }
   // the new split of a dof to every wave that reads it
   auto share = [&](int dof, double (&q)[TPW][4], int4v* S) {
     if constexpr (SPLIT == 1) {
 #pragma unroll
       for (int t = 0; t < TPW; ++t) writeSplitRowsHw(S, lo, rt[t], lane, q[t]);
     } else {
+      written();
       publish(dof, q);
-      meet();
       collect(dof, S);
-      poison(q);
-      ++epoch;
     }
     __syncthreads();
+    if constexpr (SPLIT > 1) {
+      empty(old, 1 - dof);
+      if (both) empty(old, dof);
+      both = false;
+      turn();
+    }
   };
   constexpr int RW = SPLIT * WAVES;  // waves that take the receivers' row tiles
 #pragma nounroll
@@ -406,16 +434,20 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
               writeSplitRowsHw(Ss, lo, rt[t], lane, qs[t]);
             }
           } else {
+            written();
             publish(0, qv);
             publish(1, qs);
-            meet();
+            __syncthreads();  // every read of the old splits done
             collect(0, Sv);
             collect(1, Ss);
-            poison(qv);
-            poison(qs);
-            ++epoch;
           }
           __syncthreads();  // the new splits complete
+          if constexpr (SPLIT > 1) {
+            empty(old, 0);
+            empty(old, 1);
+            both = true;
+            turn();
+          }
           // the macro step's last step is sampled when it ends at a multiple of the period
           const uint64_t sn = (uint64_t)s0 + mk + (uint64_t)(it + 1) * a.macro;
           const bool smp = act && ev > 0 && sn % ev == 0;
@@ -445,69 +477,73 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
 }
 
 template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, int SPLIT = 1>
-void launchKG(RomArgs a, uint32_t tiles, hipStream_t stream) {
+bool launchKG(RomArgs a, uint32_t tiles, hipStream_t stream) {
   constexpr size_t lds = (8 * 32 * KG + (size_t)2 * (2 * KG / SPLIT) * LL * PARTS * 64) * 16;
   static_assert(lds <= 160 * 1024 && 2 * KG <= kMaxRowTiles, "LDS of one CU, a flag per wave");
   auto go = [&](auto kernel) {
     SHAW_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if constexpr (SPLIT == 1) {
       hipLaunchKernelGGL(kernel, dim3(tiles), dim3(WAVES * 64), lds, stream, a);
+      return true;
     } else {
       void* args[] = {&a};
-      SHAW_HIP(hipLaunchCooperativeKernel((const void*)kernel, dim3((tiles + 7) / 8 * 8 * SPLIT), dim3(WAVES * 64), args,
-                                          (unsigned)lds, stream));
+      const hipError_t e = hipLaunchCooperativeKernel((const void*)kernel, dim3((tiles + 7) / 8 * 8 * SPLIT),
+                                                      dim3(WAVES * 64), args, (unsigned)lds, stream);
+      if (e == hipErrorCooperativeLaunchTooLarge) (void)hipGetLastError();
+      else SHAW_HIP(e);
+      return e == hipSuccess;
     }
   };
-  if (a.macro) go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, true, SPLIT>);
-  else go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, false, SPLIT>);
+  return a.macro ? go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, true, SPLIT>)
+                 : go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, false, SPLIT>);
 }
 
 }  // namespace
 
-uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols) {
+// The workgroups of a tile of 16 columns of a BF16 engine (1: one): four row
+// tiles each, or eight, while the chip holds all workgroups at once, one to a CU.
+// Not up to 256 modes: BF16x4 4.5 us a step in one workgroup, 4.2 in four, which
+// a cooperative launch of a few steps takes back; BF16x3 2.7, two exchanges 2.8.
+uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus) {
+  if (parts == 0 || modes < 384) return 1;
+  const uint32_t most = modes / 64;
+  for (const uint32_t split : {most, most / 2})
+    if ((tiles + 7) / 8 * 8 * split <= (uint64_t)cus) return split;
+  return 1;
+}
+uint64_t residentExchange(uint32_t modes, uint64_t tiles) { return tiles * kXbufs * 2 * 8 * modes; }
+
+uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int cus) {
   const uint64_t k = kv > ks ? kv : ks;
   // FP64 pads both dofs alike where k_rom_f64 runs them whatever the load, or
   // where that costs k_rom_steps nothing
   if (parts == 0 && cols > 2048 && k > 128 && (kv + 63) / 64 != (ks + 63) / 64) return 0;
   if (k <= 256) return (uint32_t)((k + 63) / 64 * 64);
   const uint32_t modes = k <= 384 ? 384 : 512;
-  // BF16: nearly all of the operators stream, and a square pad of unequal dofs
-  // would add to it
-  if (parts) return (kv + 127) / 128 == (ks + 127) / 128 ? modes : 0;
+  // BF16: one workgroup a tile streams nearly all of the operators, and a square
+  // pad of unequal dofs would add to it
+  if (parts)
+    return (kv + 127) / 128 == (ks + 127) / 128 || residentSplit(parts, modes, (cols + kTileCols - 1) / kTileCols, cus) > 1
+               ? modes
+               : 0;
   // FP64: K = 384, 2048 columns: 35.4 us a step against 38.2; K = 512 1024
   // columns 34.5 against 65.6, 2048 67.1 against 65.5
   return cols <= (k <= 384 ? 2048 : 1024) ? modes : 0;
 }
 
-// The workgroups of a tile of 16 columns of a BF16 engine (1: one): four row
-// tiles each, or eight, while the chip holds all workgroups at once, one to a
-// CU. Not up to 256 modes (one workgroup: BF16x4 4.3 us a step, two exchanges
-// alone 4.6), nor BF16x3 of 384 in threes (10.2 us at 1280 columns against 9.6).
-uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus) {
-  if (parts == 0 || modes < 384) return 1;
-  const uint32_t most = modes / 64;
-  auto fits = [&](uint32_t split) { return (tiles + 7) / 8 * 8 * split <= (uint64_t)cus; };
-  if (fits(most)) return most;
-  return fits(most / 2) && !(parts == 2 && modes == 384) ? most / 2 : 1;
-}
-uint64_t residentExchange(uint32_t modes, uint64_t tiles) { return tiles * 4 * 8 * modes; }
-
 void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream) {
   const int kg = (int)a.Kvp / 32;
   const uint32_t grid = a.tiles;
-  if (split > 1) {
+  // (false: the runtime sees no room for all workgroups at once)
+  auto shared = [&] {
     if (parts == 2) {
-      if (kg == 12) launchKG<2, 12, 4, 8, 4, 1, 6>(a, grid, stream);
-      else if (split == 8) launchKG<2, 16, 4, 10, 6, 1, 8>(a, grid, stream);
-      else launchKG<2, 16, 8, 9, 3, 1, 4>(a, grid, stream);
-    } else {
-      if (kg == 12 && split == 6) launchKG<3, 12, 4, 8, 4, 1, 6>(a, grid, stream);
-      else if (kg == 12) launchKG<3, 12, 8, 6, 2, 1, 3>(a, grid, stream);
-      else if (split == 8) launchKG<3, 16, 4, 12, 4, 1, 8>(a, grid, stream);
-      else launchKG<3, 16, 8, 6, 2, 1, 4>(a, grid, stream);
+      if (kg == 12) return split == 6 ? launchKG<2, 12, 4, 8, 4, 1, 6>(a, grid, stream) : launchKG<2, 12, 8, 9, 3, 1, 3>(a, grid, stream);
+      return split == 8 ? launchKG<2, 16, 4, 10, 6, 1, 8>(a, grid, stream) : launchKG<2, 16, 8, 9, 3, 1, 4>(a, grid, stream);
     }
-    return;
-  }
+    if (kg == 12) return split == 6 ? launchKG<3, 12, 4, 8, 4, 1, 6>(a, grid, stream) : launchKG<3, 12, 8, 6, 2, 1, 3>(a, grid, stream);
+    return split == 8 ? launchKG<3, 16, 4, 12, 4, 1, 8>(a, grid, stream) : launchKG<3, 16, 8, 6, 2, 1, 4>(a, grid, stream);
+  };
+  if (split > 1 && shared()) return;
   if (parts == 2) {
     switch (kg) {
       case 2: launchKG<2, 2, 4, 2, 0, 1>(a, grid, stream); break;

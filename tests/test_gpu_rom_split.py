@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 # kv, ks, columns: eight row tiles a workgroup at the first sizes of a mode
 # count, four at the last
-SIZES = [(257, 300, 1), (384, 384, 640), (384, 290, 641), (400, 512, 17), (512, 512, 512), (500, 487, 513)]
+SIZES = [(257, 300, 1), (384, 384, 640), (384, 290, 641), (380, 250, 1280), (290, 200, 1023), (400, 512, 17), (512, 512, 512), (500, 487, 513)]
 
 
 def run(arv, ars, rows, b, f, horizons, precision, macro, cols):
