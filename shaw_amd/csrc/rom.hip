@@ -924,7 +924,7 @@ struct shaw_rom {
   double dt = 0;
   int precision = 0;
   uint32_t resident = 0;  // padded modes per dof when the operators stay on the CU (k_rom_resident), else 0
-  uint32_t split = 1;     // workgroups of a tile of columns there, their exchange buffers and flags
+  uint32_t split = 1, sets = 1;  // workgroups that share columns there; FP64, the sets of four; buffers and flags
   shaw::DevBuf<uint64_t> xbuf, flags;
   uint64_t launches = 0;
   int parts() const { return precision == SHAW_ROM_FP64 ? 0 : precision == SHAW_ROM_BF16X3 ? 2 : 3; }
@@ -1046,12 +1046,14 @@ struct shaw_rom {
     a.launch = ++launches;
     const dim3 grid((unsigned)(maxCols / kTileCols));
     const size_t lds = ldsBytes();
-    if (resident && precision != SHAW_ROM_FP64) {
-      // a cooperative launch and its first meeting cost about what three steps
-      // save (1280 columns of K = 384 BF16x3, launches in a row: 4 steps 56 us
-      // against 57, 2 steps 48 against 37)
-      launchRomResident(parts(), a, nsteps >= 4 ? split : 1, stream);
-    } else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, maxCols, stream);
+    // a cooperative launch and its first meeting cost about what three steps
+    // save (1280 columns of K = 384 BF16x3, launches in a row: 4 steps 56 us
+    // against 57, 2 steps 48 against 37), about what nine do at 256 modes FP64 (4
+    // steps 41 us against 34, 16 steps 87 against 110)
+    const bool shared = split > 1 && nsteps >= (precision == SHAW_ROM_FP64 && resident == 256 ? 10 : 4);
+    if (resident && precision != SHAW_ROM_FP64) launchRomResident(parts(), a, shared ? split : 1, stream);
+    else if (shared && launchRomF64Shared(a, sets, stream)) {}
+    else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, stream);
     else if (precision == SHAW_ROM_FP64) launchRomSteps<0>(tpw, grid, lds, stream, a);
     else if (precision == SHAW_ROM_BF16X3) launchRomSteps<2>(tpw, grid, lds, stream, a);
     else launchRomSteps<3>(tpw, grid, lds, stream, a);
@@ -1308,10 +1310,10 @@ int shaw_rom_create(const shaw_rom_desc* d, shaw_rom_t* out) {
     }
     pack(cPad.data(), h->rp, d->kv, h->rp, h->kvp, h->c);
     const uint64_t C = h->maxCols;
-    h->split = residentSplit(h->resident ? h->parts() : 0, h->resident, C / kTileCols, cus);
+    h->split = residentSplit(h->parts(), h->resident, C / kTileCols, cus, h->sets);
     if (h->split > 1) {
       h->xbuf.alloc(residentExchange(h->resident, C / kTileCols));
-      h->flags.alloc(C / kTileCols * kMaxRowTiles);
+      h->flags.alloc(C / 4 * kMaxRowTiles);  // groups of columns are four or more
       SHAW_HIP(hipMemset(h->flags.p, 0, h->flags.n * sizeof(uint64_t)));
     }
     h->qv.alloc(C * h->kvp); h->qs.alloc(C * h->ksp); h->b.alloc(C * h->kvp);

@@ -46,9 +46,8 @@ struct RomArgs {
   // time of nsteps one-steps for every tile, a macro step costing w of them,
   // so tiles taking macro steps advance further (stepCol holds how far)
   uint32_t budget;
-  // tiles of 16 columns; and where several workgroups share one (k_rom_resident
-  // with SPLIT > 1): each tile's exchange buffers and kMaxRowTiles flags, and the
-  // launch's number, from 1
+  // tiles of 16 columns; and where several workgroups share columns (SPLIT > 1):
+  // exchange buffers, kMaxRowTiles flags a tile, and the launch's number, from 1
   uint32_t tiles;
   uint64_t* xbuf;
   uint64_t* flags;
@@ -63,9 +62,63 @@ typedef short shrt4 __attribute__((ext_vector_type(4)));
 typedef short shrt16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTileCols = 16;  // column slots per workgroup
-constexpr uint32_t kMaxTries = 1u << 24;  // of a bounded wait, each a read of memory (about 10 s)
 constexpr int kMaxRowTiles = 32;
 constexpr int kWaves = 8;      // waves per ROM workgroup (16 at 9..16 row tiles)
+
+// ------------------------------------------------------------ exchange
+// Workgroups that share a tile of columns exchange states through memory, in
+// device scope, 64 bits at a time. A reader takes each word from memory until it
+// is not kEmpty (four bf16 NaNs, a double's NaN), so nothing is waited for but
+// the data. Exchanges of a tile take turns on three buffers. After exchange e
+// every wave has read e - 1, and its writer empties it; that is out (written)
+// before the writer's words of e + 1, and so before anyone who has them looks
+// there for exchange e + 2. (A fourth buffer, which leaves the emptying another
+// exchange, measured the same within 2 %.)
+constexpr uint64_t kEmpty = ~0ull;
+constexpr int kXbufs = 3;
+constexpr uint32_t kMaxTries = 1u << 24;  // of a bounded wait, each a read of memory (about 10 s)
+__device__ __forceinline__ void put(uint64_t* x, uint64_t v) {
+  __hip_atomic_store(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get(const uint64_t* x) {
+  return __hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void putWord(uint64_t* x, uint64_t v) { put(x, v == kEmpty ? kEmpty >> 1 : v); }
+__device__ __forceinline__ void written() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// d[i * STRIDE] = x[i * STRIDE], i < N, once all are there. (The launch is
+// cooperative, so the other workgroups run and every word comes. Should one not,
+// lost is set and the wave goes on with what it has: kEmpty is NaN.)
+template <int N, int STRIDE>
+__device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, bool& lost) {
+  uint64_t v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = kEmpty;
+  for (uint32_t tries = 0;; ++tries) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (v[i] == kEmpty) v[i] = get(x + i * STRIDE);
+    bool missing = false;
+#pragma unroll
+    for (int i = 0; i < N; ++i) missing |= v[i] == kEmpty;
+    if (lost || __ballot(missing) == 0) break;
+    lost = tries > kMaxTries;
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) d[i * STRIDE] = v[i];
+}
+// waits until all `waves` (at most 64) waves of a tile have come here in this
+// launch with what they wrote; flags count launches, this wave's is flags[own]
+__device__ __forceinline__ void joinTile(uint64_t* flags, int own, int waves, int lane, uint64_t launch, bool& lost) {
+  written();
+  if (lane == 0) put(flags + own, launch);
+  for (uint32_t tries = 0; !lost; ++tries) {
+    uint64_t f = launch;
+    if (lane < waves) f = get(flags + lane);
+    if (__ballot(f != launch) == 0) break;
+    lost = tries > kMaxTries;
+  }
+  asm volatile("" ::: "memory");
+}
 
 // ------------------------------------------------------------ bf16 helpers
 __host__ __device__ inline unsigned short f32ToBf16(float x) {

@@ -65,13 +65,17 @@ void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t
 // columns, k_rom_steps taking the same operators with the same results).
 struct RomArgs;
 uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int cus);
-// The workgroups that share a tile of 16 columns (BF16), the 64-bit words of
-// a.xbuf that they then need, and the launch, cooperative if split > 1.
-uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus);
+// How many workgroups share a tile of 16 columns (BF16) or sets of four (FP64),
+// the 64-bit words of a.xbuf that they then need, and the launches: cooperative
+// with split > 1 and for launchRomF64Shared, which is false where the runtime
+// sees no room for all workgroups at once (launchCooperative).
+uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus, uint32_t& sets);
 uint64_t residentExchange(uint32_t modes, uint64_t tiles);
 void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream);
 bool romF64Fits(uint32_t modes, uint64_t activeTiles);
-void launchRomF64(const RomArgs& a, uint64_t cols, hipStream_t stream);
+void launchRomF64(const RomArgs& a, hipStream_t stream);
+bool launchRomF64Shared(const RomArgs& a, uint32_t sets, hipStream_t stream);
+bool launchCooperative(const void* kernel, unsigned groups, unsigned threads, size_t lds, const RomArgs& a, hipStream_t stream);
 uint64_t projPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);
 uint32_t gramChunks(uint64_t n, uint64_t Ka, uint64_t Kb);
 uint64_t gramPartDoubles(uint64_t n, uint64_t Ka, uint64_t Kb);

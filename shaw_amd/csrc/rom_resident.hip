@@ -11,10 +11,6 @@
 namespace shaw {
 namespace {
 
-// words of an exchange buffer without a value: four NaNs' bits; the buffers
-constexpr uint64_t kEmpty = ~0ull;
-constexpr int kXbufs = 3;
-
 typedef float flt2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
@@ -230,18 +226,11 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
         }
   };
   // SPLIT > 1: an exchange moves a split (or both) from the tile's waves to all
-  // its workgroups, in device scope. A reader takes each word from memory until
-  // it is not kEmpty, so nothing is waited for but the data. Exchanges take
-  // turns on three buffers. After exchange e every wave has read e - 1, and its
-  // writer empties it; that is out before the writer's words of e + 1, and so
-  // before anyone who has them looks there for exchange e + 2.
+  // its workgroups
   uint64_t* const flags = a.flags + (uint64_t)tile * kMaxRowTiles;
   uint64_t* const xbuf = a.xbuf + (uint64_t)tile * kXbufs * 2 * 8 * K;  // [buffer][dof][8 K]
   int cur = 0, old = kXbufs - 1;  // buffers of this exchange and the one before
   bool both = false, lost = false;    // the exchange before moved both dofs; a word never came
-  auto put = [](uint64_t* x, uint64_t v) { __hip_atomic_store(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  auto get = [](const uint64_t* x) { return __hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-  auto written = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
   // place of this lane's rows of tile t among the words of a buffer's dof
   auto word = [&](int t) { return 2 * ((4 * (rt[t] / 2) + lane / 16) * kTileCols + col) + rt[t] % 2; };
   auto publish = [&](int dof, double (&q)[TPW][4]) {
@@ -251,10 +240,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       u2 hl[2];
       splitRowsHw(q[t], hl[0], hl[1]);
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const uint64_t w = __builtin_bit_cast(uint64_t, hl[p]);
-        put(x + p * 2 * lo + word(t), w == kEmpty ? kEmpty >> 1 : w);
-      }
+      for (int p = 0; p < 2; ++p)
+        putWord(x + p * 2 * lo + word(t), __builtin_bit_cast(uint64_t, hl[p]));
     }
   };
   auto empty = [&](int buf, int dof) {
@@ -264,49 +251,21 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) put(x + p * 2 * lo + word(t), kEmpty);
   };
-  // (The launch is cooperative, so the other workgroups run and every word
-  // comes. Should one not, the wave goes on with what it has: kEmpty is NaNs.)
   auto collect = [&](int dof, int4v* S) {
-    const uint64_t* x = xbuf + (cur * 2 + dof) * 8 * K + tid;
-    uint64_t* d = reinterpret_cast<uint64_t*>(S) + tid;
-    constexpr int N = 8 * K / (64 * WAVES);
     static_assert(8 * K % (64 * WAVES) == 0, "whole rounds");
-    uint64_t v[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = kEmpty;
-    for (uint32_t tries = 0;; ++tries) {
-#pragma unroll
-      for (int i = 0; i < N; ++i)
-        if (v[i] == kEmpty) v[i] = get(x + i * 64 * WAVES);
-      bool missing = false;
-#pragma unroll
-      for (int i = 0; i < N; ++i) missing |= v[i] == kEmpty;
-      if (lost || __ballot(missing) == 0) break;
-      lost = tries > kMaxTries;
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) d[i * 64 * WAVES] = v[i];
+    collectWords<8 * K / (64 * WAVES), 64 * WAVES>(xbuf + (cur * 2 + dof) * 8 * K + tid, reinterpret_cast<uint64_t*>(S) + tid,
+                                                   lost);
   };
   auto turn = [&] {
     old = cur;
     cur = cur + 1 == kXbufs ? 0 : cur + 1;
   };
   if (SPLIT > 1 && steps) {
-    // once a launch: all buffers empty, in every wave of the tile, before the
-    // first exchange (flags count launches)
     for (int x = 0; x < kXbufs; ++x) {
       empty(x, 0);
       empty(x, 1);
     }
-    written();
-    if (lane == 0) put(flags + part * WAVES + wave, a.launch);
-    for (uint32_t tries = 0; !lost; ++tries) {
-      uint64_t f = a.launch;
-      if (lane < SPLIT * WAVES) f = get(flags + lane);
-      if (__ballot(f != a.launch) == 0) break;
-      lost = tries > kMaxTries;
-    }
-    asm volatile("" ::: "memory");
+    joinTile(flags, part * WAVES + wave, SPLIT * WAVES, lane, a.launch, lost);
   }
   // the new split of a dof to every wave that reads it
   auto share = [&](int dof, double (&q)[TPW][4], int4v* S) {
@@ -486,12 +445,7 @@ bool launchKG(RomArgs a, uint32_t tiles, hipStream_t stream) {
       hipLaunchKernelGGL(kernel, dim3(tiles), dim3(WAVES * 64), lds, stream, a);
       return true;
     } else {
-      void* args[] = {&a};
-      const hipError_t e = hipLaunchCooperativeKernel((const void*)kernel, dim3((tiles + 7) / 8 * 8 * SPLIT),
-                                                      dim3(WAVES * 64), args, (unsigned)lds, stream);
-      if (e == hipErrorCooperativeLaunchTooLarge) (void)hipGetLastError();
-      else SHAW_HIP(e);
-      return e == hipSuccess;
+      return launchCooperative((const void*)kernel, (tiles + 7) / 8 * 8 * SPLIT, WAVES * 64, lds, a, stream);
     }
   };
   return a.macro ? go(k_rom_resident<PARTS, KG, WAVES, RR, LL, DR, true, SPLIT>)
@@ -500,15 +454,34 @@ bool launchKG(RomArgs a, uint32_t tiles, hipStream_t stream) {
 
 }  // namespace
 
-// The workgroups of a tile of 16 columns of a BF16 engine (1: one): four row
-// tiles each, or eight, while the chip holds all workgroups at once, one to a CU.
-// Not up to 256 modes: BF16x4 4.5 us a step in one workgroup, 4.2 in four, which
-// a cooperative launch of a few steps takes back; BF16x3 2.7, two exchanges 2.8.
-uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus) {
-  if (parts == 0 || modes < 384) return 1;
+bool launchCooperative(const void* kernel, unsigned groups, unsigned threads, size_t lds, const RomArgs& a, hipStream_t stream) {
+  RomArgs copy = a;
+  void* args[] = {&copy};
+  const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(groups), dim3(threads), args, (unsigned)lds, stream);
+  if (e == hipErrorCooperativeLaunchTooLarge) (void)hipGetLastError();
+  else SHAW_HIP(e);
+  return e == hipSuccess;
+}
+
+// BF16, the workgroups of a tile of 16 columns (1: one): four row tiles each, or
+// eight, while the chip holds all workgroups at once, one to a CU. Not up to 256
+// modes: BF16x4 4.5 us a step in one workgroup, 4.2 in four, which a cooperative
+// launch of a few steps takes back; BF16x3 2.7, two exchanges 2.8. FP64, those of
+// one set of four columns or, above 256 modes, of two, four row tiles each.
+uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus, uint32_t& sets) {
+  sets = 1;
   const uint32_t most = modes / 64;
+  auto fits = [&](uint64_t groups, uint32_t split) { return (groups + 7) / 8 * 8 * split <= (uint64_t)cus; };
+  if (parts == 0) {
+    if (modes < 256) return 1;
+    if (fits(4 * tiles, most)) return most;
+    if (modes == 256 || !fits(2 * tiles, most)) return 1;
+    sets = 2;
+    return most;
+  }
+  if (modes < 384) return 1;
   for (const uint32_t split : {most, most / 2})
-    if ((tiles + 7) / 8 * 8 * split <= (uint64_t)cus) return split;
+    if (fits(tiles, split)) return split;
   return 1;
 }
 uint64_t residentExchange(uint32_t modes, uint64_t tiles) { return tiles * kXbufs * 2 * 8 * modes; }
@@ -522,10 +495,11 @@ uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int c
   const uint32_t modes = k <= 384 ? 384 : 512;
   // BF16: one workgroup a tile streams nearly all of the operators, and a square
   // pad of unequal dofs would add to it
-  if (parts)
-    return (kv + 127) / 128 == (ks + 127) / 128 || residentSplit(parts, modes, (cols + kTileCols - 1) / kTileCols, cus) > 1
-               ? modes
-               : 0;
+  if (parts) {
+    uint32_t sets;
+    const bool shared = residentSplit(parts, modes, (cols + kTileCols - 1) / kTileCols, cus, sets) > 1;
+    return shared || (kv + 127) / 128 == (ks + 127) / 128 ? modes : 0;
+  }
   // FP64: K = 384, 2048 columns: 35.4 us a step against 38.2; K = 512 1024
   // columns 34.5 against 65.6, 2048 67.1 against 65.5
   return cols <= (k <= 384 ? 2048 : 1024) ? modes : 0;
@@ -534,7 +508,6 @@ uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int c
 void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream) {
   const int kg = (int)a.Kvp / 32;
   const uint32_t grid = a.tiles;
-  // (false: the runtime sees no room for all workgroups at once)
   auto shared = [&] {
     if (parts == 2) {
       if (kg == 12) return split == 6 ? launchKG<2, 12, 4, 8, 4, 1, 6>(a, grid, stream) : launchKG<2, 12, 8, 9, 3, 1, 3>(a, grid, stream);

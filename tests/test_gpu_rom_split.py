@@ -14,27 +14,26 @@ pytestmark = pytest.mark.gpu
 
 # kv, ks, columns: eight row tiles a workgroup at the first sizes of a mode
 # count, four at the last
-SIZES = [(257, 300, 1), (384, 384, 640), (384, 290, 641), (380, 250, 1280), (290, 200, 1023), (400, 512, 17), (512, 512, 512), (500, 487, 513)]
+SIZES = [(257, 300, 1), (384, 384, 640), (384, 290, 641), (290, 200, 1023), (380, 250, 1280), (400, 512, 17),
+         (512, 512, 512), (500, 487, 513)]
 
 
-def run(arv, ars, rows, b, f, horizons, precision, macro, cols):
+def run(arv, ars, rows, b, f, horizons, precision, macro, cols, filler=0):
     rom = shaw_amd.Rom(arv, ars, 0.2, precision, rows, max_cols=cols, max_samples=f.shape[0] // 5)
     if macro:
         rom.set_macro_steps(5)
     if macro == 2:
         rom.set_time_budget(2)
     slots = rom.admit(b, f, horizons, every=5)
+    if filler:
+        rom.admit(np.ones((b.shape[0], filler)), np.zeros((f.shape[0], filler)), [f.shape[0]] * filler, every=5)
     for n in (1, 2, 7, 90, 200):
         rom.advance(n)
     states = [rom.state(s) for s in slots[:3] + slots[-3:]]
     return rom.retire_many(slots, f.shape[0] // 5), states
 
 
-@pytest.mark.parametrize("macro", [0, 1, 2])
-@pytest.mark.parametrize("precision", [shaw_amd.ROM_BF16X3, shaw_amd.ROM_BF16X4])
-@pytest.mark.parametrize("kv,ks,m", SIZES)
-def test_shared_tile_equals_one_workgroup(kv, ks, m, precision, macro):
-    print(f"[gpu] shared ROM tile kv={kv} ks={ks} M={m} precision={precision} macro={macro}", flush=True)
+def compare(kv, ks, m, precision, macro, cols, filler=0):
     rng = np.random.default_rng(1000 * kv + ks + m)
     arv = rng.standard_normal((kv, ks)) * (0.5 / np.sqrt(max(kv, ks)))
     ars = -arv.T.copy()
@@ -44,7 +43,7 @@ def test_shared_tile_equals_one_workgroup(kv, ks, m, precision, macro):
     f[100:] = 0.0
     horizons = [300 - 5 * (j % 7) for j in range(m)]
     one = run(arv, ars, rows, b, f, horizons, precision, macro, m)
-    two = run(arv, ars, rows, b, f, horizons, precision, macro, 2048)
+    two = run(arv, ars, rows, b, f, horizons, precision, macro, cols, filler)
     for x, y in zip(one[0], two[0]):
         np.testing.assert_array_equal(x, y)
     for x, y in zip(one[1], two[1]):
@@ -52,3 +51,23 @@ def test_shared_tile_equals_one_workgroup(kv, ks, m, precision, macro):
         np.testing.assert_array_equal(x[0], y[0])
         np.testing.assert_array_equal(x[1], y[1])
     assert max(np.abs(x).max() for x in one[0]) > 0
+
+
+@pytest.mark.parametrize("macro", [0, 1, 2])
+@pytest.mark.parametrize("precision", [shaw_amd.ROM_BF16X3, shaw_amd.ROM_BF16X4])
+@pytest.mark.parametrize("kv,ks,m", SIZES)
+def test_shared_tile_equals_one_workgroup(kv, ks, m, precision, macro):
+    print(f"[gpu] shared ROM tile kv={kv} ks={ks} M={m} precision={precision} macro={macro}", flush=True)
+    compare(kv, ks, m, precision, macro, 2048)
+
+
+# one set and two, at the most columns of each; the engine of many columns runs workgroups of sixteen (up to 256 modes,
+# with enough of them active)
+@pytest.mark.parametrize("kv,ks,m,cols,filler", [(193, 256, 1, 2400, 2100), (256, 256, 256, 2400, 2100),
+                                                 (257, 384, 9, 2064, 0), (384, 384, 160, 2064, 0),
+                                                 (384, 300, 320, 2064, 0),
+                                                 (500, 487, 15, 2064, 0), (512, 512, 128, 2064, 0),
+                                                 (512, 400, 256, 2064, 0)])
+def test_shared_fp64_columns(kv, ks, m, cols, filler):
+    print(f"[gpu] shared FP64 ROM columns kv={kv} ks={ks} M={m}", flush=True)
+    compare(kv, ks, m, shaw_amd.ROM_FP64, 0, cols, filler)
