@@ -16,7 +16,7 @@
 // each operator; operators are pre-packed in MFMA operand order as lane
 // items and stream from L2 through a register ring per row tile, so the
 // loads of later k-steps are in flight while the MFMAs of earlier ones run
-// (BF16 operators of up to 256 modes stay on the CU: rom_resident.hip).
+// (most BF16 operators stay on the CU as far as they fit: rom_resident.hip).
 //   FP64:   v_mfma_f64_16x16x4f64, FP64 accumulation.
 //   BF16x3: Ar = Ar_hi + Ar_lo and q = q_hi + q_lo in bf16; the product uses
 //           Ar_hi q_hi + Ar_hi q_lo + Ar_lo q_hi on v_mfma_f32_16x16x32_bf16
@@ -228,7 +228,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_steps(RomArgs a) {
 }
 
 // The BF16x3 / BF16x4 reduced leapfrog with register-resident states, for
-// operators of more than 256 modes (k_rom_resident runs the smaller ones). As
+// operators of more than 256 modes whose dofs pad to different sizes, of more
+// columns than can be shared (k_rom_resident runs the others). As
 // k_rom_steps, one workgroup advances kTileCols column slots; here the FP64
 // states live in the registers of the wave that computes them (lane l holds
 // rows 16 rt + 4 (l / 16) + r of column l % 16 of each of its row tiles, the

@@ -20,7 +20,7 @@ namespace shaw {
 //           A[16t + l%16][32g + 16s + 4(l/16) + e] at position 4s + e,
 //           s < 2, e < 4 (the state's split uses the same k order).
 // Padded sizes are multiples of kRing groups (64 for FP64, 128 for BF16), of
-// two groups (64) for BF16 operators of up to 256 modes.
+// two groups (64) for engines of up to 256 modes whose operators stay on the CU.
 struct RomArgs {
   const void* av;       // Ar_v: rows Kvp, k-dim Ksp
   const void* as;       // Ar_s: rows Ksp, k-dim Kvp
