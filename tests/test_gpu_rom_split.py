@@ -71,3 +71,29 @@ def test_shared_tile_equals_one_workgroup(kv, ks, m, precision, macro):
 def test_shared_fp64_columns(kv, ks, m, cols, filler):
     print(f"[gpu] shared FP64 ROM columns kv={kv} ks={ks} M={m}", flush=True)
     compare(kv, ks, m, shaw_amd.ROM_FP64, 0, cols, filler)
+
+
+def test_shared_engines_side_by_side():
+    """Engines whose launches each want most of the chip, enqueued on their own
+    streams without a wait between, give what each gives alone."""
+    rng = np.random.default_rng(5)
+    engines = []
+    for kv, m, precision in ((384, 512, shaw_amd.ROM_BF16X4), (512, 128, shaw_amd.ROM_FP64), (500, 500, shaw_amd.ROM_BF16X3)):
+        arv = rng.standard_normal((kv, kv)) * (0.5 / np.sqrt(kv))
+        rows, b, f = rng.standard_normal((5, kv)), rng.standard_normal((kv, m)), rng.standard_normal((400, m))
+
+        def engine():
+            rom = shaw_amd.Rom(arv, -arv.T.copy(), 0.2, precision, rows, max_cols=m, max_samples=80)
+            return rom, rom.admit(b, f, [400] * m, every=5)
+
+        rom, slots = engine()
+        rom.advance(400)
+        alone = rom.retire_many(slots, 80)
+        engines.append((*engine(), alone))
+    for _ in range(8):
+        for rom, _, _ in engines:
+            rom.advance(50)
+    for rom, slots, alone in engines:
+        for x, y in zip(rom.retire_many(slots, 80), alone):
+            np.testing.assert_array_equal(x, y)
+            assert np.isfinite(x).all()
