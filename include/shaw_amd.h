@@ -564,6 +564,12 @@ int shaw_debug_mfma(int kind, const double* a, const double* b, double* d);
  * w[n] eigenvalues (unordered), v row-major [n x n] with eigenvectors in its
  * columns. CPU only. No reference counterpart.                             */
 int shaw_debug_symeig(int n, const double* a, double* w, double* v);
+/* How often a wave of workgroups that share ROM columns looks in vain before it
+ * gives up: at the launch's start, for the others to come (its columns then run
+ * unshared, with the same results), and within the launch, for a value of
+ * theirs (every later call on the engine that waits for it then fails with
+ * SHAW_ERR_HIP). Both 2^24 by default. No reference counterpart.            */
+int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, uint32_t word_tries);
 /* Time `reps` launches of a plain streaming copy kernel (k_copy) of `bytes`
  * bytes (read `bytes`, write `bytes`); used to calibrate the HBM traffic
  * counters and to state the achievable copy bandwidth. No reference

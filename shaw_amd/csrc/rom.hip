@@ -925,9 +925,15 @@ struct shaw_rom {
   double dt = 0;
   int precision = 0;
   uint32_t resident = 0;  // padded modes per dof when the operators stay on the CU (k_rom_resident), else 0
-  uint32_t split = 1, sets = 1;  // workgroups that share columns there; FP64, the sets of four; buffers and flags
-  shaw::DevBuf<uint64_t> xbuf, flags;
+  uint32_t split = 1, sets = 1;  // workgroups that share columns there; FP64, the sets of four
+  shaw::DevBuf<uint64_t> xbuf, meet;  // their exchange buffers and meeting words
+  uint64_t* gaveUp = nullptr;         // pinned, [2]: RomArgs::gaveUp
+  uint32_t meetTries = shaw::kMaxTries, wordTries = shaw::kMaxTries;
   uint64_t launches = 0;
+  // the last shared launch, unchecked until it is known that every group met
+  // or a repeating launch is on the stream
+  shaw::RomArgs sharedArgs{};
+  bool unchecked = false;
   int parts() const { return precision == SHAW_ROM_FP64 ? 0 : precision == SHAW_ROM_BF16X3 ? 2 : 3; }
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -980,8 +986,33 @@ struct shaw_rom {
     }
     return static_cast<double*>(pinned);
   }
+  // Runs the groups that did not meet in the last shared launch, each in one
+  // workgroup, before anything else is enqueued; nothing where the stream is idle
+  // and the launch has not said that there are any. True if it enqueued a launch.
+  bool repeatShared(bool idle) {
+    if (!unchecked) return false;
+    const bool all = idle && __atomic_load_n(gaveUp, __ATOMIC_ACQUIRE) != sharedArgs.launch;
+    if (!all) {
+      shaw::RomArgs a = sharedArgs;
+      a.repeat = sets;
+      if (precision == SHAW_ROM_FP64) launchRomF64(a, stream);
+      else launchRomResident(parts(), a, 1, stream);
+      SHAW_HIP(hipGetLastError());
+    }
+    unchecked = false;
+    return !all;
+  }
+  bool idle() const {
+    const hipError_t e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) (void)hipGetLastError();
+    else SHAW_HIP(e);
+    return e == hipSuccess;
+  }
   void settle() {
     SHAW_HIP(hipStreamSynchronize(stream));
+    if (repeatShared(true)) SHAW_HIP(hipStreamSynchronize(stream));
+    SHAW_REQUIRE(!gaveUp || __atomic_load_n(gaveUp + 1, __ATOMIC_ACQUIRE) == 0, SHAW_ERR_HIP,
+                 "workgroups that share ROM columns lost each other within a launch: the engine's states are invalid");
     if (stepsOnDevice) {
       // through the pinned slot-table buffer (its uploads are done: the
       // stream is idle), on the engine's stream
@@ -1008,6 +1039,7 @@ struct shaw_rom {
     if (pinned) (void)hipHostFree(pinned);
     if (admitPinned) (void)hipHostFree(admitPinned);
     if (slotPinned) (void)hipHostFree(slotPinned);
+    if (gaveUp) (void)hipHostFree(gaveUp);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
@@ -1043,8 +1075,10 @@ struct shaw_rom {
     a.macro = precision == SHAW_ROM_FP64 ? 0 : macro;
     a.budget = a.macro ? timeBudget : 0;
     a.tiles = (uint32_t)(maxCols / kTileCols);
-    a.xbuf = xbuf.p; a.flags = flags.p;
+    a.xbuf = xbuf.p; a.meet = meet.p; a.gaveUp = gaveUp;
+    a.meetTries = meetTries; a.wordTries = wordTries;
     a.launch = ++launches;
+    if (unchecked) (void)repeatShared(idle());
     const dim3 grid((unsigned)(maxCols / kTileCols));
     const size_t lds = ldsBytes();
     // a cooperative launch and its first meeting cost about what three steps
@@ -1052,12 +1086,13 @@ struct shaw_rom {
     // against 57, 2 steps 48 against 37), about what nine do at 256 modes FP64 (4
     // steps 41 us against 34, 16 steps 87 against 110)
     const bool shared = split > 1 && nsteps >= (precision == SHAW_ROM_FP64 && resident == 256 ? 10 : 4);
-    if (resident && precision != SHAW_ROM_FP64) launchRomResident(parts(), a, shared ? split : 1, stream);
-    else if (shared && launchRomF64Shared(a, sets, stream)) {}
+    if (resident && precision != SHAW_ROM_FP64) unchecked = launchRomResident(parts(), a, shared ? split : 1, stream);
+    else if (shared && launchRomF64Shared(a, sets, stream)) unchecked = true;
     else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, stream);
     else if (precision == SHAW_ROM_FP64) launchRomSteps<0>(tpw, grid, lds, stream, a);
     else if (precision == SHAW_ROM_BF16X3) launchRomSteps<2>(tpw, grid, lds, stream, a);
     else launchRomSteps<3>(tpw, grid, lds, stream, a);
+    if (unchecked) sharedArgs = a;
     SHAW_HIP(hipGetLastError());
     if (a.budget) {
       stepsOnDevice = true;
@@ -1314,8 +1349,10 @@ int shaw_rom_create(const shaw_rom_desc* d, shaw_rom_t* out) {
     h->split = residentSplit(h->parts(), h->resident, C / kTileCols, cus, h->sets);
     if (h->split > 1) {
       h->xbuf.alloc(residentExchange(h->resident, C / kTileCols));
-      h->flags.alloc(C / 4 * kMaxRowTiles);  // groups of columns are four or more
-      SHAW_HIP(hipMemset(h->flags.p, 0, h->flags.n * sizeof(uint64_t)));
+      h->meet.alloc(C / 4 * kMeetStride);  // groups of columns are four or more
+      SHAW_HIP(hipMemset(h->meet.p, 0, h->meet.n * sizeof(uint64_t)));
+      SHAW_HIP(hipHostMalloc((void**)&h->gaveUp, 2 * sizeof(uint64_t)));
+      h->gaveUp[0] = h->gaveUp[1] = 0;
     }
     h->qv.alloc(C * h->kvp); h->qs.alloc(C * h->ksp); h->b.alloc(C * h->kvp);
     SHAW_HIP(hipMemset(h->qv.p, 0, h->qv.n * 8)); SHAW_HIP(hipMemset(h->qs.p, 0, h->qs.n * 8));
@@ -1638,12 +1675,10 @@ int shaw_rom_query(shaw_rom_t h, int* idle) {
   using namespace shaw;
   return guarded([&] {
     SHAW_REQUIRE(h && idle, SHAW_ERR_ARG, "null argument");
-    const hipError_t e = hipStreamQuery(h->stream);
-    if (e == hipErrorNotReady) {
+    if (!h->idle()) {
       *idle = 0;
       return;
     }
-    SHAW_HIP(e);
     h->settle();  // idle: reads back the steps of a time-budget launch
     *idle = 1;
   });
@@ -1663,6 +1698,10 @@ int shaw_rom_time(shaw_rom_t h, uint64_t nsteps, double* total) {
     h->launch(nsteps);
     SHAW_HIP(hipEventRecord(h->ev1, h->stream));
     SHAW_HIP(hipEventSynchronize(h->ev1));
+    if (h->repeatShared(true)) {
+      SHAW_HIP(hipEventRecord(h->ev1, h->stream));
+      SHAW_HIP(hipEventSynchronize(h->ev1));
+    }
     float ms = 0;
     SHAW_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
     *total = ms;
@@ -1737,6 +1776,14 @@ int shaw_debug_symeig(int n, const double* a, double* w, double* v) {
     symmetricEigen(A, n, ww, VV);
     std::copy(ww.begin(), ww.end(), w);
     std::copy(VV.begin(), VV.end(), v);
+  });
+}
+
+int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, uint32_t word_tries) {
+  return guarded([&] {
+    SHAW_REQUIRE(h, SHAW_ERR_ARG, "null handle");
+    h->meetTries = meet_tries;
+    h->wordTries = word_tries;
   });
 }
 

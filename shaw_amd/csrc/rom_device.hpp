@@ -47,11 +47,19 @@ struct RomArgs {
   // so tiles taking macro steps advance further (stepCol holds how far)
   uint32_t budget;
   // tiles of 16 columns; and where several workgroups share columns (SPLIT > 1):
-  // exchange buffers, kMaxRowTiles flags a tile, and the launch's number, from 1
+  // exchange buffers, the groups' meeting words (joinGroup), the launch's number,
+  // from 1, how often a wave looks in vain before it gives up, and host memory
+  // that says so: [0] the last launch in which a group did not meet, [1] the last
+  // in which a word of an exchange never came
   uint32_t tiles;
   uint64_t* xbuf;
-  uint64_t* flags;
+  uint64_t* meet;
   uint64_t launch;
+  uint32_t meetTries, wordTries;
+  uint64_t* gaveUp;
+  // sets > 0: a launch that repeats `launch` for the groups that did not meet in
+  // it, of that many workgroups of an unshared launch each; the others return
+  uint32_t repeat;
 };
 
 namespace {
@@ -62,12 +70,11 @@ typedef short shrt4 __attribute__((ext_vector_type(4)));
 typedef short shrt16 __attribute__((ext_vector_type(16)));
 
 constexpr int kTileCols = 16;  // column slots per workgroup
-constexpr int kMaxRowTiles = 32;
 constexpr int kWaves = 8;      // waves per ROM workgroup (16 at 9..16 row tiles)
 
 // ------------------------------------------------------------ exchange
 // Workgroups that share a tile of columns exchange states through memory, in
-// device scope, 64 bits at a time. A reader takes each word from memory until it
+// device scope, 64 bits at a time. (They have met first: joinGroup.) A reader takes each word from memory until it
 // is not kEmpty (four bf16 NaNs, a double's NaN), so nothing is waited for but
 // the data. Exchanges of a tile take turns on three buffers. After exchange e
 // every wave has read e - 1, and its writer empties it; that is out (written)
@@ -76,7 +83,8 @@ constexpr int kWaves = 8;      // waves per ROM workgroup (16 at 9..16 row tiles
 // exchange, measured the same within 2 %.)
 constexpr uint64_t kEmpty = ~0ull;
 constexpr int kXbufs = 3;
-constexpr uint32_t kMaxTries = 1u << 24;  // of a bounded wait, each a read of memory (about 10 s)
+constexpr int kMeetStride = 16;  // words from one group's meeting word to the next: a cache line each
+constexpr uint32_t kMaxTries = 1u << 24;  // looks of a bounded wait, each a read of memory (about 10 s)
 __device__ __forceinline__ void put(uint64_t* x, uint64_t v) {
   __hip_atomic_store(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -85,11 +93,11 @@ __device__ __forceinline__ uint64_t get(const uint64_t* x) {
 }
 __device__ __forceinline__ void putWord(uint64_t* x, uint64_t v) { put(x, v == kEmpty ? kEmpty >> 1 : v); }
 __device__ __forceinline__ void written() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-// d[i * STRIDE] = x[i * STRIDE], i < N, once all are there. (The launch is
-// cooperative, so the other workgroups run and every word comes. Should one not,
-// lost is set and the wave goes on with what it has: kEmpty is NaN.)
+// d[i * STRIDE] = x[i * STRIDE], i < N, once all are there. (The workgroups have
+// met, so all run and every word comes. Should one not, lost is set, the wave
+// goes on with what it has and reportLost tells the host.)
 template <int N, int STRIDE>
-__device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, bool& lost) {
+__device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, uint32_t maxTries, bool& lost) {
   uint64_t v[N];
 #pragma unroll
   for (int i = 0; i < N; ++i) v[i] = kEmpty;
@@ -101,23 +109,52 @@ __device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, boo
 #pragma unroll
     for (int i = 0; i < N; ++i) missing |= v[i] == kEmpty;
     if (lost || __ballot(missing) == 0) break;
-    lost = tries > kMaxTries;
+    lost = tries >= maxTries;
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) d[i * STRIDE] = v[i];
 }
-// waits until all `waves` (at most 64) waves of a tile have come here in this
-// launch with what they wrote; flags count launches, this wave's is flags[own]
-__device__ __forceinline__ void joinTile(uint64_t* flags, int own, int waves, int lane, uint64_t launch, bool& lost) {
+__device__ __forceinline__ void tellHost(uint64_t* word, uint64_t v) {
+  __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void reportLost(const RomArgs& a, bool lost, int lane) {
+  if (lost && lane == 0) tellHost(a.gaveUp + 1, a.launch);
+}
+// A group's meeting word: launch number, kNotMet, waves that came. All `waves`
+// waves of a group meet in a launch or none of them does: a wave that looked in
+// vain too often puts kNotMet in by a compare-exchange against a count that is not
+// full, which fails once the last wave has come, and a wave that finds kNotMet
+// gives up too. (A cooperative launch makes sure of the room on an empty chip only:
+// a long launch of another stream can keep part of a group waiting for a CU.) What
+// the wave wrote before is out when the others have met it.
+constexpr uint64_t kNotMet = 1u << 15;
+__device__ __forceinline__ bool joinGroup(const RomArgs& a, uint32_t group, uint32_t waves, int lane) {
   written();
-  if (lane == 0) put(flags + own, launch);
-  for (uint32_t tries = 0; !lost; ++tries) {
-    uint64_t f = launch;
-    if (lane < waves) f = get(flags + lane);
-    if (__ballot(f != launch) == 0) break;
-    lost = tries > kMaxTries;
+  bool met = false;
+  if (lane == 0) {
+    uint64_t* const word = a.meet + (uint64_t)group * kMeetStride;
+    (void)__hip_atomic_fetch_max(word, a.launch << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint64_t v = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+    for (uint32_t tries = 0;; ++tries) {
+      if (v & kNotMet) break;
+      met = (v & (kNotMet - 1)) == waves;
+      if (met) break;
+      if (tries < a.meetTries) {
+        v = get(word);
+      } else if (__hip_atomic_compare_exchange_strong(word, &v, v | kNotMet, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT)) {
+        tellHost(a.gaveUp, a.launch);
+        break;
+      }  // (else v is the word as it was: a wave has come or given up meanwhile, at most `waves` times)
+    }
   }
   asm volatile("" ::: "memory");
+  return __builtin_amdgcn_readfirstlane((int)met) != 0;
+}
+// whether an unshared workgroup of a repeating launch has anything to do
+__device__ __forceinline__ bool repeats(const RomArgs& a, uint32_t workgroup) {
+  const uint64_t v = a.meet[(uint64_t)(workgroup / a.repeat) * kMeetStride];
+  return (v >> 16) == a.launch && (v & kNotMet) != 0;
 }
 
 // ------------------------------------------------------------ bf16 helpers

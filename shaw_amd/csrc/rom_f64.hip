@@ -49,6 +49,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64(RomArgs a) {
   double* Xv = sm;           // [K][4] q_v
   double* Xs = Xv + K * kCols;
   dbl4* Al = reinterpret_cast<dbl4*>(Xs + K * kCols);  // [operator][tile][LL][lane]
+  if (a.repeat && !repeats(a, blockIdx.x)) return;
   const int slot0 = blockIdx.x * kCols;
   const int tid = threadIdx.x, lane = tid % 64, col = lane % kCols;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -370,7 +371,6 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
     nextIdx[u] = ev[u] ? (s0[u] + 1) / ev[u] : 0;
   }
   constexpr int RW = SPLIT * WAVES;  // waves that take the receivers' row tiles
-  static_assert(RW <= kMaxRowTiles, "a flag per wave");
   // exchanges of set u: half-steps 0 (q_v), 1 (q_s), 2, ... of the launch
   uint64_t* const xbuf = a.xbuf + (uint64_t)group * SETS * kXbufs * K * kCols;  // [set][buffer][K][4]
   int cur = 0, old = kXbufs - 1;  // buffers of this half-step and the one before
@@ -383,7 +383,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
 #pragma unroll
   for (int u = 0; u < SETS; ++u)
     for (int x = 0; x < kXbufs; ++x) empty(u, x);
-  joinTile(a.flags + (uint64_t)group * kMaxRowTiles, part * WAVES + wave, RW, lane, a.launch, lost);
+  if (!joinGroup(a, group, RW, lane)) return;  // nothing is changed: a repeating launch runs the columns
   // the new rows of q_v or q_s to all that read them
   auto share = [&](auto dofc) {
     constexpr int dof = decltype(dofc)::value;
@@ -396,7 +396,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
     static_assert(K * kCols % (64 * WAVES) == 0, "whole rounds");
 #pragma unroll
     for (int u = 0; u < SETS; ++u)
-      collectWords<K * kCols / (64 * WAVES), 64 * WAVES>(buffer(u, cur) + tid, reinterpret_cast<uint64_t*>(X(u, dof)) + tid, lost);
+      collectWords<K * kCols / (64 * WAVES), 64 * WAVES>(buffer(u, cur) + tid, reinterpret_cast<uint64_t*>(X(u, dof)) + tid,
+                                                        a.wordTries, lost);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < SETS; ++u) empty(u, old);
@@ -482,6 +483,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
       a.qv[at0] = q[u][0][t];
       a.qs[at0] = q[u][1][t];
     }
+  reportLost(a, lost, lane);
   // (all workgroups of the columns have read the counters: they have met)
   if (part == 0 && tid < kCols * SETS) {
     const uint64_t h = a.horizon[slot0 + tid];

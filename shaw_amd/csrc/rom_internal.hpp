@@ -67,11 +67,13 @@ struct RomArgs;
 uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int cus);
 // How many workgroups share a tile of 16 columns (BF16) or sets of four (FP64),
 // the 64-bit words of a.xbuf that they then need, and the launches: cooperative
-// with split > 1 and for launchRomF64Shared, which is false where the runtime
-// sees no room for all workgroups at once (launchCooperative).
+// with split > 1 and for launchRomF64Shared. Both return whether columns are
+// shared: not where the runtime sees no room for all workgroups at once
+// (launchCooperative). Groups that do not meet in a shared launch are left as
+// they were and run in an unshared one of the same arguments with a.repeat = sets.
 uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus, uint32_t& sets);
 uint64_t residentExchange(uint32_t modes, uint64_t tiles);
-void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream);
+bool launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream);
 bool romF64Fits(uint32_t modes, uint64_t activeTiles);
 void launchRomF64(const RomArgs& a, hipStream_t stream);
 bool launchRomF64Shared(const RomArgs& a, uint32_t sets, hipStream_t stream);

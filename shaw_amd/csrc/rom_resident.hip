@@ -81,6 +81,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   const int tile = SPLIT == 1 ? (int)blockIdx.x : (int)(blockIdx.x / (8 * SPLIT) * 8 + blockIdx.x % 8);
   const int part = SPLIT == 1 ? 0 : (int)(blockIdx.x / 8 % SPLIT);
   if (SPLIT > 1 && tile >= (int)a.tiles) return;
+  if (SPLIT == 1 && a.repeat && !repeats(a, blockIdx.x)) return;
   const int slot0 = tile * kTileCols;
   const int tid = threadIdx.x, lane = tid % 64, col = lane % 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -227,7 +228,6 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   };
   // SPLIT > 1: an exchange moves a split (or both) from the tile's waves to all
   // its workgroups
-  uint64_t* const flags = a.flags + (uint64_t)tile * kMaxRowTiles;
   uint64_t* const xbuf = a.xbuf + (uint64_t)tile * kXbufs * 2 * 8 * K;  // [buffer][dof][8 K]
   int cur = 0, old = kXbufs - 1;  // buffers of this exchange and the one before
   bool both = false, lost = false;    // the exchange before moved both dofs; a word never came
@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   auto collect = [&](int dof, int4v* S) {
     static_assert(8 * K % (64 * WAVES) == 0, "whole rounds");
     collectWords<8 * K / (64 * WAVES), 64 * WAVES>(xbuf + (cur * 2 + dof) * 8 * K + tid, reinterpret_cast<uint64_t*>(S) + tid,
-                                                   lost);
+                                                   a.wordTries, lost);
   };
   auto turn = [&] {
     old = cur;
@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       empty(x, 0);
       empty(x, 1);
     }
-    joinTile(flags, part * WAVES + wave, SPLIT * WAVES, lane, a.launch, lost);
+    if (!joinGroup(a, tile, SPLIT * WAVES, lane)) return;  // nothing is changed: a repeating launch runs the tile
   }
   // the new split of a dof to every wave that reads it
   auto share = [&](int dof, double (&q)[TPW][4], int4v* S) {
@@ -424,6 +424,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       a.qv[colQ + rt[t] * 16 + rowBf16(lane, r)] = qv[t][r];
       a.qs[colQ + rt[t] * 16 + rowBf16(lane, r)] = qs[t][r];
     }
+  if constexpr (SPLIT > 1) reportLost(a, lost, lane);
   // (no workgroup of the tile is still to read its counters or states: a tile
   // with steps has had an exchange, one without writes what it read)
   if (part == 0 && tid < kTileCols) {
@@ -438,7 +439,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
 template <int PARTS, int KG, int WAVES, int RR, int LL, int DR, int SPLIT = 1>
 bool launchKG(RomArgs a, uint32_t tiles, hipStream_t stream) {
   constexpr size_t lds = (8 * 32 * KG + (size_t)2 * (2 * KG / SPLIT) * LL * PARTS * 64) * 16;
-  static_assert(lds <= 160 * 1024 && 2 * KG <= kMaxRowTiles, "LDS of one CU, a flag per wave");
+  static_assert(lds <= 160 * 1024, "LDS of one CU");
   auto go = [&](auto kernel) {
     SHAW_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if constexpr (SPLIT == 1) {
@@ -505,7 +506,7 @@ uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int c
   return cols <= (k <= 384 ? 2048 : 1024) ? modes : 0;
 }
 
-void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream) {
+bool launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream) {
   const int kg = (int)a.Kvp / 32;
   const uint32_t grid = a.tiles;
   auto shared = [&] {
@@ -516,7 +517,7 @@ void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t 
     if (kg == 12) return split == 6 ? launchKG<3, 12, 4, 8, 4, 1, 6>(a, grid, stream) : launchKG<3, 12, 8, 6, 2, 1, 3>(a, grid, stream);
     return split == 8 ? launchKG<3, 16, 4, 12, 4, 1, 8>(a, grid, stream) : launchKG<3, 16, 8, 6, 2, 1, 4>(a, grid, stream);
   };
-  if (split > 1 && shared()) return;
+  if (split > 1 && shared()) return true;
   if (parts == 2) {
     switch (kg) {
       case 2: launchKG<2, 2, 4, 2, 0, 1>(a, grid, stream); break;
@@ -536,6 +537,7 @@ void launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t 
       default: launchKG<3, 16, 8, 0, 0, 1>(a, grid, stream); break;
     }
   }
+  return false;
 }
 
 }  // namespace shaw
