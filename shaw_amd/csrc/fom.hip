@@ -903,8 +903,9 @@ __global__ void __launch_bounds__(512) k_fusedN(StepArgsN<T, NS> aa) {
 // rotates by one lane (gfx9 family), a VALU move instead of a round trip
 // through the LDS crossbar. fromWest: lane p receives lane p - 1 (lane 0
 // receives lane 63, wave_ror:1); fromEast: lane p receives lane p + 1 (lane
-// 63 receives lane 0, wave_rol:1).
-constexpr int kDppWaveRol1 = 0x134, kDppWaveRor1 = 0x13C;
+// 63 receives lane 0, wave_rol:1). westOrZero, eastOrZero: shifts, which give
+// zero to the lane that has no neighbour (wave_shr:1, wave_shl:1).
+constexpr int kDppWaveRol1 = 0x134, kDppWaveRor1 = 0x13C, kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
 template <int CTRL>
 __device__ __forceinline__ int dppMove(int x) {
   return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true);
@@ -924,6 +925,10 @@ template <class T>
 __device__ __forceinline__ T fromWest(T x) { return dppMove<kDppWaveRor1>(x); }
 template <class T>
 __device__ __forceinline__ T fromEast(T x) { return dppMove<kDppWaveRol1>(x); }
+template <class T>
+__device__ __forceinline__ T westOrZero(T x) { return dppMove<kDppWaveShr1>(x); }
+template <class T>
+__device__ __forceinline__ T eastOrZero(T x) { return dppMove<kDppWaveShl1>(x); }
 
 // ColumnForcing for k_fusedW: the increments of the NS steps sit in a small
 // LDS table of the wave ([NS][CPT], written once by the wave's first CPT
@@ -1255,7 +1260,8 @@ __global__ void __launch_bounds__(256) k_fusedW(StepArgsN<T, NS> aa) {
 // 4.0, M = 8 11.2 -> 6.9; 509 x 2051 M = 1 14.9 -> 5.8.
 // Every value is the one-step kernel's expression in its order. Where it
 // clamps a neighbour at the mesh's edge (a merged coefficient beside a zero
-// one), the merged coefficient moves to the neighbour that exists.
+// one), the merged coefficient moves to the neighbour that exists; the other
+// one is zero, never another lane's value (which may not be finite).
 template <class T>
 struct TileArgs {
   const T* vIn;
@@ -1415,7 +1421,7 @@ __global__ void __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV
       for (int r = RT - 1; r >= 0; --r)
 #pragma unroll
         for (int k = 0; k < CPT; ++k) {
-          const T W = fromWest(st[r][k]);
+          const T W = westOrZero(st[r][k]);
           T sum = c[r][0] * sr[r][k] + c[r][1] * (r ? sr[r ? r - 1 : 0][k] : below[k]);
           sum = sum + c[r][2] * W;
           sum = sum + c[r][3] * st[r][k];
@@ -1469,7 +1475,7 @@ __global__ void __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(WV
         for (int k = 0; k < CPT; ++k) {
           const T vUp = r + 1 < RT ? v[r + 1 < RT ? r + 1 : 0][k] : above[k];
           sr[r][k] = sr[r][k] + a.dt * (c[r][4] * vUp + c[r][5] * v[r][k]);
-          const T vE = fromEast(v[r][k]);
+          const T vE = eastOrZero(v[r][k]);
           st[r][k] = st[r][k] + a.dt * (c[r][6] * v[r][k] + c[r][7] * vE);
         }
 #pragma unroll
