@@ -564,6 +564,13 @@ int shaw_debug_mfma(int kind, const double* a, const double* b, double* d);
  * w[n] eigenvalues (unordered), v row-major [n x n] with eigenvectors in its
  * columns. CPU only. No reference counterpart.                             */
 int shaw_debug_symeig(int n, const double* a, double* w, double* v);
+/* How shaw_rom_create lays an engine out on a device of `cus` CUs (0: one
+ * without cooperative launches): the modes that both dofs are padded to where
+ * the operators stay on the CU, 0 where they are streamed at their own sizes; the
+ * workgroups that share columns (1: none do) and, FP64, their sets of four
+ * columns. CPU only. No reference counterpart.                               */
+int shaw_debug_rom_shape(int precision, uint64_t kv, uint64_t ks, uint64_t max_cols, int cus, uint32_t* modes,
+                         uint32_t* split, uint32_t* sets);
 /* How often a wave of workgroups that share ROM columns looks in vain before it
  * gives up: at the launch's start, for the others to come (its columns then run
  * unshared, with the same results), and within the launch, for a value of

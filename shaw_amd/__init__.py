@@ -146,6 +146,7 @@ def lib():
         "shaw_pod_basis": (i32, [vp, u64, u64, u64, vp, vp]),
         "shaw_pod_basis_upto": (i32, [vp, u64, u64, u64, vp, vp, P(u64)]),
         "shaw_reconstruct": (i32, [vp, u64, u64, vp, u64, vp]),
+        "shaw_debug_rom_shape": (i32, [i32, u64, u64, u64, i32] + [P(C.c_uint32)] * 3),
         "shaw_debug_rom_waits": (i32, [vp, C.c_uint32, C.c_uint32]),
         "shaw_debug_copy": (i32, [u64, i32, P(dbl)]),
         "shaw_debug_symeig": (i32, [i32, vp, vp, vp]),
@@ -789,6 +790,14 @@ def rom_run(ar_v, ar_s, B, ftab, dt, nsteps, C=None, seis_freq=0, precision=ROM_
             seis[j] = y
     rom.close()
     return {"seismogram": seis if (R and T) else None, "qv": qv, "qs": qs}
+
+
+def debug_rom_shape(precision, kv: int, ks: int, max_cols: int, cus: int = 256):
+    """(padded modes, workgroups that share columns, sets of four) of an engine
+    (see include/shaw_amd.h)."""
+    v = [C.c_uint32() for _ in range(3)]
+    _check(lib().shaw_debug_rom_shape(precision, kv, ks, max_cols, cus, *[C.byref(x) for x in v]))
+    return tuple(x.value for x in v)
 
 
 def debug_rom_waits(rom: Rom, meet_tries: int, word_tries: int) -> None:

@@ -1779,6 +1779,17 @@ int shaw_debug_symeig(int n, const double* a, double* w, double* v) {
   });
 }
 
+int shaw_debug_rom_shape(int precision, uint64_t kv, uint64_t ks, uint64_t max_cols, int cus, uint32_t* modes,
+                         uint32_t* split, uint32_t* sets) {
+  return guarded([&] {
+    SHAW_REQUIRE(kv > 0 && ks > 0 && kv <= 512 && ks <= 512 && max_cols > 0 && modes && split && sets, SHAW_ERR_ARG,
+                 "bad argument");
+    const int parts = precision == SHAW_ROM_FP64 ? 0 : precision == SHAW_ROM_BF16X3 ? 2 : 3;
+    *modes = shaw::residentModes(parts, kv, ks, max_cols, cus);
+    *split = shaw::residentSplit(parts, *modes, (max_cols + shaw::kTileCols - 1) / shaw::kTileCols, cus, *sets);
+  });
+}
+
 int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, uint32_t word_tries) {
   return guarded([&] {
     SHAW_REQUIRE(h, SHAW_ERR_ARG, "null handle");

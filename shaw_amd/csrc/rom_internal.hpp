@@ -62,7 +62,8 @@ void gemmNN(const double* X, uint64_t n, uint32_t kin, const double* W, uint32_t
 // k_rom_steps* run it. Such an engine has a.Kvp = a.Ksp = that size and runs
 // launchRomResident (BF16, rom_resident.hip) or launchRomF64 (FP64, rom_f64.hip;
 // romF64Fits says whether that is the faster kernel for the active tiles of 16
-// columns, k_rom_steps taking the same operators with the same results).
+// columns, k_rom_steps taking the same operators with the same results). 0 also
+// where the dofs are so unequal that the square product costs more than it saves.
 struct RomArgs;
 uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int cus);
 // How many workgroups share a tile of 16 columns (BF16) or sets of four (FP64),

@@ -487,23 +487,35 @@ uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus, uint3
 }
 uint64_t residentExchange(uint32_t modes, uint64_t tiles) { return tiles * kXbufs * 2 * 8 * modes; }
 
+// FP64, padded dofs lo <= hi: up to how many rounds of workgroups of four columns
+// (64 tiles of 16 columns each, all CUs) the square product in k_rom_f64 is
+// faster than k_rom_steps, which computes the dofs as they are, 16 columns a
+// workgroup. A round against k_rom_steps, us: hi = 128: 1.6 against 3.7 (lo = 64);
+// 192: 3.8 against 5.0 (64), 8.4 (128); 256: 7.1 against 6.0 (64), 10.2 (128),
+// 14.1 (192); 384 18 against 14.6 (64), 26.6 (128), 35.1 (320), of 320 modes 13.2
+// (64), 26.6 (192), 32.4 (320), and two rounds 35.4 against 38.2 (384 both); 512
+// 34 against 23.1 (64), 42.3 (128), of 448 modes 21.1 (64), 38.6 (128). Equal dofs
+// of up to 256 modes pad alike either way: romF64Fits chooses for each launch.
+static uint64_t squareRounds(uint32_t lo, uint32_t hi) {
+  if (lo == hi && hi <= 256) return ~0ull;
+  if (hi == 128) return 2;
+  if (lo == 64) return hi == 192 ? 1 : 0;
+  return hi == 192 || (lo == 384 && hi == 384) ? 2 : 1;
+}
+
 uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int cus) {
-  const uint64_t k = kv > ks ? kv : ks;
-  // FP64 pads both dofs alike where k_rom_f64 runs them whatever the load, or
-  // where that costs k_rom_steps nothing
-  if (parts == 0 && cols > 2048 && k > 128 && (kv + 63) / 64 != (ks + 63) / 64) return 0;
-  if (k <= 256) return (uint32_t)((k + 63) / 64 * 64);
-  const uint32_t modes = k <= 384 ? 384 : 512;
-  // BF16: one workgroup a tile streams nearly all of the operators, and a square
-  // pad of unequal dofs would add to it
-  if (parts) {
-    uint32_t sets;
-    const bool shared = residentSplit(parts, modes, (cols + kTileCols - 1) / kTileCols, cus, sets) > 1;
-    return shared || (kv + 127) / 128 == (ks + 127) / 128 ? modes : 0;
-  }
-  // FP64: K = 384, 2048 columns: 35.4 us a step against 38.2; K = 512 1024
-  // columns 34.5 against 65.6, 2048 67.1 against 65.5
-  return cols <= (k <= 384 ? 2048 : 1024) ? modes : 0;
+  const uint64_t k = kv > ks ? kv : ks, tiles = (cols + kTileCols - 1) / kTileCols;
+  const uint32_t modes = k <= 256 ? (uint32_t)((k + 63) / 64 * 64) : k <= 384 ? 384 : 512;
+  uint32_t sets;
+  const bool shared = residentSplit(parts, modes, tiles, cus, sets) > 1;
+  const uint32_t lo = (uint32_t)(((kv < ks ? kv : ks) + 63) / 64 * 64), hi = (uint32_t)((k + 63) / 64 * 64);
+  // BF16 above 256 modes: one workgroup a tile streams nearly all of the
+  // operators, and a square pad of unequal dofs would add to it; shared tiles of
+  // 512 modes nearly fill the chip from 57 on (BF16x3 960 columns 11.5 us a step,
+  // of dofs of 512 and 128 modes 11.4 in one workgroup a tile; 896 columns 10.3)
+  if (parts == 2 && modes == 512 && lo <= 128 && tiles > 56) return 0;
+  if (parts) return k <= 256 || shared || (kv + 127) / 128 == (ks + 127) / 128 ? modes : 0;
+  return shared || (tiles + 63) / 64 <= squareRounds(lo, hi) ? modes : 0;
 }
 
 bool launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream) {
