@@ -1081,11 +1081,7 @@ struct shaw_rom {
     if (unchecked) (void)repeatShared(idle());
     const dim3 grid((unsigned)(maxCols / kTileCols));
     const size_t lds = ldsBytes();
-    // a cooperative launch and its first meeting cost about what three steps
-    // save (1280 columns of K = 384 BF16x3, launches in a row: 4 steps 56 us
-    // against 57, 2 steps 48 against 37), about what nine do at 256 modes FP64 (4
-    // steps 41 us against 34, 16 steps 87 against 110)
-    const bool shared = split > 1 && nsteps >= (precision == SHAW_ROM_FP64 && resident == 256 ? 10 : 4);
+    const bool shared = split > 1 && nsteps >= shareFrom(parts(), kv, ks, resident, split);
     if (resident && precision != SHAW_ROM_FP64) unchecked = launchRomResident(parts(), a, shared ? split : 1, stream);
     else if (shared && launchRomF64Shared(a, sets, stream)) unchecked = true;
     else if (resident && romF64Fits(resident, activeTiles())) launchRomF64(a, stream);

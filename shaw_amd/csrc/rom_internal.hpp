@@ -73,6 +73,8 @@ uint32_t residentModes(int parts, uint64_t kv, uint64_t ks, uint64_t cols, int c
 // (launchCooperative). Groups that do not meet in a shared launch are left as
 // they were and run in an unshared one of the same arguments with a.repeat = sets.
 uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus, uint32_t& sets);
+// the steps of a launch from which they share
+uint64_t shareFrom(int parts, uint64_t kv, uint64_t ks, uint32_t modes, uint32_t split);
 uint64_t residentExchange(uint32_t modes, uint64_t tiles);
 bool launchRomResident(int parts, const RomArgs& a, uint32_t split, hipStream_t stream);
 bool romF64Fits(uint32_t modes, uint64_t activeTiles);

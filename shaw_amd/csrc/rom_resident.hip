@@ -485,6 +485,20 @@ uint32_t residentSplit(int parts, uint32_t modes, uint64_t tiles, int cus, uint3
     if (fits(tiles, split)) return split;
   return 1;
 }
+// A cooperative launch and its first meeting cost about what three unshared steps
+// do (1280 columns of K = 384 BF16x3, launches in a row: 4 steps 59 us against 57,
+// 2 steps 48 against 37), about what nine do at 256 modes FP64 (4 steps 41 us
+// against 34, 16 steps 87 against 110). Unshared steps of dofs so unequal that the
+// square pad costs more than it saves are dearer (64 columns, FP64 512 and 64
+// modes: 28.9 us each and a shared launch of one 41; 384: 14.9 and 39 of two; 256:
+// 6.2 and 43 of four; BF16x4 512 and 64: 21 and 43 of two, but with half as many
+// workgroups a tile on a fuller chip 27 and 76).
+uint64_t shareFrom(int parts, uint64_t kv, uint64_t ks, uint32_t modes, uint32_t split) {
+  const uint64_t lo = kv < ks ? kv : ks, hi = kv < ks ? ks : kv;
+  if (parts) return split == modes / 64 && (hi + 127) / 128 > (lo + 127) / 128 + 1 ? 2 : 4;
+  if (lo <= 64) return hi <= 256 ? 5 : hi <= 384 ? 2 : 1;
+  return hi <= 256 ? 10 : 4;
+}
 uint64_t residentExchange(uint32_t modes, uint64_t tiles) { return tiles * kXbufs * 2 * 8 * modes; }
 
 // FP64, padded dofs lo <= hi: up to how many rounds of workgroups of four columns
