@@ -571,12 +571,12 @@ int shaw_debug_symeig(int n, const double* a, double* w, double* v);
  * columns. CPU only. No reference counterpart.                               */
 int shaw_debug_rom_shape(int precision, uint64_t kv, uint64_t ks, uint64_t max_cols, int cus, uint32_t* modes,
                          uint32_t* split, uint32_t* sets);
-/* How often a wave of workgroups that share ROM columns looks in vain before it
- * gives up: at the launch's start, for the others to come (its columns then run
- * unshared, with the same results), and within the launch, for a value of
- * theirs (every later call on the engine that waits for it then fails with
- * SHAW_ERR_HIP). Both 2^24 by default. No reference counterpart.            */
-int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, uint32_t word_tries);
+/* The waits of workgroups that share ROM columns, for tests: how often a wave
+ * looks in vain for the others at a launch's start (2^24 by default; the columns
+ * then run unshared, with the same results), and whether it takes what is there
+ * of their values within the launch (every later call on the engine that waits
+ * for it then fails with SHAW_ERR_HIP). No reference counterpart.            */
+int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, int no_words);
 /* Time `reps` launches of a plain streaming copy kernel (k_copy) of `bytes`
  * bytes (read `bytes`, write `bytes`); used to calibrate the HBM traffic
  * counters and to state the achievable copy bandwidth. No reference

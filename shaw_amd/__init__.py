@@ -147,7 +147,7 @@ def lib():
         "shaw_pod_basis_upto": (i32, [vp, u64, u64, u64, vp, vp, P(u64)]),
         "shaw_reconstruct": (i32, [vp, u64, u64, vp, u64, vp]),
         "shaw_debug_rom_shape": (i32, [i32, u64, u64, u64, i32] + [P(C.c_uint32)] * 3),
-        "shaw_debug_rom_waits": (i32, [vp, C.c_uint32, C.c_uint32]),
+        "shaw_debug_rom_waits": (i32, [vp, C.c_uint32, i32]),
         "shaw_debug_copy": (i32, [u64, i32, P(dbl)]),
         "shaw_debug_symeig": (i32, [i32, vp, vp, vp]),
         "shaw_rom_time": (i32, [vp, u64, P(dbl)]),
@@ -800,9 +800,9 @@ def debug_rom_shape(precision, kv: int, ks: int, max_cols: int, cus: int = 256):
     return tuple(x.value for x in v)
 
 
-def debug_rom_waits(rom: Rom, meet_tries: int, word_tries: int) -> None:
-    """Bound the waits of workgroups that share columns (see include/shaw_amd.h)."""
-    _check(lib().shaw_debug_rom_waits(rom.handle, meet_tries, word_tries))
+def debug_rom_waits(rom: Rom, meet_tries: int = 1 << 24, no_words: bool = False) -> None:
+    """Shorten the waits of workgroups that share columns (see include/shaw_amd.h)."""
+    _check(lib().shaw_debug_rom_waits(rom.handle, meet_tries, no_words))
 
 
 def debug_mfma(kind: int, a, b) -> np.ndarray:

@@ -928,7 +928,7 @@ struct shaw_rom {
   uint32_t split = 1, sets = 1;  // workgroups that share columns there; FP64, the sets of four
   shaw::DevBuf<uint64_t> xbuf, meet;  // their exchange buffers and meeting words
   uint64_t* gaveUp = nullptr;         // pinned, [2]: RomArgs::gaveUp
-  uint32_t meetTries = shaw::kMaxTries, wordTries = shaw::kMaxTries;
+  uint32_t meetTries = shaw::kMaxTries, noWords = 0;
   uint64_t launches = 0;
   // the last shared launch, unchecked until it is known that every group met
   // or a repeating launch is on the stream
@@ -1076,7 +1076,7 @@ struct shaw_rom {
     a.budget = a.macro ? timeBudget : 0;
     a.tiles = (uint32_t)(maxCols / kTileCols);
     a.xbuf = xbuf.p; a.meet = meet.p; a.gaveUp = gaveUp;
-    a.meetTries = meetTries; a.wordTries = wordTries;
+    a.meetTries = meetTries; a.noWords = noWords;
     a.launch = ++launches;
     if (unchecked) (void)repeatShared(idle());
     const dim3 grid((unsigned)(maxCols / kTileCols));
@@ -1786,11 +1786,11 @@ int shaw_debug_rom_shape(int precision, uint64_t kv, uint64_t ks, uint64_t max_c
   });
 }
 
-int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, uint32_t word_tries) {
+int shaw_debug_rom_waits(shaw_rom_t h, uint32_t meet_tries, int no_words) {
   return guarded([&] {
     SHAW_REQUIRE(h, SHAW_ERR_ARG, "null handle");
     h->meetTries = meet_tries;
-    h->wordTries = word_tries;
+    h->noWords = no_words != 0;
   });
 }
 

@@ -48,14 +48,14 @@ struct RomArgs {
   uint32_t budget;
   // tiles of 16 columns; and where several workgroups share columns (SPLIT > 1):
   // exchange buffers, the groups' meeting words (joinGroup), the launch's number,
-  // from 1, how often a wave looks in vain before it gives up, and host memory
-  // that says so: [0] the last launch in which a group did not meet, [1] the last
-  // in which a word of an exchange never came
+  // from 1, how often a wave looks in vain for the others, whether it does not wait
+  // for their words at all (a test), and host memory: [0] the last launch in which
+  // a group did not meet, [1] the last in which a word of an exchange never came
   uint32_t tiles;
   uint64_t* xbuf;
   uint64_t* meet;
   uint64_t launch;
-  uint32_t meetTries, wordTries;
+  uint32_t meetTries, noWords;
   uint64_t* gaveUp;
   // sets > 0: a launch that repeats `launch` for the groups that did not meet in
   // it, of that many workgroups of an unshared launch each; the others return
@@ -74,13 +74,13 @@ constexpr int kWaves = 8;      // waves per ROM workgroup (16 at 9..16 row tiles
 
 // ------------------------------------------------------------ exchange
 // Workgroups that share a tile of columns exchange states through memory, in
-// device scope, 64 bits at a time. (They have met first: joinGroup.) A reader takes each word from memory until it
-// is not kEmpty (four bf16 NaNs, a double's NaN), so nothing is waited for but
-// the data. Exchanges of a tile take turns on three buffers. After exchange e
-// every wave has read e - 1, and its writer empties it; that is out (written)
-// before the writer's words of e + 1, and so before anyone who has them looks
-// there for exchange e + 2. (A fourth buffer, which leaves the emptying another
-// exchange, measured the same within 2 %.)
+// device scope, 64 bits at a time. (They have met first: joinGroup.) A reader
+// takes each word from memory until it is not kEmpty (four bf16 NaNs, a double's
+// NaN), so nothing is waited for but the data. Exchanges of a tile take turns on
+// three buffers. After exchange e every wave has read e - 1, and its writer
+// empties it; that is out (written) before the writer's words of e + 1, and so
+// before anyone who has them looks there for exchange e + 2. (A fourth buffer,
+// which leaves the emptying another exchange, measured the same within 2 %.)
 constexpr uint64_t kEmpty = ~0ull;
 constexpr int kXbufs = 3;
 constexpr int kMeetStride = 16;  // words from one group's meeting word to the next: a cache line each
@@ -97,7 +97,7 @@ __device__ __forceinline__ void written() { asm volatile("s_waitcnt vmcnt(0)" ::
 // met, so all run and every word comes. Should one not, lost is set, the wave
 // goes on with what it has and reportLost tells the host.)
 template <int N, int STRIDE>
-__device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, uint32_t maxTries, bool& lost) {
+__device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, bool& lost) {
   uint64_t v[N];
 #pragma unroll
   for (int i = 0; i < N; ++i) v[i] = kEmpty;
@@ -109,7 +109,7 @@ __device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, uin
 #pragma unroll
     for (int i = 0; i < N; ++i) missing |= v[i] == kEmpty;
     if (lost || __ballot(missing) == 0) break;
-    lost = tries >= maxTries;
+    lost = tries > kMaxTries;
   }
 #pragma unroll
   for (int i = 0; i < N; ++i) d[i * STRIDE] = v[i];
@@ -117,8 +117,14 @@ __device__ __forceinline__ void collectWords(const uint64_t* x, uint64_t* d, uin
 __device__ __forceinline__ void tellHost(uint64_t* word, uint64_t v) {
   __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-__device__ __forceinline__ void reportLost(const RomArgs& a, bool lost, int lane) {
-  if (lost && lane == 0) tellHost(a.gaveUp + 1, a.launch);
+// (The arguments are read again from the kernel's argument block: kept in registers
+// from the start they displaced others of the step loop.)
+__device__ __forceinline__ void reportLost(bool lost, int lane) {
+  if (!lost) return;
+  typedef const __attribute__((address_space(4))) RomArgs* Args;
+  Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  if (lane == 0) tellHost(a->gaveUp + 1, a->launch);
 }
 // A group's meeting word: launch number, kNotMet, waves that came. All `waves`
 // waves of a group meet in a launch or none of them does: a wave that looked in

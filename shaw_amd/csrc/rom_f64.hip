@@ -374,7 +374,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
   // exchanges of set u: half-steps 0 (q_v), 1 (q_s), 2, ... of the launch
   uint64_t* const xbuf = a.xbuf + (uint64_t)group * SETS * kXbufs * K * kCols;  // [set][buffer][K][4]
   int cur = 0, old = kXbufs - 1;  // buffers of this half-step and the one before
-  bool lost = false;
+  bool lost = a.noWords != 0;
   auto buffer = [&](int u, int x) { return xbuf + (u * kXbufs + x) * K * kCols; };
   auto empty = [&](int u, int x) {
 #pragma unroll
@@ -396,8 +396,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
     static_assert(K * kCols % (64 * WAVES) == 0, "whole rounds");
 #pragma unroll
     for (int u = 0; u < SETS; ++u)
-      collectWords<K * kCols / (64 * WAVES), 64 * WAVES>(buffer(u, cur) + tid, reinterpret_cast<uint64_t*>(X(u, dof)) + tid,
-                                                        a.wordTries, lost);
+      collectWords<K * kCols / (64 * WAVES), 64 * WAVES>(buffer(u, cur) + tid, reinterpret_cast<uint64_t*>(X(u, dof)) + tid, lost);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < SETS; ++u) empty(u, old);
@@ -483,7 +482,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
       a.qv[at0] = q[u][0][t];
       a.qs[at0] = q[u][1][t];
     }
-  reportLost(a, lost, lane);
+  reportLost(lost, lane);
   // (all workgroups of the columns have read the counters: they have met)
   if (part == 0 && tid < kCols * SETS) {
     const uint64_t h = a.horizon[slot0 + tid];

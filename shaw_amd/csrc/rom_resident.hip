@@ -230,7 +230,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   // its workgroups
   uint64_t* const xbuf = a.xbuf + (uint64_t)tile * kXbufs * 2 * 8 * K;  // [buffer][dof][8 K]
   int cur = 0, old = kXbufs - 1;  // buffers of this exchange and the one before
-  bool both = false, lost = false;    // the exchange before moved both dofs; a word never came
+  // the group did not meet; the exchange before moved both dofs; a word never came
+  bool missed = false, both = false, lost = a.noWords != 0;
   // place of this lane's rows of tile t among the words of a buffer's dof
   auto word = [&](int t) { return 2 * ((4 * (rt[t] / 2) + lane / 16) * kTileCols + col) + rt[t] % 2; };
   auto publish = [&](int dof, double (&q)[TPW][4]) {
@@ -254,7 +255,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
   auto collect = [&](int dof, int4v* S) {
     static_assert(8 * K % (64 * WAVES) == 0, "whole rounds");
     collectWords<8 * K / (64 * WAVES), 64 * WAVES>(xbuf + (cur * 2 + dof) * 8 * K + tid, reinterpret_cast<uint64_t*>(S) + tid,
-                                                   a.wordTries, lost);
+                                                   lost);
   };
   auto turn = [&] {
     old = cur;
@@ -265,7 +266,15 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       empty(x, 0);
       empty(x, 1);
     }
-    if (!joinGroup(a, tile, SPLIT * WAVES, lane)) return;  // nothing is changed: a repeating launch runs the tile
+    // not met: nothing is changed, a repeating launch runs the tile. (Eight waves
+    // without macro steps skip all steps instead of returning here, which spills
+    // two more registers: BF16x4 K = 384, 1024 columns 6.5 us a step against 7.0;
+    // the others are faster so: K = 512, 512 columns 6.0 against 6.7)
+    if (!joinGroup(a, tile, SPLIT * WAVES, lane)) {
+      if constexpr (WAVES < 8 || MACRO) return;
+      missed = true;
+      steps = mk2 = 0;
+    }
   }
   // the new split of a dof to every wave that reads it
   auto share = [&](int dof, double (&q)[TPW][4], int4v* S) {
@@ -424,7 +433,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
       a.qv[colQ + rt[t] * 16 + rowBf16(lane, r)] = qv[t][r];
       a.qs[colQ + rt[t] * 16 + rowBf16(lane, r)] = qs[t][r];
     }
-  if constexpr (SPLIT > 1) reportLost(a, lost, lane);
+  if (SPLIT > 1 && missed) return;  // (the states are as they were read)
+  if constexpr (SPLIT > 1) reportLost(lost, lane);
   // (no workgroup of the tile is still to read its counters or states: a tile
   // with steps has had an exchange, one without writes what it read)
   if (part == 0 && tid < kTileCols) {

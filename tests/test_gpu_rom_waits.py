@@ -1,8 +1,8 @@
 """Engines whose columns are shared among workgroups: waits that end without the
 others. Groups that do not meet at a launch's start run unshared and give the
 same values bit for bit, with the launches enqueued in a row or waited for one
-by one; a value that never comes within a launch is an error, not a result. The
-bounds are set to nothing looked for in vain; every kernel ends normally."""
+by one; a value that does not come within a launch is an error, not a result. The
+waits are set to nothing looked for in vain; every kernel ends normally."""
 import numpy as np
 import pytest
 
@@ -44,7 +44,7 @@ def test_groups_that_do_not_meet_run_unshared(kv, ks, m, precision, macro, budge
         rom, slots = engine(kv, ks, m, precision, macro, budget)
         for j, n in enumerate((20, 60, 2, 90, 30, 98)):
             if tries is not None:  # by turns: nothing waited for, ordinary launches
-                shaw_amd.debug_rom_waits(rom, tries if j % 3 != 1 else 1 << 24, 1 << 24)
+                shaw_amd.debug_rom_waits(rom, tries if j % 3 != 1 else 1 << 24)
             rom.advance(n)
             if waited:
                 rom.sync()
@@ -62,7 +62,7 @@ def test_groups_that_do_not_meet_run_unshared(kv, ks, m, precision, macro, budge
 def test_a_value_that_never_comes_is_an_error(kv, ks, m, precision):
     print(f"[gpu] ROM exchange lost kv={kv} M={m} precision={precision}", flush=True)
     rom, slots = engine(kv, ks, m, precision, 0, 0)
-    shaw_amd.debug_rom_waits(rom, 1 << 24, 0)
+    shaw_amd.debug_rom_waits(rom, no_words=True)
     rom.advance(100)
     with pytest.raises(shaw_amd.ShawError, match="lost each other"):
         rom.sync()
