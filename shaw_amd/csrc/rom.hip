@@ -1071,6 +1071,8 @@ struct shaw_rom {
     a.Kvp = kvp; a.Ksp = ksp; a.Rp = rp; a.R = (uint32_t)R;
     a.maxSteps = maxSteps; a.Tcap = maxSamples; a.nsteps = nsteps; a.dt = dt;
     a.gvv = gvv.p; a.gvs = gvs.p; a.gsv = gsv.p; a.gss = gss.p;
+    a.groupsV = (uint32_t)(kv + 63) / 64 * 2;
+    a.groupsS = (uint32_t)(ks + 63) / 64 * 2;
     a.quiet = quiet.p;
     a.macro = precision == SHAW_ROM_FP64 ? 0 : macro;
     a.budget = a.macro ? timeBudget : 0;

@@ -40,6 +40,7 @@ struct RomArgs {
   // one-step matrix of [q_v; q_s]: G_vv [Kvp x Kvp], G_vs [Kvp x Ksp], G_sv,
   // G_ss, packed as the operators; m = 0 turns them off
   const void *gvv, *gvs, *gsv, *gss;
+  uint32_t groupsV, groupsS;  // the dofs' k-groups of 32 modes that are not all padding, even
   const uint32_t* quiet;  // [slot] first step from which the column's forcing is negligible
   uint32_t macro;
   // time budget (macro steps on): 0, nsteps steps for every tile; w > 0, the

@@ -358,13 +358,31 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
     if constexpr (MACRO) {
       if (seg == 0 && mk2) {
         // macro steps: the blocks of G stream from L2 through a two-deep
-        // ring, which starts on the next block while one ends
+        // ring, which starts on the next block while one ends. At 256 modes groups
+        // that are all padding are left out: unequal dofs pad alike (256 and 128
+        // modes, 1024 columns: BF16x3 8.1 -> 6.3 us a macro step, BF16x4 11.4 ->
+        // 9.1; kernels of the dofs' own sizes take 6.6 and 9.1). In a loop, which
+        // costs equal dofs 2 %; smaller and shared ones are faster without
         const bool act = s0 + mk < hz;
         Item mring[2][TPW];
-        auto stream = [&](auto zero, const char* G, const char* next, const int4v* X) {
+        auto stream = [&](auto zero, const char* G, uint32_t groups, const char* next, const int4v* X) {
           if constexpr (decltype(zero)::value)
 #pragma unroll
             for (int t = 0; t < TPW; ++t) acc[t] = Acc{0, 0, 0, 0};
+          if (KG == 8 && groups < KG) {
+#pragma nounroll
+            for (uint32_t g = 0; g < groups; g += 2) {
+              const char* src = g + 2 < groups ? G + (size_t)(g + 2) * 64 * sizeof(Item) : next;
+#pragma unroll
+              for (int q = 0; q < 2; ++q) {
+                groupProducts<PARTS, TPW>(mring[q], (int)g + q, X, lo, lane, acc);
+#pragma unroll
+                for (int t = 0; t < TPW; ++t) mring[q][t] = at(src, t, q);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+            }
+            return;
+          }
 #pragma unroll
           for (int g = 0; g < KG; ++g) {
             groupProducts<PARTS, TPW>(mring[g % 2], g, X, lo, lane, acc);
@@ -380,15 +398,15 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_resident(RomArgs a) {
         __syncthreads();  // both splits are in LDS
         for (uint32_t it = 0; it < mk2; ++it) {
           const char *gvv = opaque(a.gvv), *gvs = opaque(a.gvs), *gsv = opaque(a.gsv), *gss = opaque(a.gss);
-          stream(std::true_type{}, gvv, gvs, Sv);
-          stream(std::false_type{}, gvs, gsv, Ss);
+          stream(std::true_type{}, gvv, a.groupsV, gvs, Sv);
+          stream(std::false_type{}, gvs, a.groupsS, gsv, Ss);
           if (act)
 #pragma unroll
             for (int t = 0; t < TPW; ++t)
 #pragma unroll
               for (int r = 0; r < 4; ++r) qv[t][r] = qv[t][r] + a.dt * (double)acc[t][r];
-          stream(std::true_type{}, gsv, gss, Sv);
-          stream(std::false_type{}, gss, gvv, Ss);
+          stream(std::true_type{}, gsv, a.groupsV, gss, Sv);
+          stream(std::false_type{}, gss, a.groupsS, gvv, Ss);
           if (act)
 #pragma unroll
             for (int t = 0; t < TPW; ++t)
