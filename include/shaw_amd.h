@@ -170,11 +170,12 @@ typedef struct {
                            falls back to fewer steps per launch; the last steps of a
                            run (up to two 7-step launches on one-wavefront strips)
                            go in as few, evenly split launches
-                           (with every tile option at its default the launches are
-                           planned from the grid instead, window tiles of 6 to 16
-                           steps or strips of 4 to 7: shaw_fom_launch_shape; same
-                           results bit for bit)                                        */
-  int graph_steps;      /* 0 = default (64, rounded up to an even number of launches);
+                           (with every tile option at its default and graph_steps <= 0
+                           the launches are planned from the grid instead, window tiles
+                           of 6 to 16 steps or strips of 4 to 7: shaw_fom_launch_shape;
+                           same results bit for bit)                                   */
+  int graph_steps;      /* 0 = default: 64, rounded up to an even number of launches,
+                           where a tile option is given; planned launches run eagerly;
                            < 0: no graphs. Fused kernel without snapshots: whole chunks
                            of this many steps replay one captured HIP graph (kernels
                            read their step from a device counter); a multiple of

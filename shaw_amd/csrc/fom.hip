@@ -1681,7 +1681,7 @@ class FomEngine final : public shaw_fom {
                    "3 or 4 steps per launch need a column block of fewer than 2^32 stress values");
       setStrips();
       const bool asked = o.cols_per_thread > 0 || o.strip > 0 || o.segment > 0 || o.prefetch_rows > 0 ||
-                         o.steps_per_launch > 0 || o.col_block > 0;
+                         o.steps_per_launch > 0 || o.col_block > 0 || o.graph_steps > 0;  // (planned launches run eagerly)
       if (!asked) plan();
     }
     SHAW_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
