@@ -258,11 +258,12 @@ int shaw_fom_config(shaw_fom_t h, int* kernel, int* cols_per_thread, int* strip,
  * explicit options, the autotuner and graphs start from (any may be null). */
 int shaw_fom_launch_shape(shaw_fom_t h, uint64_t nsteps, uint64_t* launches, int* steps, int* segment);
 /* Tile autotuner of the fused kernel (no counterpart in the reference, whose
- * launch shapes are fixed Kokkos policies): times every valid (columns per
- * thread, strip, segment, rows prefetched, steps per launch) for
- * trial_steps launches on the
- * current state, keeps the fastest (read it back with shaw_fom_config) and
- * restores the state. Needs the forcing table to cover the next step.     */
+ * launch shapes are fixed Kokkos policies): times the planned launches of
+ * a handle of default options and every valid (columns per thread, strip,
+ * segment, rows prefetched, steps per launch) for trial_steps launches on the
+ * current state, keeps the fastest (read it back with shaw_fom_launch_shape and
+ * shaw_fom_config) and restores the state. Needs the forcing table to cover the
+ * next two steps.                                                          */
 int shaw_fom_autotune(shaw_fom_t h, uint64_t trial_steps, double* best_ms_per_step);
 /* POD basis of the device snapshot buffer of `dof` (all configured columns,
  * all samples: LayoutLeft [n x (T * ncols)]) without a host round trip, as

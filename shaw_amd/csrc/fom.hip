@@ -2181,11 +2181,12 @@ class FomEngine final : public shaw_fom {
     hipLaunchKernelGGL((k_stress<T, CPT>), gs, dim3(256), 0, stream_, a);
     snapshot(1, a.sOut);
   }
-  // Tile autotuner of the fused kernel: every valid (columns per thread,
-  // strip, segment, rows prefetched), and k_tile where the defaults run it, is timed for `trialSteps` steps on the
-  // current state (after one untimed step), the fastest is kept, and the
-  // state is restored: the trials do not advance the run, record receivers
-  // or take snapshots.
+  // Tile autotuner of the fused kernel: the planned launches (window tiles and
+  // strips, where the defaults run them) and every valid (columns per thread,
+  // strip, segment, rows prefetched, steps) are timed for `trialSteps` launches
+  // on the current state (after one untimed launch), the fastest is kept, and the
+  // state is restored: the trials do not advance the run, record receivers or
+  // take snapshots. Planned launches are cut to the steps the forcing table has left.
   void autotune(uint64_t trialSteps, double* bestMs) override {
     SHAW_REQUIRE(kernel_ == SHAW_KERNEL_FUSED, SHAW_ERR_STATE, "the autotuner tunes the fused kernel");
     SHAW_REQUIRE(trialSteps >= 1 && trialSteps <= 1000, SHAW_ERR_ARG, "trial steps must be in 1..1000");
@@ -2199,63 +2200,83 @@ class FomEngine final : public shaw_fom {
     SHAW_HIP(hipMemcpy(sv.p, v_[cur0].p, sv.n * sizeof(T), hipMemcpyDeviceToDevice));
     SHAW_HIP(hipMemcpy(ss.p, s_[cur0].p, ss.n * sizeof(T), hipMemcpyDeviceToDevice));
     struct Cfg { int cpt; uint32_t P, SEG; int pf, spl; };
-    Cfg best{cpt_, P_, SEG_, pf_, spl_};
-    double bestT = 1e300, tileT = 1e300;
-    packSteps_ = 0;  // the trials' shapes rule from here on
-    if (tile_.steps && step_ + tile_.steps <= ftabSteps_ && step_ + tile_.steps < (1ull << 32)) {
-      launchTile(tile_.steps, true);
-      SHAW_HIP(hipEventRecord(ev0_, stream_));
-      for (uint64_t k = 0; k < trialSteps; ++k) launchTile(tile_.steps, true);
-      SHAW_HIP(hipEventRecord(ev1_, stream_));
-      SHAW_HIP(hipEventSynchronize(ev1_));
-      float ms = 0;
-      SHAW_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
-      tileT = ms / (double)(trialSteps * tile_.steps);
-    }
+    const Cfg given{cpt_, P_, SEG_, pf_, spl_};
+    const Tile tile = tile_;
+    const int pack = packSteps_;
     auto apply = [&](const Cfg& c) {
       cpt_ = c.cpt; P_ = c.P; SEG_ = c.SEG; pf_ = c.pf; spl_ = c.spl;
       graphSteps_ = graphStepsFor(spl_);
       setStrips();
     };
-    for (int cpt : {1, 2, 4, 8}) {
-      if (MC_ % cpt) continue;
-      const uint32_t tpp = MC_ / cpt;
-      for (uint32_t P : {8u, 16u, 32u, 64u, 128u, 256u}) {
-        if (P * tpp > 512 || P * tpp < 64) continue;
-        for (uint32_t SEG : {2u, 4u, 8u, 16u, 32u, 64u, 128u, 256u})
-          for (int pf : {1, 2})
-            for (int spl = 1; spl <= kMaxSpl; ++spl) {
-              // the multi-step kernels load one row ahead, k_fusedW one or two
-              if (spl >= 2 && pf == 2 && !(spl >= 3 && spl <= 4 && waveStrip(cpt, P))) continue;
-              if (spl >= 5 && !waveStrip(cpt, P)) continue;  // 5 to 7 steps: one-wavefront strips only
-              if (spl >= 2 && P < 2u * spl) continue;
-              if (step_ + spl > ftabSteps_) continue;  // a trial reads the forcing of its steps
-              if (graphStepsFor(spl) % (2 * spl)) continue;  // a requested graph length must fit
-              if (ldsBytes(cpt, P, spl) > kMaxLds) continue;
-              if (spl >= 3 && !fits32()) continue;
-              // short segments only where the grid is too small to fill the chip
-              if (SEG < 16 && launchWaves(cpt, P, SEG, spl) > 16 * kMinWaves) continue;
-              const Cfg c{cpt, P, SEG, pf, spl};
-              apply(c);
-              trialLaunch();
-              SHAW_HIP(hipEventRecord(ev0_, stream_));
-              for (uint64_t k = 0; k < trialSteps; ++k) trialLaunch();
-              SHAW_HIP(hipEventRecord(ev1_, stream_));
-              SHAW_HIP(hipEventSynchronize(ev1_));
-              float ms = 0;
-              SHAW_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
-              const double perStep = ms / (double)(trialSteps * spl);
-              if (perStep < bestT) { bestT = perStep; best = c; }
-            }
+    // ms per step of launches of `steps` steps
+    auto timed = [&](uint64_t steps, auto launch) {
+      launch();
+      SHAW_HIP(hipEventRecord(ev0_, stream_));
+      for (uint64_t k = 0; k < trialSteps; ++k) launch();
+      SHAW_HIP(hipEventRecord(ev1_, stream_));
+      SHAW_HIP(hipEventSynchronize(ev1_));
+      float ms = 0;
+      SHAW_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
+      return ms / (double)(trialSteps * steps);
+    };
+    Cfg best = given;
+    double bestT = 1e300, tileT = 1e300, packT = 1e300;
+    try {
+      const uint64_t left = ftabSteps_ - step_;
+      if (tile.steps && step_ + tile.steps < (1ull << 32)) {
+        const uint64_t steps = std::min<uint64_t>(tile.steps, left);
+        tileT = timed(steps, [&] { launchTile(steps, true); });
       }
+      if (pack) {
+        const uint64_t steps = std::min<uint64_t>(pack, left);
+        packT = timed(steps, [&] { trialLaunch((int)steps); });
+      }
+      packSteps_ = 0;  // the trials' shapes rule from here on
+      for (int cpt : {1, 2, 4, 8}) {
+        if (MC_ % cpt) continue;
+        const uint32_t tpp = MC_ / cpt;
+        for (uint32_t P : {8u, 16u, 32u, 64u, 128u, 256u}) {
+          if (P * tpp > 512 || P * tpp < 64) continue;
+          for (uint32_t SEG : {2u, 4u, 8u, 16u, 32u, 64u, 128u, 256u})
+            for (int pf : {1, 2})
+              for (int spl = 1; spl <= kMaxSpl; ++spl) {
+                // the multi-step kernels load one row ahead, k_fusedW one or two
+                if (spl >= 2 && pf == 2 && !(spl >= 3 && spl <= 4 && waveStrip(cpt, P))) continue;
+                if (spl >= 5 && !waveStrip(cpt, P)) continue;  // 5 to 7 steps: one-wavefront strips only
+                if (spl >= 2 && P < 2u * spl) continue;
+                if (step_ + spl > ftabSteps_) continue;  // a trial reads the forcing of its steps
+                if (graphStepsFor(spl) % (2 * spl)) continue;  // a requested graph length must fit
+                if (ldsBytes(cpt, P, spl) > kMaxLds) continue;
+                if (spl >= 3 && !fits32()) continue;
+                // short segments only where the grid is too small to fill the chip
+                if (SEG < 16 && launchWaves(cpt, P, SEG, spl) > 16 * kMinWaves) continue;
+                const Cfg c{cpt, P, SEG, pf, spl};
+                apply(c);
+                const double t = timed(spl, [&] { trialLaunch(spl_); });
+                if (t < bestT) { bestT = t; best = c; }
+              }
+        }
+      }
+    } catch (...) {
+      apply(given);
+      packSteps_ = pack;
+      tile_ = tile;
+      cur_ = cur0;
+      throw;
     }
-    apply(best);
-    if (tileT < bestT) bestT = tileT;
-    else tile_.steps = 0;
+    if (tileT < bestT && tileT < packT) {
+      packSteps_ = pack;
+      apply(given);
+    } else {
+      tile_.steps = 0;
+      const bool planned = packT < bestT;
+      packSteps_ = planned ? pack : 0;
+      apply(planned ? given : best);
+    }
     SHAW_HIP(hipMemcpy(v_[cur0].p, sv.p, sv.n * sizeof(T), hipMemcpyDeviceToDevice));
     SHAW_HIP(hipMemcpy(s_[cur0].p, ss.p, ss.n * sizeof(T), hipMemcpyDeviceToDevice));
     cur_ = cur0;
-    if (bestMs) *bestMs = bestT;
+    if (bestMs) *bestMs = std::min(bestT, std::min(tileT, packT));
   }
   // graph chunk for `spl` steps per launch: the requested length, or 64
   // rounded up to an even number of launches; 0 = no graphs
@@ -2305,31 +2326,22 @@ class FomEngine final : public shaw_fom {
     const uint64_t wavesPerBlock = ((uint64_t)P * (MC_ / cpt) + 63) / 64;
     return strips * segs * nb_ * wavesPerBlock;
   }
-  // one launch of the current shape (one step or a pair) that records
-  // nothing and does not advance the run
-  void trialLaunch() {
-    if (spl_ >= 3) {
-      switch (spl_) {
-        case 3: trialPackN<3>(); break;
-        case 4: trialPackN<4>(); break;
-        case 5: trialPackN<5>(); break;
-        case 6: trialPackN<6>(); break;
-        default: trialPackN<7>(); break;
-      }
-    } else if (spl_ == 2) {
-      StepArgs2<T> aa;
-      pairArgs(aa);
-      aa.s1.recv = aa.s2.recv = nullptr;
-      switch (cpt_) {
-        case 1: launchFused2<1>(aa, false); break;
-        case 2: launchFused2<2>(aa, false); break;
-        case 4: launchFused2<4>(aa, false); break;
-        default: launchFused2<8>(aa, false); break;
-      }
-      SHAW_HIP(hipGetLastError());
-    } else {
-      trialStep();
+  // one launch of ns steps that records nothing and does not advance the run
+  void trialLaunch(int ns) {
+    switch (ns) {
+      case 1: trialStep(); return;
+      case 2: break;
+      case 3: trialPackN<3>(); return;
+      case 4: trialPackN<4>(); return;
+      case 5: trialPackN<5>(); return;
+      case 6: trialPackN<6>(); return;
+      default: trialPackN<7>(); return;
     }
+    StepArgs2<T> aa;
+    pairArgs(aa);
+    aa.s1.recv = aa.s2.recv = nullptr;
+    dispatchPair(aa, false);
+    SHAW_HIP(hipGetLastError());
   }
   template <int NS>
   void trialPackN() {

@@ -38,3 +38,39 @@ def test_graph_steps_are_replayed(nr, nth, m):
         for x, y in zip(out[0], other):
             np.testing.assert_array_equal(x, y)
     assert np.abs(out[0][0]).max() > 0
+
+
+def test_autotune_keeps_window_tiles_near_the_tables_end():
+    """Fewer steps left than a window tile takes: it is timed at those."""
+    say("[gpu] autotune 21x51, 5 steps left")
+    fom = engine(21, 51, 1, 50)
+    fom.advance(45)
+    before = fom.state()
+    assert fom.launch_shape(5)["segment"] == 0
+    ms = fom.autotune(3)
+    assert ms > 0 and fom.launch_shape(5)["segment"] == 0
+    for x, y in zip(before, fom.state()):
+        np.testing.assert_array_equal(x, y)
+    fom.close()
+
+
+def test_autotune_is_not_slower_than_the_plan():
+    """509 x 2051, 15 columns: the planned 85-row segments run in one round of the
+    chip, the candidates' 64 rows in two and 128 rows with a third more work. What the
+    tuner keeps takes no longer than the plan (5 % for the spread of a timing)."""
+    say("[gpu] autotune 509x2051 M=15")
+    fom = engine(509, 2051, 15, 3000)
+    planned = fom.launch_shape(70)
+    assert planned["segment"] not in (0, 64, 128)
+
+    def ms():
+        fom.reset()
+        fom.advance(70)
+        return min(fom.time(140)[0] for _ in range(5))
+
+    before = ms()
+    fom.autotune(3)
+    after = ms()
+    say(f"  plan {planned} {before:.3f} ms, tuned {fom.launch_shape(70)} {after:.3f} ms")
+    assert after <= 1.05 * before
+    fom.close()
