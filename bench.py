@@ -551,10 +551,10 @@ def main() -> int:
     value = w.m * args.steps / (total_ms / 1000.0)
     log(f"{total_ms:.2f} ms for {args.steps} steps -> {ms_per_step:.4f} ms/step, {value:.0f} forcing-steps/s")
     kernel_bytes, model_bytes = fom.bytes_per_step()
-    bytes_per_launch = kernel_bytes * fom.config()["steps_per_launch"]  # whatever a launch's steps
     # the launches as planned: k steps and rows per segment
     shape = fom.launch_shape(ROOF_STEPS)
     spl = shape["steps_per_launch"]
+    bytes_per_launch = kernel_bytes * spl
     cfg = {**fom.config(), "steps_per_launch": spl, "segment": shape["segment"]}
     # the dominant kernel alone: whole launches, HIP events on the FOM stream
     roof_launches = ROOF_STEPS // spl

@@ -244,7 +244,9 @@ int shaw_fom_complexity(uint64_t nvp, uint64_t nsp, uint64_t nnz_vp, uint64_t nn
                         double* mem_mb, double* flops);
 /* Algorithmic HBM bytes of one leapfrog step of the selected kernel (the
  * state read and written once per launch, the coefficients read once per
- * launch, divided by the steps per launch), and the reference model
+ * launch, divided by the steps per launch of a long run, shaw_fom_launch_shape;
+ * of a grid that one window tile holds, which takes a run in one launch, by
+ * those of a larger grid's window), and the reference model
  * s*m*3*(nvp+nsp) + 8*(4*nvp + 2*nsp).                                    */
 int shaw_fom_bytes_per_step(shaw_fom_t h, double* kernel_bytes, double* model_bytes);
 /* Kernel configuration actually used: kernel, cols_per_thread, strip, segment,

@@ -2053,9 +2053,9 @@ class FomEngine final : public shaw_fom {
     const double coef = (4.0 * nVp_ + 2.0 * nSp_) * s;
     if (kernel) {
       // fused: read + write each state once; split: v (r+w) + s (r) / v (r) + s (r+w)
-      // (per step: a launch of the k-step kernel moves these bytes for k steps)
+      // (per step: a launch of k steps moves these bytes for k of them)
       const double passes = kernel_ == SHAW_KERNEL_FUSED ? 2.0 : 3.0;
-      *kernel = (s * cols * passes * (double)(nVp_ + nSp_) + coef) / (kernel_ == SHAW_KERNEL_FUSED ? spl_ : 1);
+      *kernel = (s * cols * passes * (double)(nVp_ + nSp_) + coef) / launchSteps();
     }
     if (model) *model = s * (double)M_ * 3.0 * (double)(nVp_ + nSp_) + 8.0 * (4.0 * nVp_ + 2.0 * nSp_);
   }
@@ -2112,9 +2112,13 @@ class FomEngine final : public shaw_fom {
     if (pf) *pf = pf_;
     if (spl) *spl = kernel_ == SHAW_KERNEL_FUSED ? spl_ : 1;
   }
+  // steps of a launch in the middle of a long run
+  uint32_t launchSteps() const {
+    return tile_.steps ? tile_.steps : packSteps_ ? packSteps_ : kernel_ == SHAW_KERNEL_FUSED ? spl_ : 1;
+  }
   // of an advance by nsteps without snapshots
   void launchShape(uint64_t nsteps, uint64_t* launches, int* steps, int* segment) const override {
-    const uint32_t top = tile_.steps ? tile_.steps : packSteps_ ? packSteps_ : kernel_ == SHAW_KERNEL_FUSED ? spl_ : 1;
+    const uint32_t top = launchSteps();
     const bool whole = tile_.steps && nth_ <= 64 && nr_ <= kTileWaves * tile_.rows;
     const uint64_t n = whole ? 1 : (nsteps + top - 1) / top;
     const uint64_t len = n ? (nsteps + n - 1) / n : 0;

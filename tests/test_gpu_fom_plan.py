@@ -74,3 +74,17 @@ def test_autotune_is_not_slower_than_the_plan():
     say(f"  plan {planned} {before:.3f} ms, tuned {fom.launch_shape(70)} {after:.3f} ms")
     assert after <= 1.05 * before
     fom.close()
+
+
+@pytest.mark.parametrize("nr,nth,m", [(200, 1000, 1), (200, 1000, 24)])
+@pytest.mark.parametrize("kw", [{}, dict(steps_per_launch=3), dict(kernel=shaw_amd.KERNEL_SPLIT)])
+def test_bytes_per_step_are_of_the_launches_that_run(nr, nth, m, kw):
+    say(f"[gpu] bytes per step {nr}x{nth} M={m} {kw}")
+    fom = engine(nr, nth, m, 10, **kw)
+    steps = fom.launch_shape(5040)["steps_per_launch"]  # a multiple of every planned length
+    nvp, nsp = nr * nth, (nr - 1) * nth + nr * (nth - 1)
+    passes = 3 if "kernel" in kw else 2
+    want = 8.0 * (m * passes * (nvp + nsp) + 4 * nvp + 2 * nsp) / steps
+    assert fom.bytes_per_step()[0] == pytest.approx(want, rel=1e-12)
+    assert kw or m > 1 or steps != fom.config()["steps_per_launch"]  # window tiles
+    fom.close()
