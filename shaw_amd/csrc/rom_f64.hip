@@ -496,7 +496,7 @@ void launchF64(const RomArgs& a, uint64_t cols, hipStream_t stream) {
   constexpr size_t lds = (size_t)2 * 16 * G * kCols * 8 + (size_t)2 * G * LL * 64 * 32;
   static_assert(lds <= 160 * 1024, "LDS of one CU");
   const auto kernel = k_rom_f64<G, WAVES, RR, LL, DR>;
-  (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  SHAW_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   hipLaunchKernelGGL(kernel, dim3((unsigned)(cols / kCols)), dim3(WAVES * 64), lds, stream, a);
 }
 
