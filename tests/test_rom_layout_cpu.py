@@ -4,6 +4,7 @@ equal dofs and few columns as before."""
 import pytest
 
 import shaw_amd
+from tests.test_gpu_rom_split import SIZES
 
 # kv, ks, columns, padded modes (0: the dofs keep their own sizes)
 FP64 = [(100, 64, 2048, 128), (100, 64, 2064, 0), (64, 100, 4096, 0), (128, 128, 4096, 128),
@@ -36,3 +37,14 @@ def test_bf16x3_pads(kv, ks, cols, modes):
     got, split, sets = shaw_amd.debug_rom_shape(shaw_amd.ROM_BF16X3, kv, ks, cols)
     assert got == modes
     assert (split > 1) == (0 < modes and cols <= {384: 1280, 512: 1024}[modes])
+
+
+@pytest.mark.parametrize("precision", [shaw_amd.ROM_BF16X3, shaw_amd.ROM_BF16X4])
+@pytest.mark.parametrize("kv,ks,m", SIZES)
+def test_few_bf16_columns_are_shared(kv, ks, m, precision):
+    """What the GPU tests of shared tiles compare is shared on one side only."""
+    modes, split, _ = shaw_amd.debug_rom_shape(precision, kv, ks, m)
+    most = modes // 64
+    assert modes == (384 if max(kv, ks) <= 384 else 512)
+    assert split == (most if (m + 15) // 16 <= {384: 40, 512: 32}[modes] else most // 2)
+    assert shaw_amd.debug_rom_shape(precision, kv, ks, 2048)[1] == 1
