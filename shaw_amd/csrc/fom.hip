@@ -1826,7 +1826,12 @@ class FomEngine final : public shaw_fom {
       if (snap_[d].ncols) SHAW_REQUIRE(last / snap_[d].every <= snap_[d].Tcap, SHAW_ERR_STATE, "snapshot buffer too small");
     uint64_t k = 0;
     if (tile_.steps && last < (1ull << 32)) {
-      while (k < nsteps) k += launchTile(nsteps - k);
+      while (k < nsteps) {
+        const uint64_t ns = tileSteps(nsteps - k);
+        if (ns < tile_.steps && !wholeTile() && marchShort_[ns]) launchMarch((int)ns);
+        else launchTile(ns);
+        k += ns;
+      }
       SHAW_HIP(hipGetLastError());
       return;
     }
@@ -1868,18 +1873,21 @@ class FomEngine final : public shaw_fom {
         else if (left <= 2 * top) ns = (int)((left + 1) / 2);      // two, balanced
       }
       while (ns > 1 && (k + ns > nsteps || packBlocked(ns))) --ns;
-      switch (ns) {
-        case 1: launchStep(); break;
-        case 2: launchPair(); break;
-        case 3: launchPackN<3>(); break;
-        case 4: launchPackN<4>(); break;
-        case 5: launchPackN<5>(); break;
-        case 6: launchPackN<6>(); break;
-        default: launchPackN<7>(); break;
-      }
+      launchMarch(ns);
       k += ns;
     }
     SHAW_HIP(hipGetLastError());
+  }
+  void launchMarch(int ns) {
+    switch (ns) {
+      case 1: launchStep(); break;
+      case 2: launchPair(); break;
+      case 3: launchPackN<3>(); break;
+      case 4: launchPackN<4>(); break;
+      case 5: launchPackN<5>(); break;
+      case 6: launchPackN<6>(); break;
+      default: launchPackN<7>(); break;
+    }
   }
   // the most steps one launch of the current shape takes: at six steps per
   // launch the wave kernel (one-wavefront strips, one row loaded ahead) also
@@ -2119,12 +2127,13 @@ class FomEngine final : public shaw_fom {
   // of an advance by nsteps without snapshots
   void launchShape(uint64_t nsteps, uint64_t* launches, int* steps, int* segment) const override {
     const uint32_t top = launchSteps();
-    const bool whole = tile_.steps && nth_ <= 64 && nr_ <= kTileWaves * tile_.rows;
+    const bool whole = tile_.steps && wholeTile();
     const uint64_t n = whole ? 1 : (nsteps + top - 1) / top;
     const uint64_t len = n ? (nsteps + n - 1) / n : 0;
     if (launches) *launches = n;
     if (steps) *steps = (int)len;
-    if (segment) *segment = tile_.steps ? 0 : packSteps_ && len <= (uint64_t)kMaxSpl && packSeg_[len] ? (int)packSeg_[len] : (int)SEG_;
+    const bool march = !tile_.steps || (!whole && len < tile_.steps && marchShort_[len]);
+    if (segment) *segment = !march ? 0 : packSteps_ && len <= (uint64_t)kMaxSpl && packSeg_[len] ? (int)packSeg_[len] : (int)SEG_;
   }
 
  private:
@@ -2513,7 +2522,11 @@ class FomEngine final : public shaw_fom {
   struct Tile {
     uint32_t rows = 4, steps = 0, cbPer = 1;
   } tile_;
-  static constexpr uint32_t kTileWaves = 12;
+  static constexpr uint32_t kTileWaves = 12, kTileSteps = 16;
+  // launches of fewer steps (advance by a few, snapshots): the window of each
+  // number of steps, or whether the marching kernels take it
+  Tile tileOf_[kTileSteps + 1];
+  bool marchShort_[kTileSteps + 1] = {};
   // windows of `size` cells over n, overlapping by `halo` on each inner side
   static uint32_t windows(uint64_t n, uint32_t size, uint32_t halo) {
     return n <= size ? 1 : (uint32_t)((n - 2 * halo + (size - 2 * halo) - 1) / (size - 2 * halo));
@@ -2528,12 +2541,45 @@ class FomEngine final : public shaw_fom {
   double tileCost(const Tile& t) const {
     const uint32_t rows = kTileWaves * t.rows;
     const bool whole = nth_ <= 64 && nr_ <= rows;
-    const uint32_t wg = windows(nth_, 64, t.steps) * windows(nr_, rows, t.steps) * ((nb_ + t.cbPer - 1) / t.cbPer);
     const double kb100 = rows * 64.0 * sizeof(T) / 1e5, steps = whole ? 200 : t.steps;
     const double step = 0.095 * t.rows * MC_ + 0.27;
     const double block = 4.26 * 3 * MC_ * kb100 + steps * step;
-    return 1.08 * (0.8 + ((wg + 255) / 256) * (3.2 * 8 * kb100 + std::min(t.cbPer, nb_) * block)) / steps;
+    return 1.08 * (0.8 + tileRounds(t) * (3.2 * 8 * kb100 + std::min(t.cbPer, nb_) * block)) / steps;
   }
+  uint32_t tileRounds(const Tile& t) const {
+    const uint32_t rows = kTileWaves * t.rows, groups = (nb_ + t.cbPer - 1) / t.cbPer;
+    return (windows(nth_, 64, t.steps) * windows(nr_, rows, t.steps) * groups + 255) / 256;
+  }
+  // Microseconds of a launch of up to five steps, where the loads of all windows
+  // coincide: their bytes against the last-level cache's rate, and the chain of a
+  // workgroup. Fitted to 474 launches of 1 to 6 steps on 42 grids, standard
+  // deviation 6 %.
+  double shortTileCost(const Tile& t) const {
+    const uint32_t rows = kTileWaves * t.rows;
+    const double kb100 = rows * 64.0 * sizeof(T) / 1e5, groups = (nb_ + t.cbPer - 1) / t.cbPer;
+    const double block = 2.98 * 3 * MC_ * kb100 + t.steps * (0.155 * t.rows * MC_ + 0.05);
+    const double chain = 4.1 + tileRounds(t) * (0.5 * 8 * kb100 + std::min(t.cbPer, nb_) * block);
+    const double cells = (double)windows(nth_, 64, t.steps) * windows(nr_, rows, t.steps) * rows * 64;
+    const double mb = (cells * (8 * groups + 3.0 * MC_ * nb_) + 3.0 * nVp_ * MC_ * nb_) * sizeof(T) / 1e6;
+    return both(chain, 0.1 + mb / 6.2, 2.25);
+  }
+  // and of the marching kernels' launch of n steps: one row after another, or
+  // bytes; up to three steps fitted to the same grids (5 to 7 %)
+  double shortMarchCost(int n) const {
+    if (n > 3) return marchCost(n, packSeg_[n]) * n;
+    const uint32_t halo = n == 1 ? 1 : 2 * n - 1, share = n == 3 ? waveGroup() : 1;
+    const uint64_t strips = (nth_ + (63 - halo)) / (64 - halo), segs = (nr_ + SEG_ - 1) / SEG_;
+    const double rows = std::min<uint64_t>(SEG_, nr_) + halo;
+    const double mb = ((double)strips * 64 * (nr_ + segs * halo) * nb_ * (3.0 * MC_ + 8.0 / share) + 3.0 * nVp_ * MC_ * nb_) *
+                      sizeof(T) / 1e6;
+    if (n == 1) return std::max(1.0 + 1.05 * rows, 3.0 + mb / 7.1);
+    const double fill = (double)(strips * segs * ((nb_ + share - 1) / share) * share) / (sizeof(T) == 8 ? 2048 : 4096);
+    const double lone = (n == 2 ? 1.05 : 1.2) * (MC_ == 1 ? 0.8 : 1.0), full = n == 2 ? 1.09 : 1.17;
+    const double row = std::max(lone, fill <= 1 ? full * fill : full * std::ceil(fill) * (n == 2 ? 1.13 : 0.93));
+    return n == 2 ? both(4.1 + row * rows, 2.2 + mb / 8.2, 2.4) : both(1.9 + row * rows, 4.3 + mb / 9.1, 2.5);
+  }
+  // of two bounds that add up where they are alike
+  static double both(double x, double y, double p) { return std::pow(std::pow(x, p) + std::pow(y, p), 1.0 / p); }
   // both copies of the states and the coefficients in (about) the last-level
   // cache of 256 MB
   bool inCache() const { return (6.0 * MC_ * nb_ + 8.0) * sizeof(T) * (double)nVp_ < 300e6; }
@@ -2566,13 +2612,33 @@ class FomEngine final : public shaw_fom {
     if (inCache() && (sizeof(T) == 8 || state <= 42e6)) {
       double best = march;
       for (uint32_t rows = 2; rows <= 4; ++rows)
-        for (uint32_t steps = 6; steps <= 16 && 2 * steps < kTileWaves * rows; steps += 2)
+        for (uint32_t steps = 6; steps <= kTileSteps && 2 * steps < kTileWaves * rows; steps += 2)
           for (uint32_t cb = 1; cb <= 4; cb *= 2) {
             if (cb > 1 && cb > nb_) continue;
             const Tile t{rows, steps, cb};
             const double c = tileCost(t);
             if (c < best) { best = c; tile_ = t; }
           }
+      planShort();
+    }
+  }
+  // Launches of fewer steps than tile_'s. The long launch's windows, tall and for
+  // several column blocks, leave CUs idle there and load mostly for nothing, and a
+  // step or two is often fewer bytes for the marching kernels. Per launch, tile_'s
+  // windows -> now: 200 x 1000 M = 1, one step 9.6 -> 6.6 us; 230 x 1000 M = 7, 27.5 ->
+  // 23; 400 x 1200 M = 6 46 -> 34, three steps 53 -> 43; 200 x 500 M = 3 12.9 -> 8.0.
+  void planShort() {
+    for (uint32_t steps = 1; steps < tile_.steps; ++steps) {
+      double best = 1e300;
+      for (uint32_t rows = 2; rows <= 4; ++rows)
+        for (uint32_t cb = 1; cb <= 4 && 2 * steps < kTileWaves * rows; cb *= 2) {
+          if (cb >= 2 * nb_) continue;
+          const Tile t{rows, steps, cb};
+          const double c = steps < 6 ? shortTileCost(t) : tileCost(t) * steps;
+          if (c < best) { best = c; tileOf_[steps] = t; }
+        }
+      // (where the estimates are alike, the marching kernels of up to three steps)
+      marchShort_[steps] = steps <= (uint32_t)kMaxSpl && shortMarchCost((int)steps) < best * (steps <= 3 ? 1.08 : 1.0);
     }
   }
   // Microseconds per step of k_fusedW at ns steps a launch in segments of seg
@@ -2606,18 +2672,22 @@ class FomEngine final : public shaw_fom {
     const uint64_t n = (left + packSteps_ - 1) / packSteps_;
     return n ? (left + n - 1) / n : 0;
   }
-  // one launch of at most `left` steps, evenly split up to the next snapshot
-  // or the end of the run; returns its steps. A trial records nothing and
-  // does not advance the run.
-  uint64_t launchTile(uint64_t left, bool trial = false) {
-    const uint32_t rows = kTileWaves * tile_.rows;
+  // one window holds the whole grid: launches of any number of steps
+  bool wholeTile() const { return nth_ <= 64 && nr_ <= kTileWaves * tile_.rows; }
+  // steps of the next launch of at most `left`, evenly split up to the next
+  // snapshot or the end of the run
+  uint64_t tileSteps(uint64_t left) const {
     uint64_t ns = left;
     for (int d = 0; d < 2; ++d)
-      if (snap_[d].ncols && !trial) ns = std::min(ns, snap_[d].every - step_ % snap_[d].every);
-    if (nth_ > 64 || nr_ > rows) {  // one window holds the whole grid: any number of steps
-      const uint64_t n = (ns + tile_.steps - 1) / tile_.steps;
-      ns = (ns + n - 1) / n;
-    }
+      if (snap_[d].ncols) ns = std::min(ns, snap_[d].every - step_ % snap_[d].every);
+    if (wholeTile()) return ns;
+    const uint64_t n = (ns + tile_.steps - 1) / tile_.steps;
+    return (ns + n - 1) / n;
+  }
+  // one launch of ns steps. A trial records nothing and does not advance the run.
+  void launchTile(uint64_t ns, bool trial = false) {
+    const Tile t = ns < tile_.steps && !wholeTile() ? tileOf_[ns] : tile_;
+    const uint32_t rows = kTileWaves * t.rows;
     TileArgs<T> a{};
     a.vIn = v_[cur_].p;
     a.sIn = s_[cur_].p;
@@ -2640,15 +2710,15 @@ class FomEngine final : public shaw_fom {
     a.nth = (uint32_t)nth_;
     a.M = (uint32_t)M_;
     a.nb = nb_;
-    a.cbPer = tile_.cbPer;
+    a.cbPer = t.cbPer;
     a.haloX = nth_ <= 64 ? 0 : (uint32_t)ns;
     a.haloY = nr_ <= rows ? 0 : (uint32_t)ns;
     a.nTx = windows(nth_, 64, a.haloX);
     a.nTy = windows(nr_, rows, a.haloY);
     a.dt = (T)dt_;
     a.rank1 = rank1_;
-    if (MC_ == 1) tileKernel<1>(a);
-    else tileKernel<2>(a);
+    if (MC_ == 1) tileKernel<1>(a, t.rows);
+    else tileKernel<2>(a, t.rows);
     cur_ ^= 1;
     if (!trial) {
       step_ += ns;
@@ -2656,12 +2726,11 @@ class FomEngine final : public shaw_fom {
       snapshot(0, v_[cur_].p);
       snapshot(1, s_[cur_].p);
     }
-    return ns;
   }
   template <int CPT>
-  void tileKernel(const TileArgs<T>& a) {
+  void tileKernel(const TileArgs<T>& a, uint32_t rows) {
     const dim3 grid(a.nTx * a.nTy * ((a.nb + a.cbPer - 1) / a.cbPer)), block(kTileWaves * 64);
-    switch (tile_.rows) {
+    switch (rows) {
       case 2: hipLaunchKernelGGL((k_tile<T, CPT, 2, kTileWaves>), grid, block, 0, stream_, a); break;
       case 3: hipLaunchKernelGGL((k_tile<T, CPT, 3, kTileWaves>), grid, block, 0, stream_, a); break;
       default: hipLaunchKernelGGL((k_tile<T, CPT, 4, kTileWaves>), grid, block, 0, stream_, a); break;

@@ -1,5 +1,7 @@
 """What the plan of a default handle's launches leaves to the options, the
 autotuner and the byte counts."""
+import time
+
 import numpy as np
 import pytest
 
@@ -88,3 +90,26 @@ def test_bytes_per_step_are_of_the_launches_that_run(nr, nth, m, kw):
     assert fom.bytes_per_step()[0] == pytest.approx(want, rel=1e-12)
     assert kw or m > 1 or steps != fom.config()["steps_per_launch"]  # window tiles
     fom.close()
+
+
+def test_single_steps_are_not_slower_than_strips():
+    """200 x 500, 3 columns: advances by one step, which long launches' windows take
+    1.6 times as long for as the strips of explicit options (a quarter allowed for the
+    spread of a timing)."""
+    say("[gpu] single steps 200x500 M=3")
+    best = {}
+    for name, kw in (("default", {}), ("strips", dict(strip=64))):
+        fom = engine(200, 500, 3, 2000, **kw)
+        fom.advance(8)
+        fom.sync()
+        times = []
+        for _ in range(5):
+            t = time.perf_counter()
+            for _ in range(200):
+                fom.advance(1)
+            fom.sync()
+            times.append(time.perf_counter() - t)
+        best[name] = min(times)
+        fom.close()
+    say(f"  us per step {({k: round(v * 5e3, 2) for k, v in best.items()})}")
+    assert best["default"] <= 1.25 * best["strips"]

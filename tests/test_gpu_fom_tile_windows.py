@@ -57,3 +57,42 @@ def test_windows_equal_single_steps(grid, steps):
     for x, y in zip(*out):
         np.testing.assert_array_equal(x, y)
         assert np.isfinite(x).all() and np.abs(x).max() > 0
+
+
+@pytest.mark.parametrize("precision", [shaw_amd.FP64, shaw_amd.FP32])
+@pytest.mark.parametrize("nr,nth,m", [(49, 130, 2), (200, 500, 3), (230, 1000, 7), (400, 1200, 5), (160, 750, 13),
+                                      (150, 900, 1)])
+def test_short_launches_equal_single_steps(nr, nth, m, precision):
+    """Advances by a few steps and snapshots every few: launches of 1 to 9 steps,
+    by windows of their own or the marching kernels."""
+    say(f"[gpu] short launches {nr}x{nth} M={m} precision={precision}")
+    rng = np.random.default_rng(nr + nth + m)
+    app = shaw_amd.App.structured(nr, nth, LAYERED)
+    src = rng.integers(0, nr, m) * nth + rng.integers(0, nth, m)
+    recv = rng.integers(0, nr, 20) * nth + rng.integers(0, nth, 20)
+    runs = [1, 1, 2, 3, 4, 5, 6, 7, 8, 9]
+    total = sum(runs) + 24
+    table = rng.standard_normal((total, m))
+    state = [rng.standard_normal((n, m)) * 1e-3 for n in (app.nVp, app.nSp)]
+    out = []
+    for kw in ({}, dict(steps_per_launch=1)):
+        fom = shaw_amd.Fom(app, m, 0.2, precision=precision, **kw)
+        if not kw:
+            assert fom.launch_shape(5040)["segment"] == 0
+        fom.set_sources(src)
+        fom.set_forcing(table)
+        fom.set_receivers(recv, 1, total)
+        fom.set_state(*state)
+        for n in runs:
+            fom.advance(n)
+        got = [fom.seismogram(), *fom.state()]
+        fom.reset()
+        fom.set_snapshots("vp", 5, [0], 4)
+        fom.set_snapshots("sp", 2, [m - 1], 12)
+        fom.advance(24)
+        got += [fom.snapshots("vp"), fom.snapshots("sp"), *fom.state()]
+        out.append(got)
+        fom.close()
+    for x, y in zip(*out):
+        np.testing.assert_array_equal(x, y)
+        assert np.isfinite(x).all() and np.abs(x).max() > 0
