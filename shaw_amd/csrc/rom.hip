@@ -145,7 +145,8 @@ __device__ __forceinline__ void halfStep(const RomArgs& a, const void* A, int ro
 }
 
 // The FP64 reduced leapfrog for the engines and loads that k_rom_f64
-// (rom_f64.hip) does not take: more than 128 active tiles above 128 modes. One
+// (rom_f64.hip) does not take (residentModes, romF64Fits): many active tiles, and
+// dofs too unequal to be padded alike. One
 // workgroup (WAVES waves: 16 when the operators have 9 to 16 row tiles, one
 // tile per wave, which doubles the loads in flight per CU for the same operator
 // stream; else 8) owns kTileCols column slots and advances them a.nsteps steps,

@@ -513,11 +513,14 @@ bool launchF64Shared(const RomArgs& a, hipStream_t stream) {
 }  // namespace
 
 // Four columns a workgroup while the CUs they fill pay for re-reading the
-// operators: at K <= 128, resident, always (4096 columns: 64 1.9 us against
-// 2.6, 128 6.1 against 6.5); above, one round of workgroups per 64 active tiles
-// of 16 columns (K = 256: 7.7 us a round) against k_rom_steps' 18 us for up to
-// 256 of them: two rounds.
-bool romF64Fits(uint32_t modes, uint64_t activeTiles) { return modes <= 128 || activeTiles <= 128; }
+// operators: at K = 64, resident, always (4096 columns 1.9 us against 2.6, 32768
+// 14.0 against 17.0); at 128 up to 448 active tiles of 16 columns, 1.6 us a round of
+// 64 (4096 columns 6.9 us against 7.1, 7168 11.7 against 12.2, 8192 13.2 against 12.7);
+// above, one round of workgroups per 64 tiles (K = 256: 7.7 us a round) against
+// k_rom_steps' 18 us for up to 256 of them: two rounds.
+bool romF64Fits(uint32_t modes, uint64_t activeTiles) {
+  return modes <= 64 || activeTiles <= (modes <= 128 ? 448 : 128);
+}
 
 void launchRomF64(const RomArgs& a, hipStream_t stream) {
   const uint64_t cols = (uint64_t)a.tiles * kTileCols;

@@ -72,14 +72,14 @@ def test_bf16_equals_streaming(kv, ks, m, slots, precision, macro):
 
 # columns, slots just beyond those shared; slots and active columns of the
 # sixteen-column engine
-FP64 = [(193, 256, 9, 272, 2400, 2100), (256, 256, 272, 272, 2400, 2100), (384, 384, 30, 336, 2064, 0),
+FP64 = [(128, 128, 20, 48, 7300, 7250), (193, 256, 9, 272, 2400, 2100), (256, 256, 272, 272, 2400, 2100), (384, 384, 30, 336, 2064, 0),
         (330, 384, 336, 336, 2064, 0), (512, 512, 20, 272, 1040, 0), (449, 512, 272, 272, 1040, 0)]
 
 
 @pytest.mark.parametrize("kv,ks,m,slots,many,filler", FP64)
 def test_fp64_four_columns_long_launches(kv, ks, m, slots, many, filler):
     print(f"[gpu] FP64 ROM long launches kv={kv} ks={ks} M={m}", flush=True)
-    square = {256: 256, 384: 384, 512: 512}[ks]
+    square = {128: 128, 256: 256, 384: 384, 512: 512}[ks]
     assert shaw_amd.debug_rom_shape(shaw_amd.ROM_FP64, kv, ks, slots)[:2] == (square, 1)
     assert shaw_amd.debug_rom_shape(shaw_amd.ROM_FP64, square, square, many)[:2] == (square if filler else 0, 1)
     arv, ars, rows, b, f = operators(kv, ks, m, 120, False)
