@@ -2667,10 +2667,14 @@ class FomEngine final : public shaw_fom {
                                        : std::max(lone, fill * full * bytes);
     return row * (seg + 2 * ns - 1) / ns;
   }
-  // steps of the next planned pack when `left` steps are to go
+  // steps of the next planned pack when `left` steps are to go. Up to seven go in
+  // one where two cost more (300 x 1000 M = 40 FP32, packs of four: seven steps as
+  // 4 + 3 177 us, as one launch 155)
   uint64_t packOf(uint64_t left) const {
-    const uint64_t n = (left + packSteps_ - 1) / packSteps_;
-    return n ? (left + n - 1) / n : 0;
+    const uint64_t n = (left + packSteps_ - 1) / packSteps_, len = n ? (left + n - 1) / n : 0;
+    const bool one = n == 2 && left <= (uint64_t)kMaxSpl &&
+                     shortMarchCost((int)left) < shortMarchCost((int)len) + shortMarchCost((int)(left - len));
+    return one ? left : len;
   }
   // one window holds the whole grid: launches of any number of steps
   bool wholeTile() const { return nth_ <= 64 && nr_ <= kTileWaves * tile_.rows; }
