@@ -33,6 +33,7 @@ METRIC = "forcing-steps/s, plain FP64 vs batched ROM at err<=1e-3; p50/p99 laten
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "fom_fused_config2_traffic.txt")
+TRAFFIC_FILES = (TRAFFIC_FILE, TRAFFIC_FILE.replace("fom_fused_", "fom_planned_"))  # six-step launches; the planned ones
 
 
 def measured_traffic(kernel_cfg: dict):
@@ -40,17 +41,18 @@ def measured_traffic(kernel_cfg: dict):
     counter summary (FETCH_SIZE and WRITE_SIZE, each scaled by what the same
     counter reads for a copy kernel of known size), when it was measured for
     this kernel configuration; otherwise None."""
-    try:
-        kv = dict(line.split(":", 1) for line in open(TRAFFIC_FILE) if ":" in line and not line.startswith(" "))
-    except OSError:
-        return None
-    kv = {k.strip(): v.strip() for k, v in kv.items()}
     want = (f"cols_per_thread={kernel_cfg['cols_per_thread']} strip={kernel_cfg['strip']} "
             f"segment={kernel_cfg['segment']} prefetch_rows={kernel_cfg['prefetch_rows']} "
             f"steps_per_launch={kernel_cfg['steps_per_launch']} col_block={kernel_cfg['col_block']}")
-    if kv.get("kernel_config") != want:
-        return None
-    return float(kv["traffic_bytes_per_launch"])
+    for path in TRAFFIC_FILES:
+        try:
+            kv = dict(line.split(":", 1) for line in open(path) if ":" in line and not line.startswith(" "))
+        except OSError:
+            continue
+        kv = {k.strip(): v.strip() for k, v in kv.items()}
+        if kv.get("kernel_config") == want:
+            return float(kv["traffic_bytes_per_launch"])
+    return None
 
 
 def fused_kernel_name(cfg: dict) -> str:
@@ -399,14 +401,16 @@ def config5_section(args) -> dict:
         fom.set_receivers(rec, w.seis_every, n_tab // w.seis_every)
         tuned = fom.autotune(3)
         cfg = fom.config()
+        shape = fom.launch_shape(ROOF_STEPS)  # of the launches that run: the planned ones where they were the fastest
+        ran = {**cfg, "steps_per_launch": shape["steps_per_launch"], "segment": shape["segment"]}
         fom.advance(args.warmup)
         fom.sync()
         total, per = fom.time(args.steps)
         kb, mb = fom.bytes_per_step()
         out[name] = {"ms_per_step": per, "forcing_steps_per_s": w.m / (per / 1e3),
                      "algorithmic_GB_s": kb / (per / 1e3) / 1e9, "hbm_frac": kb / (per / 1e3) / 1e9 / HBM_PEAK_GBS,
-                     "bytes_per_step": kb, "autotuned": {"config": cfg, "trial_ms_per_step": tuned}}
-        log(f"config5 {name}: {per:.3f} ms/step, {kb / (per / 1e3) / 1e9:.0f} GB/s, config {cfg}")
+                     "bytes_per_step": kb, "autotuned": {"config": ran, "trial_ms_per_step": tuned}}
+        log(f"config5 {name}: {per:.3f} ms/step, {kb / (per / 1e3) / 1e9:.0f} GB/s, config {ran}")
         fom.close()
         # error run from zero state over the first n_err steps
         fom = shaw_amd.Fom(app, w.m, w.dt, precision=prec, rank1_forcing=False, cols_per_thread=cfg["cols_per_thread"],
