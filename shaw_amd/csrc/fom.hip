@@ -32,7 +32,8 @@
 //  * k_fusedW: three to seven steps per launch when a 64-point strip is one
 //    wavefront (one thread per point, all columns of a 1- or 2-column block);
 //    neighbours move between lanes, and the waves of a workgroup share only
-//    a coefficient ring. The default: six steps per launch.
+//    a coefficient ring. The default on larger grids, four to seven steps per
+//    launch as planned.
 //  * k_tile: six to sixteen steps per launch on grids whose states stay in
 //    the last-level cache; a workgroup holds a window of the grid, states and
 //    coefficients, in registers.

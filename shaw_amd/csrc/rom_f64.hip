@@ -226,7 +226,8 @@ __global__ void __launch_bounds__(WAVES * 64) k_rom_f64(RomArgs a) {
 // k_rom_f64 -> this: K = 256 6.3 us -> 4.0 at 16 columns, 4.2 at 256; 384 15.4 ->
 // 5.1 at 160, 8.3 at 320; 512 30.1 -> 7.6 at 128, 10.4 at 256. (Two sets of 256
 // modes, half the row tiles each, 1024 columns: 9.2 us against 8.0; two sets by
-// turns, one's exchange behind the other's products, 10.0.)
+// turns, one's exchange behind the other's products, 10.0.) A kernel of its own: as
+// an instantiation of this body k_rom_f64 lost 3 to 8 % at K = 64.
 template <int G, int WAVES, int RR, int LL, int DR, int SPLIT, int SETS>
 __global__ void __launch_bounds__(WAVES * 64) k_rom_f64_shared(RomArgs a) {
   constexpr int K = 16 * G, OWN = G / SPLIT, TPW = OWN / WAVES;

@@ -1,8 +1,9 @@
 """The window-tile FOM kernel (the default on grids whose states stay in the
-last-level cache) at the edges of its windows: 64 points by 24, 36 or 48 rows,
-whole grids in one window, remainders of one point or row, one to five columns,
-split runs. Every output equals the oracle's bit for bit (no FMA, the same
-expressions in the same order), and FP32 states those of single FP32 steps."""
+last-level cache) at the edges of its windows: 64 points by 24 rows (taller ones
+in test_gpu_fom_tile_windows.py), whole grids in one window of up to 48,
+remainders of one point or row, one to five columns, split runs. Every output
+equals the oracle's bit for bit (no FMA, the same expressions in the same order),
+and FP32 states those of single FP32 steps."""
 import numpy as np
 import pytest
 

@@ -1,4 +1,5 @@
-"""FP64 reduced-order engines: workgroups of four columns (k_rom_f64) against
+"""FP64 reduced-order engines: workgroups of four columns (k_rom_f64; from 193
+modes on shared among workgroups in launches of ten, above 256 of four steps) against
 workgroups of sixteen (k_rom_steps). The kernels add a product's terms in the
 same order with one rounding each, so every value must agree bit for bit. The
 sixteen-column kernel runs the same problem when more than 128 tiles of columns

@@ -1,9 +1,11 @@
 """BF16 reduced-order engines of up to 256 modes keep their operators on the
-CU; larger ones stream them every step. Zero modes change no value of the
-others, so an engine whose operators are padded with zeros past 256 modes runs
-the streaming kernel on the same problem: both must agree bit for bit, at the
-edges of the padded sizes (64, 128, 192, 256), with kv != ks, with uneven
-horizons, split runs, partly filled tiles and macro steps."""
+CU; larger ones share them among workgroups where columns are few. Zero modes
+change no value of the others, so an engine whose operators are padded with zeros
+past 256 modes runs the same problem as a shared one of 384 (in launches below
+four steps as one workgroup): both must agree bit for bit (with the kernels that
+stream their operators, test_gpu_rom_streaming.py compares), at the edges of the
+padded sizes (64, 128, 192, 256), with kv != ks, with uneven horizons, split
+runs, partly filled tiles and macro steps."""
 import numpy as np
 import pytest
 
