@@ -69,3 +69,59 @@ def test_a_value_that_never_comes_is_an_error(kv, ks, m, precision):
     with pytest.raises(shaw_amd.ShawError, match="lost each other"):
         rom.state(slots[0])
     rom.close()
+
+
+@pytest.mark.parametrize("tries", [100, 1 << 24])
+def test_shared_engine_beside_a_long_launch(tries):
+    """Another engine's launch holds most CUs for a tenth of a second: groups that
+    cannot be placed wait for it, or give up early and run unshared after it."""
+    print(f"[gpu] shared ROM beside a long launch, {tries} tries", flush=True)
+    rng = np.random.default_rng(3)
+    k, m = 512, 4000
+    big = shaw_amd.Rom(rng.standard_normal((k, k)) * 0.01, rng.standard_normal((k, k)) * 0.01, 0.2, shaw_amd.ROM_FP64,
+                       rng.standard_normal((2, k)), max_cols=m, max_samples=20)
+    big.admit_signals(rng.standard_normal((k, m)), ["ricker"] * m, np.full(m, 20.0), np.full(m, 5.0), 2000, every=100)
+    for kv, ks, cols, precision in ((384, 384, 640, shaw_amd.ROM_BF16X4), (512, 512, 128, shaw_amd.ROM_FP64)):
+        out = []
+        for beside in (False, True):
+            rom, slots = engine(kv, ks, cols, precision, 0, 0)
+            rom.sync()
+            if beside:
+                shaw_amd.debug_rom_waits(rom, tries)
+                big.advance(800)
+            for n in (100, 150, 50):
+                rom.advance(n)
+            out.append(results(rom, slots))
+        for x, y in zip(out[0][0], out[1][0]):
+            np.testing.assert_array_equal(x, y)
+        for x, y in zip(out[0][1], out[1][1]):
+            assert x[2] == y[2]
+            np.testing.assert_array_equal(x[0], y[0])
+            np.testing.assert_array_equal(x[1], y[1])
+    big.sync()
+
+
+@pytest.mark.parametrize("kv,ks,m,precision", [(384, 384, 40, shaw_amd.ROM_BF16X4), (512, 300, 20, shaw_amd.ROM_BF16X3),
+                                               (256, 256, 20, shaw_amd.ROM_FP64), (384, 384, 300, shaw_amd.ROM_FP64)])
+def test_nonfinite_columns_stay_their_own(kv, ks, m, precision):
+    """A column that is infinite or undefined goes through the exchange as such and
+    leaves the others alone, as in an engine that shares nothing."""
+    print(f"[gpu] shared ROM with non-finite columns kv={kv} M={m} precision={precision}", flush=True)
+    rng = np.random.default_rng(kv + m)
+    arv = rng.standard_normal((kv, ks)) * (0.5 / np.sqrt(max(kv, ks)))
+    rows, b, f = rng.standard_normal((3, kv)), rng.standard_normal((kv, m)), rng.standard_normal((60, m))
+    f[7, 0], f[11, 5], f[13, 18] = np.nan, np.inf, -np.inf
+    out = []
+    for slots in (m, 2400):
+        assert (shaw_amd.debug_rom_shape(precision, kv, ks, slots)[1] > 1) == (slots == m)
+        rom = shaw_amd.Rom(arv, -arv.T.copy(), 0.2, precision, rows, max_cols=slots, max_samples=60)
+        ids = rom.admit(b, f, [60] * m, every=1)
+        rom.advance(60)
+        states = [rom.state(s) for s in ids]
+        out.append((rom.retire_many(ids, 60), states))
+    for j, (x, y) in enumerate(zip(out[0][0], out[1][0])):
+        np.testing.assert_array_equal(x, y)
+        assert np.isfinite(x).all() == (j not in (0, 5, 18))
+    for (v, s, _), (w, t, _) in zip(out[0][1], out[1][1]):
+        np.testing.assert_array_equal(v, w)
+        np.testing.assert_array_equal(s, t)
